@@ -121,12 +121,26 @@ __device__ __forceinline__ void store16(void* p, uint4 v) {
     else *q = r;
 }
 
-template <bool NT>
-__device__ __forceinline__ void store8(void* p, uint2 v) {
-    MCEP_GLOBAL u32x2* q = (MCEP_GLOBAL u32x2*)(uintptr_t)p;
-    const u32x2 r = {v.x, v.y};
-    if (NT) __builtin_nontemporal_store(r, q);
-    else *q = r;
+// How a payload row leaves the CU.
+//   kStorePlain    into the XCD's L2, written back when the line is evicted or, at the latest, at the end of the
+//                  kernel - which holds up the next one for as long as 8 x 4 MB of dirty lines take;
+//   kStoreStream   streaming (nontemporal): not kept in L2 nor in the 256 MB memory-side cache;
+//   kStoreThrough  written through the L2 (sc1) to the memory side as it is issued: nothing is dirty in the L2 when
+//                  the kernel ends, and the line may still wait in the memory-side cache for its reader.
+enum : int { kStorePlain = 0, kStoreStream = 1, kStoreThrough = 2 };
+
+// 16 bytes at `off` of a row of `row_bytes` bytes; `row` is wave-uniform, off + 16 <= row_bytes.
+template <int HINT>
+__device__ __forceinline__ void store16_row(uint64_t row, int off, uint4 v, int row_bytes) {
+    if (HINT == kStoreThrough) {
+        // the cache-policy operand of a buffer store is the one way to ask for write-through on 16 bytes at once
+        constexpr int kBufferFlags = 0x00027000, kSc1 = 0x10;
+        __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)row, 0, row_bytes, kBufferFlags);
+        const u32x4 r = {v.x, v.y, v.z, v.w};
+        __builtin_amdgcn_raw_buffer_store_b128(r, rsrc, off, 0, kSc1);
+    } else {
+        store16<HINT == kStoreStream>((void*)(uintptr_t)(row + (uint64_t)off), v);
+    }
 }
 
 __device__ __forceinline__ float load_f32(uint64_t addr) { return *(const MCEP_GLOBAL float*)(uintptr_t)addr; }
@@ -588,7 +602,7 @@ __device__ __forceinline__ uint4 quantise16(uint4 a, uint4 b, float* scale_inv) 
 // column-major output with coalesced stores (writing them there from here would
 // be 4-byte stores 16 KB apart).
 //   NATIVE  which of the reference's two statements of the scale arithmetic (see quantise16)
-template <bool NTL, bool NATIVE, bool NTS>
+template <bool NTL, bool NATIVE, int HINT>
 __global__ __launch_bounds__(512) void pack_fp8_kernel(const uint64_t* __restrict__ tbl,
                                                         RoutingScratch sc, DispatchSource src,
                                                         float* __restrict__ scale_stage, int R, int E, int K,
@@ -632,12 +646,12 @@ __global__ __launch_bounds__(512) void pack_fp8_kernel(const uint64_t* __restric
     for (int k = 0; k < K; ++k) {
         const uint64_t row = read_lane_u64(dst.row, k * sel_lanes);
         if (row == 0) continue;
-        if (active) store16<NTS>((void*)(row + elem0), out);
+        if (active) store16_row<HINT>(row, elem0, out, H);
     }
 }
 
 // bf16: plain row copy, two unit-stride 16-byte pieces per lane.
-template <bool NTL, bool NTS>
+template <bool NTL, int HINT>
 __global__ __launch_bounds__(512) void pack_bf16_kernel(const uint64_t* __restrict__ tbl,
                                                          RoutingScratch sc, DispatchSource src,
                                                          float* __restrict__ /*scale_stage*/, int R, int E, int K,
@@ -662,14 +676,14 @@ __global__ __launch_bounds__(512) void pack_bf16_kernel(const uint64_t* __restri
     const int64_t* idx_row;
     if (!pack_token(tbl, src, R, K, H, r, t, &xbase, &idx_row)) return;
 
-    int64_t off[2];
+    int off[2];
     bool active[2];
     uint4 v[2];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
         const int elem = s * 1024 + p * 512 + lane * 8;
         active[p] = elem < H;
-        off[p] = (int64_t)elem * 2;
+        off[p] = elem * 2;
         v[p] = make_uint4(0, 0, 0, 0);
         if (active[p]) v[p] = load16<NTL>(xbase + off[p]);
     }
@@ -681,7 +695,7 @@ __global__ __launch_bounds__(512) void pack_bf16_kernel(const uint64_t* __restri
         if (row == 0) continue;
 #pragma unroll
         for (int p = 0; p < 2; ++p)
-            if (active[p]) store16<NTS>((void*)(row + off[p]), v[p]);
+            if (active[p]) store16_row<HINT>(row, off[p], v[p], H * 2);
     }
 }
 
@@ -1655,31 +1669,36 @@ static hipError_t launch_pack_t(Kern kern, const uint64_t* d_tbl, const RoutingS
 hipError_t launch_pack(const uint64_t* d_tbl, const RoutingScratch& sc, const DispatchSource& src, float* scale_stage,
                        const Dims& d, bool use_fp8, const Tuning& t, bool run_pack, bool run_finish,
                        hipStream_t stream) {
-    // Streaming hints (bit 0: loads, bit 1: stores).  Default: streaming loads when a token's row goes to many
-    // experts, ordinary stores.  Both hints together always lose (+6 to +9 us on the decode workloads).
-    // Streaming stores with ordinary loads win in the steady state - 2 % of the DeepSeek-V3 decode step, 5 to
-    // 13 % of a dispatch whose payload is several times the 256 MB memory-side cache - but lose under the
-    // reference's timing protocol, a written cache flush before every timed call (8 x 1024 tokens, hidden 7168,
-    // top-8, bf16: 218 against 180 us), and a consumer that reads a cacheable payload next finds it in memory
-    // instead of that cache.  They are an option (pack_nt = 2), not the default.
-    const int nt = t.pack_nt >= 0 ? t.pack_nt : (d.K > 4 ? 1 : 0);
-    const bool ntl = (nt & 1) != 0, nts = (nt & 2) != 0;
+    // Cache hints (bit 0: streaming loads; bit 1: streaming stores, bit 2: write-through stores).  What is measured is
+    // the whole dispatch -> consumer -> combine cycle with the tensors of three cycles in rotation, because the stores
+    // decide where the consumer finds the payload and who waits for its write-back.
+    //   fp8, 80 MiB of payload and more: streaming stores, ordinary loads.  235 MB (32 x 128 tokens, hidden 7168,
+    //     top-8): 167 -> 152 us the cycle with expert rows given, 129 -> 124 with the packed combine, 302 -> 296 with
+    //     the cast back in between; 115 MB: 90.7 -> 83.2, 76.2 -> 72.1, 161.6 -> 154.9; 57 MB: 51.0 -> 51.8,
+    //     41.7 -> 46.0, 90.9 -> 92.4, so below that the payload is left to the cache.
+    //   otherwise: write-through stores, and streaming loads from top-5 up.  bf16, 268 MB (16 x 256 tokens, hidden 4096,
+    //     top-8): 104.3 -> 102.7 when combine reads the payload (112.1 with streaming stores), 200.5 -> 198.3 with the
+    //     cast back in between, 120.4 -> 119.2 with expert rows given; fp8, 57 MB: 51.0 -> 49.6, 41.7 -> 41.5.
+    // A cache flush between the calls of a cycle hides what ordinary stores put off (their write-back falls into the
+    // flush) and so turns the first line around: it is right for callers whose calls follow each other.
+    constexpr long long kStreamBytes = 80ll << 20;
+    const bool stream_out = use_fp8 && (long long)d.R * d.Tgrid * d.K * d.H >= kStreamBytes;
+    const int nt = t.pack_nt >= 0 ? t.pack_nt : (stream_out ? 2 : (d.K > 4 ? 5 : 4));
+    const bool ntl = (nt & 1) != 0;
     if (use_fp8 && scale_stage == nullptr) return hipErrorInvalidValue;
     hipError_t err = hipSuccess;
     if (run_pack) {
-#define MCEP_PF(A, B)                                                                                   \
-    (nts ? launch_pack_t(pack_fp8_kernel<A, B, true>, d_tbl, sc, src, scale_stage, d, t, stream)        \
-         : launch_pack_t(pack_fp8_kernel<A, B, false>, d_tbl, sc, src, scale_stage, d, t, stream))
-#define MCEP_PB(A)                                                                                      \
-    (nts ? launch_pack_t(pack_bf16_kernel<A, true>, d_tbl, sc, src, scale_stage, d, t, stream)          \
-         : launch_pack_t(pack_bf16_kernel<A, false>, d_tbl, sc, src, scale_stage, d, t, stream))
+#define MCEP_HINT(KERNEL, ...)                                                                                       \
+    ((nt & 4) ? launch_pack_t(KERNEL<__VA_ARGS__, kStoreThrough>, d_tbl, sc, src, scale_stage, d, t, stream)         \
+     : (nt & 2) ? launch_pack_t(KERNEL<__VA_ARGS__, kStoreStream>, d_tbl, sc, src, scale_stage, d, t, stream)        \
+                : launch_pack_t(KERNEL<__VA_ARGS__, kStorePlain>, d_tbl, sc, src, scale_stage, d, t, stream))
         if (!use_fp8)
-            err = ntl ? MCEP_PB(true) : MCEP_PB(false);
+            err = ntl ? MCEP_HINT(pack_bf16_kernel, true) : MCEP_HINT(pack_bf16_kernel, false);
+        else if (t.fp8_arith == 1)
+            err = ntl ? MCEP_HINT(pack_fp8_kernel, true, true) : MCEP_HINT(pack_fp8_kernel, false, true);
         else
-            err = ntl ? (t.fp8_arith == 1 ? MCEP_PF(true, true) : MCEP_PF(true, false))
-                      : (t.fp8_arith == 1 ? MCEP_PF(false, true) : MCEP_PF(false, false));
-#undef MCEP_PB
-#undef MCEP_PF
+            err = ntl ? MCEP_HINT(pack_fp8_kernel, true, false) : MCEP_HINT(pack_fp8_kernel, false, false);
+#undef MCEP_HINT
     }
     if (err != hipSuccess || !use_fp8 || !run_finish) return err;
     int parts = 1;
