@@ -49,6 +49,10 @@ constexpr int kMaxTopK = 16;          // the reference caps top-k at 11 (mooncak
 constexpr int kTableChunk = 384;      // table words one writer launch carries in its kernel arguments
 constexpr size_t kZeroRowBytes = 64 * 1024;   // zero row that masked selections read: hidden <= 32768
 
+// A rank table of this many words (dispatch, combine: 32 ranks) travels in the arguments of the kernels that need it;
+// larger worlds, and calls whose first kernel does not run now, have it written to memory by a launch of its own.
+constexpr int kArgTableWords = 288;
+
 struct TableChunk {
     uint64_t v[kTableChunk];
 };
@@ -122,6 +126,8 @@ struct CombineSource {
     RankPtr topk_idx, topk_weights, out;
     RankPtr x;              // the rows combine reads (expert outputs, or the packed payload)
     RankPtr scales;         // packed combine of an fp8 payload
+    RankPtr active;
+    bool packed_fp8 = false;   // `scales` is read
     int tokens = -1;
 };
 
@@ -133,6 +139,7 @@ struct Dims {
     int max_tokens;   // num_max_dispatch_tokens_per_rank
     int Tgrid;        // max over ranks of T_r (grid extent in tokens per rank)
     UnitPlan plan;    // set by plan_units()
+    const uint64_t* host_table = nullptr;   // the call's rank table, to travel in kernel arguments; null: it is on the device
     int units_per_rank() const { return plan.per_rank; }
     int units() const { return plan.total; }
 };
@@ -165,8 +172,10 @@ struct Tuning {
 };
 
 // Chooses the unit plan for a shape (summed when allowed, the shape permits and there are tokens).
-// (plan_units, count_lds_bytes and cast_back_chunks are host arithmetic: ep_plan.cpp.)
+// (plan_units, combine_reads_table, count_lds_bytes and cast_back_chunks are host arithmetic: ep_plan.cpp.)
 void plan_units(Dims& d, const Tuning& t);
+// Whether the reduce kernels look anything up in the rank table: nothing when every tensor they touch is evenly spaced.
+bool combine_reads_table(const CombineSource& src, bool direct);
 
 hipError_t launch_table_write(uint64_t* d_tbl, const uint64_t* h_tbl, int n_words, hipStream_t stream);
 

@@ -154,6 +154,22 @@ __global__ void table_write_kernel(uint64_t* dst, TableChunk chunk, int n) {
     if (i < n) dst[i] = chunk.v[i];
 }
 
+// A rank table that travels in a kernel's arguments (N words; 0: the kernel reads it from memory).  A call whose
+// tensors lie elsewhere than the last call's would otherwise have to put its table into memory first, a launch of
+// 4.6 us in front of kernels that take 5 to 90.
+template <int N>
+struct ArgTable {
+    uint64_t v[N > 0 ? N : 1];
+};
+
+template <int N>
+static ArgTable<N> arg_table(const uint64_t* words, int n) {
+    ArgTable<N> t{};
+    if (N > 0)
+        for (int i = 0; i < n; ++i) t.v[i] = words[i];
+    return t;
+}
+
 // Clears `words` 32-bit words at each of n addresses carried in kernel
 // arguments: one launch where a per-rank hipMemsetAsync would be n launches.
 __global__ void clear_words_kernel(TableChunk chunk, int n, int words) {
@@ -180,10 +196,13 @@ __device__ __forceinline__ uint64_t rank_ptr(const uint64_t* __restrict__ tbl, c
 // (A token is expected to name an expert at most once; if it names one twice,
 // each occurrence gets its own row, as in the reference kernel, which sends
 // once per k: mooncake_ep_kernel.cu:230,273.)
-template <int UNIT>
-__global__ __launch_bounds__(UNIT) void count_kernel(const uint64_t* __restrict__ tbl, RoutingScratch sc,
+// TW > 0: the call's rank table comes in the arguments; the blocks put it into memory (tbl_mem), where the launches
+// that follow read it.  TW == 0: it is there already.
+template <int UNIT, int TW>
+__global__ __launch_bounds__(UNIT) void count_kernel(uint64_t* __restrict__ tbl_mem, RoutingScratch sc,
                                                       DispatchSource src, int R, int E, int K, int max_tokens,
-                                                      int upr) {
+                                                      int upr, ArgTable<TW> arg_tbl) {
+    const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
     extern __shared__ unsigned long long lds_count[];
     constexpr int NW = UNIT / 64;
     unsigned long long* wmask = lds_count;                     // [NW][E] lanes of the wave that name e
@@ -196,6 +215,8 @@ __global__ __launch_bounds__(UNIT) void count_kernel(const uint64_t* __restrict_
     const int T = src.tokens >= 0 ? src.tokens : (int)tbl[DF_NUM_TOKENS * R + r];
     const int n = T * K;
     const int sel = c * UNIT + tid;                            // index into the rank's [T, K] list
+    if (TW > 0)
+        for (int i = u * UNIT + tid; i < (int)DF_COUNT * R; i += (int)gridDim.x * UNIT) tbl_mem[i] = arg_tbl.v[i];
 
     int64_t e64 = -1;
     if (sel < n) e64 = ((const int64_t*)rank_ptr(tbl, src.topk_idx, DF_TOPK_IDX, R, r))[sel];
@@ -892,10 +913,12 @@ __global__ __launch_bounds__(256) void dispatch_small_kernel(SmallTable tb, int3
 // src_info; each row finds its k in the token's top-k list and leaves the
 // row's address and weight there.  Experts on ranks the owner sees as
 // inactive, and rows of ranks that take no part, leave no route.
-template <bool PACKED>
-__global__ __launch_bounds__(256) void resolve_kernel(const uint64_t* __restrict__ tbl,
+template <bool PACKED, int TW>
+__global__ __launch_bounds__(256) void resolve_kernel(const uint64_t* __restrict__ tbl_mem,
                                                        CombineRoute* __restrict__ routes, uint32_t stamp, int R,
-                                                       int E, int K, int H, int max_tokens, int total_tasks) {
+                                                       int E, int K, int H, int max_tokens, int total_tasks,
+                                                       ArgTable<TW> arg_tbl) {
+    const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
     const int lane = wave_lane();
     const int task = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     if (task >= total_tasks) return;
@@ -958,16 +981,16 @@ struct DirectRow {
 };
 
 __device__ __forceinline__ DirectRow direct_row(const uint64_t* __restrict__ tbl, const RoutingScratch& sc,
-                                                const RankPtr& x, const RankPtr& topk_idx, int R, int E, int K,
-                                                int max_tokens, int r, int t, int lane) {
+                                                const CombineSource& cs, int R, int E, int K, int max_tokens, int r,
+                                                int t, int lane) {
     const int RM = R * max_tokens;
     const int L = E / R;
-    const uint64_t active = tbl[CF_ACTIVE * R + r];
+    const uint64_t active = rank_ptr(tbl, cs.active, CF_ACTIVE, R, r);
     const int li = lane < K ? lane : 0;
     // The selection as combine is given it, next to the row the dispatch left (two independent loads):
     // combine reads topk_idx itself and skips what is negative there (mooncake_ep_kernel.cu:719-732), so
     // a selection masked - or pointed elsewhere - after the dispatch has no row.
-    const int64_t now = ((const MCEP_GLOBAL int64_t*)(uintptr_t)rank_ptr(tbl, topk_idx, CF_TOPK_IDX, R, r))[(int64_t)t * K + li];
+    const int64_t now = ((const MCEP_GLOBAL int64_t*)(uintptr_t)rank_ptr(tbl, cs.topk_idx, CF_TOPK_IDX, R, r))[(int64_t)t * K + li];
     const int sr = sc.selrow[((int64_t)r * max_tokens + t) * K + li];
     DirectRow d;
     d.has = lane < K && sr >= 0 && now == (int64_t)(sr / RM);
@@ -975,7 +998,7 @@ __device__ __forceinline__ DirectRow direct_row(const uint64_t* __restrict__ tbl
     d.slot = d.has ? sr - d.e * RM : 0;
     d.q = d.e / L;
     d.le = d.e - d.q * L;
-    d.base = rank_ptr(tbl, x, CF_X, R, d.q);
+    d.base = rank_ptr(tbl, cs.x, CF_X, R, d.q);
     d.grow = (int64_t)d.le * RM + d.slot;
     // `live` is asked for last, behind whatever the base address had to wait for (a table entry when the
     // ranks' tensors are not evenly spaced): loads complete in order for a waiting wave, so a load issued
@@ -993,13 +1016,15 @@ __device__ __forceinline__ DirectRow direct_row(const uint64_t* __restrict__ tbl
 //   DIRECT   the handle is the one the last dispatch produced: rows come from
 //            that dispatch's routing state, no resolve kernel has run;
 //   !DIRECT  rows come from the routes the resolve kernel left.
-template <int KMAX, int CH, bool NTL, bool NTS, bool DIRECT>
-__global__ __launch_bounds__(512) void reduce_kernel(const uint64_t* __restrict__ tbl,
+//   TW       words of the rank table in the arguments; 0: in memory, or not needed (every tensor evenly spaced).
+template <int KMAX, int CH, bool NTL, bool NTS, bool DIRECT, int TW>
+__global__ __launch_bounds__(512) void reduce_kernel(const uint64_t* __restrict__ tbl_mem,
                                                       const CombineRoute* __restrict__ routes, uint32_t stamp,
                                                       RoutingScratch sc, CombineSource cs,
                                                       const void* __restrict__ zero_row, int R, int E, int K,
                                                       int max_tokens, int H, int slabs, int Tgrid,
-                                                      int total_tasks) {
+                                                      int total_tasks, ArgTable<TW> arg_tbl) {
+    const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
     const int lane = wave_lane();
     const int task = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     if (task >= total_tasks) return;
@@ -1016,7 +1041,7 @@ __global__ __launch_bounds__(512) void reduce_kernel(const uint64_t* __restrict_
         if (t >= T) return;
         const uint64_t w_row = rank_ptr(tbl, cs.topk_weights, CF_TOPK_W, R, r) + (uint64_t)((int64_t)t * K) * 4;
         const float wl = load_f32(w_row + (uint64_t)(lane < K ? lane : 0) * 4);
-        const DirectRow d = direct_row(tbl, sc, cs.x, cs.topk_idx, R, E, K, max_tokens, r, t, lane);
+        const DirectRow d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, lane);
         if (d.has && d.base != 0) {
             src = d.base + (uint64_t)d.grow * (uint64_t)H * 2;
             w = wl;
@@ -1133,14 +1158,15 @@ __device__ __forceinline__ uint32_t scale_round_twice(float a, float b, float s,
 // variant ran 5 % slower.  (Sixteen rows in flight do not fit that budget.)
 //   CH  bf16 payloads only: 16-byte chunks per lane and row, 512 elements apart (two when there are few
 //       rows per token, as in reduce_kernel: half as many waves, each with as many loads in flight)
-template <int KMAX, bool FP8, bool FACTOR, bool DIRECT, int CH = 1>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ? 8 : 4, 8))) void reduce_packed_kernel(const uint64_t* __restrict__ tbl,
+template <int KMAX, bool FP8, bool FACTOR, bool DIRECT, int CH, int TW>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ? 8 : 4, 8))) void reduce_packed_kernel(const uint64_t* __restrict__ tbl_mem,
                                                              const CombineRoute* __restrict__ routes, uint32_t stamp,
                                                              RoutingScratch sc, CombineSource cs,
                                                              const void* __restrict__ zero_row,
                                                              const float* __restrict__ factor, int R, int E, int K,
                                                              int max_tokens, int H, int slabs, int Tgrid,
-                                                             int group_blocks) {
+                                                             int group_blocks, ArgTable<TW> arg_tbl) {
+    const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
     static_assert(!FP8 || CH == 1, "an fp8 payload is one 16-byte chunk of 16 elements per lane");
     constexpr int kSlab = FP8 ? 1024 : 512 * CH;
     constexpr int kChunkElems = FP8 ? 16 : 8;          // elements in a lane's 16-byte chunk
@@ -1187,7 +1213,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
         if (DIRECT) {
             const uint64_t w_row = rank_ptr(tbl, cs.topk_weights, CF_TOPK_W, R, r) + (uint64_t)((int64_t)t * K) * 4;
             wl = load_f32(w_row + (uint64_t)(lane < K ? lane : 0) * 4);
-            const DirectRow d = direct_row(tbl, sc, cs.x, cs.topk_idx, R, E, K, max_tokens, r, t, lane);
+            const DirectRow d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, lane);
             ok = d.has;
             e = d.e;
             slot = d.slot;
@@ -1607,19 +1633,26 @@ hipError_t launch_count(const uint64_t* d_tbl, const RoutingScratch& sc, const D
                         hipStream_t stream) {
     const size_t lds = count_lds_bytes(d);
     if (lds > kMaxCountLdsBytes) return hipErrorInvalidValue;
-    const void* kern = d.plan.shift == 10 ? (const void*)count_kernel<kBigUnitSelections>
-                                          : (const void*)count_kernel<kUnitSelections>;
-    if (lds > 48 * 1024) {
-        hipError_t err = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (err != hipSuccess) return err;
-    }
-    if (d.plan.shift == 10)
-        hipLaunchKernelGGL(count_kernel<kBigUnitSelections>, dim3(d.units()), dim3(kBigUnitSelections), lds, stream,
-                           d_tbl, sc, src, d.R, d.E, d.K, d.max_tokens, d.units_per_rank());
-    else
-        hipLaunchKernelGGL(count_kernel<kUnitSelections>, dim3(d.units()), dim3(kUnitSelections), lds, stream, d_tbl,
-                           sc, src, d.R, d.E, d.K, d.max_tokens, d.units_per_rank());
-    hipError_t err = hipGetLastError();
+    auto launch = [&](auto kern, auto arg, int unit) -> hipError_t {
+        if (lds > 48 * 1024) {
+            hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (err != hipSuccess) return err;
+        }
+        hipLaunchKernelGGL(kern, dim3(d.units()), dim3(unit), lds, stream, const_cast<uint64_t*>(d_tbl), sc, src, d.R,
+                           d.E, d.K, d.max_tokens, d.units_per_rank(), arg);
+        return hipGetLastError();
+    };
+    // the fewer argument bytes the cheaper the launch (2 KB cost the host about a microsecond)
+    constexpr int kFew = (int)DF_COUNT * 8;
+    const int words = (int)DF_COUNT * d.R;
+    if (d.host_table != nullptr && words > kArgTableWords) return hipErrorInvalidValue;
+#define MCEP_COUNT(UNIT, TW) launch(count_kernel<UNIT, TW>, arg_table<TW>(d.host_table, words), UNIT)
+#define MCEP_COUNT_UNIT(UNIT)                                                                   \
+    (d.host_table == nullptr ? MCEP_COUNT(UNIT, 0)                                              \
+                             : (words <= kFew ? MCEP_COUNT(UNIT, kFew) : MCEP_COUNT(UNIT, kArgTableWords)))
+    hipError_t err = d.plan.shift == 10 ? MCEP_COUNT_UNIT(kBigUnitSelections) : MCEP_COUNT_UNIT(kUnitSelections);
+#undef MCEP_COUNT_UNIT
+#undef MCEP_COUNT
     if (err != hipSuccess) return err;
     if (d.plan.carried) return hipSuccess;   // the prefix pass rides in the pack launch
     const size_t plds = (size_t)kPrefixWaves * (d.units() + 1) * sizeof(int);
@@ -1744,12 +1777,16 @@ hipError_t launch_resolve(const uint64_t* d_tbl, CombineRoute* d_routes, uint32_
     if (total > 0x7fffffffll) return hipErrorInvalidValue;
     const int wpb = 4;
     const int blocks = (int)((total + wpb - 1) / wpb);
-    if (packed)
-        hipLaunchKernelGGL(resolve_kernel<true>, dim3(blocks), dim3(wpb * 64), 0, stream, d_tbl, d_routes, stamp, d.R,
-                           d.E, d.K, d.H, d.max_tokens, (int)total);
-    else
-        hipLaunchKernelGGL(resolve_kernel<false>, dim3(blocks), dim3(wpb * 64), 0, stream, d_tbl, d_routes, stamp, d.R,
-                           d.E, d.K, d.H, d.max_tokens, (int)total);
+    const int words = (int)CF_COUNT * d.R;
+    if (d.host_table != nullptr && words > kArgTableWords) return hipErrorInvalidValue;
+#define MCEP_RESOLVE(PACKED, TW)                                                                                   \
+    hipLaunchKernelGGL((resolve_kernel<PACKED, TW>), dim3(blocks), dim3(wpb * 64), 0, stream, d_tbl, d_routes, stamp, \
+                       d.R, d.E, d.K, d.H, d.max_tokens, (int)total, arg_table<TW>(d.host_table, words))
+    if (packed && d.host_table != nullptr) MCEP_RESOLVE(true, kArgTableWords);
+    else if (packed) MCEP_RESOLVE(true, 0);
+    else if (d.host_table != nullptr) MCEP_RESOLVE(false, kArgTableWords);
+    else MCEP_RESOLVE(false, 0);
+#undef MCEP_RESOLVE
     return hipGetLastError();
 }
 
@@ -1780,14 +1817,18 @@ static hipError_t launch_reduce_t(const ReduceLaunch& rl, const Dims& d, const T
     // 41.1 at 20).  The limit is imposed with unused dynamic LDS: a CU's 160 KiB hold so many blocks and no more.
     const int occupancy = t.combine_occupancy >= 0 ? t.combine_occupancy : (d.K >= 7 ? 20 : 0);
     const size_t pad = occupancy_pad_bytes(occupancy, wpb);
-#define MCEP_REDUCE(A, B)                                                                                        \
-    hipLaunchKernelGGL((reduce_kernel<KMAX, CH, A, B, DIRECT>), dim3(blocks), dim3(wpb * 64), pad, stream, rl.d_tbl, \
-                       rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row, d.R, d.E, d.K, d.max_tokens, d.H,    \
-                       slabs, d.Tgrid, (int)total)
-    if (ntl && nts) MCEP_REDUCE(true, true);
-    else if (ntl) MCEP_REDUCE(true, false);
-    else if (nts) MCEP_REDUCE(false, true);
-    else MCEP_REDUCE(false, false);
+    const int words = (int)CF_COUNT * d.R;
+    const bool in_args = d.host_table != nullptr && combine_reads_table(rl.src, DIRECT);
+    if (in_args && (words > kArgTableWords || !(ntl && nts))) return hipErrorInvalidValue;
+#define MCEP_REDUCE(A, B, TW)                                                                                    \
+    hipLaunchKernelGGL((reduce_kernel<KMAX, CH, A, B, DIRECT, TW>), dim3(blocks), dim3(wpb * 64), pad, stream,   \
+                       rl.d_tbl, rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row, d.R, d.E, d.K,             \
+                       d.max_tokens, d.H, slabs, d.Tgrid, (int)total, arg_table<TW>(d.host_table, words))
+    if (in_args) MCEP_REDUCE(true, true, kArgTableWords);
+    else if (ntl && nts) MCEP_REDUCE(true, true, 0);
+    else if (ntl) MCEP_REDUCE(true, false, 0);
+    else if (nts) MCEP_REDUCE(false, true, 0);
+    else MCEP_REDUCE(false, false, 0);
 #undef MCEP_REDUCE
     return hipGetLastError();
 }
@@ -1834,9 +1875,17 @@ static hipError_t launch_reduce_packed_t(const ReduceLaunch& rl, const float* d_
         blocks = rounds * 8 * group_blocks;
     }
     if (blocks > 0x7fffffffll) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((reduce_packed_kernel<KMAX, FP8, FACTOR, DIRECT, CH>), dim3((unsigned)blocks), dim3(wpb * 64), 0,
-                       stream, rl.d_tbl, rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row, d_factor, d.R, d.E, d.K,
-                       d.max_tokens, d.H, slabs, d.Tgrid, group_blocks);
+    const int words = (int)CF_COUNT * d.R;
+    const bool in_args = d.host_table != nullptr && combine_reads_table(rl.src, DIRECT);
+    if (in_args && words > kArgTableWords) return hipErrorInvalidValue;
+#define MCEP_PACKED(TW)                                                                                             \
+    hipLaunchKernelGGL((reduce_packed_kernel<KMAX, FP8, FACTOR, DIRECT, CH, TW>), dim3((unsigned)blocks),           \
+                       dim3(wpb * 64), 0, stream, rl.d_tbl, rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row,    \
+                       d_factor, d.R, d.E, d.K, d.max_tokens, d.H, slabs, d.Tgrid, group_blocks,                    \
+                       arg_table<TW>(d.host_table, words))
+    if (in_args) MCEP_PACKED(kArgTableWords);
+    else MCEP_PACKED(0);
+#undef MCEP_PACKED
     return hipGetLastError();
 }
 

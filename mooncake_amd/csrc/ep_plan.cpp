@@ -30,6 +30,14 @@ void plan_units(Dims& d, const Tuning& t) {
     d.plan = p;
 }
 
+bool combine_reads_table(const CombineSource& src, bool direct) {
+    if (src.tokens < 0 || src.out.base == 0) return true;
+    // rows come as addresses from the routes, except that the packed combine looks its tensors up either way
+    if (!direct) return src.x.base == 0 || (src.packed_fp8 && src.scales.base == 0);
+    return src.topk_idx.base == 0 || src.topk_weights.base == 0 || src.active.base == 0 || src.x.base == 0 ||
+           (src.packed_fp8 && src.scales.base == 0);
+}
+
 long long cast_back_chunks(long long max_rows, int num_experts) {
     // every row is in one chunk, and each expert has at most one partly filled chunk
     return (max_rows + kCastRows - 1) / kCastRows + num_experts;

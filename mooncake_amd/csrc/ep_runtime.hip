@@ -603,7 +603,9 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
                         "dispatch holds " + std::to_string(kStaticScratchBytes) + " (use mc_ep_world_dispatch)");
         // the table travels in kernel arguments on the call's own stream, every time: a recorded call
         // then carries its own copy, and nothing of the world's eager state is involved
-        if (!fused) {
+        if (!fused && (int)tbl_words <= kArgTableWords) {
+            d.host_table = tbl;
+        } else if (!fused) {
             MC_HIP(launch_table_write(s_tbl, tbl, (int)tbl_words, stream));
             w->launches += ((int)tbl_words + kTableChunk - 1) / kTableChunk;
         }
@@ -628,7 +630,17 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
                 stage = w->d_scale_stage;
             }
             const std::vector<uint64_t> tbl_vec(tbl, tbl + tbl_words);
-            if (int rc = upload_table(w, 0, tbl_vec, cap, stream, &d_tbl)) return rc;
+            if (!cap.active && (phases & MC_EP_PHASE_LAYOUT) && (int)tbl_words <= kArgTableWords) {
+                // a new table goes up with the count kernel (a recorded call's is in its own slot instead: what a
+                // replay wrote into the shared one, eager calls would not know of)
+                d_tbl = w->d_tbl[0];
+                if (w->tbl_cache[0] != tbl_vec) {
+                    d.host_table = tbl;
+                    w->tbl_cache[0].clear();              // until the launch has succeeded
+                }
+            } else if (int rc = upload_table(w, 0, tbl_vec, cap, stream, &d_tbl)) {
+                return rc;
+            }
         }
         sc = routing_scratch(w);
     }
@@ -664,6 +676,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     if (phases & MC_EP_PHASE_LAYOUT) {
         MC_HIP(launch_count(d_tbl, sc, src, d, stream));
         w->launches += d.plan.carried ? 1 : 2;    // the prefix pass is a launch of its own unless it rides in pack's
+        if (!static_scratch && d.host_table != nullptr) w->tbl_cache[0].assign(tbl, tbl + tbl_words);
         if (!static_scratch) remember(false);
     }
     if ((phases & (MC_EP_PHASE_DATA | MC_EP_PHASE_FINISH)) && tgrid > 0) {
@@ -726,8 +739,6 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     if (int rc = capture_of(stream, &cap)) return rc;
     RecordingScope recording(cap.active);
     if (int rc = order_begin(w, stream, cap)) return rc;
-    const uint64_t* d_tbl = nullptr;
-    if (int rc = upload_table(w, 1, tbl, cap, stream, &d_tbl)) return rc;
     Dims d{R, num_experts, num_topk, hidden, max_tokens, tgrid};
 
     // Is this the handle (and the routing input) of the last dispatch?  Then the
@@ -756,7 +767,20 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     src.out = uniform_ptr(out, R, uni);
     src.x = uniform_ptr(x, R, uni);
     if (ps.scales != nullptr) src.scales = uniform_ptr(ps.scales, R, uni);
+    src.packed_fp8 = ps.scales != nullptr;
+    src.active = uniform_ptr(active_ranks, R, uni);
     src.tokens = uniform_tokens(num_tokens, R, uni);
+    // The rank table: not needed when every tensor is evenly spaced, else in the kernels' arguments (a recorded call
+    // then carries its own), in memory only for worlds too large for that and for the streaming hints that have no
+    // such variant.
+    const uint64_t* d_tbl = nullptr;
+    if (!direct || combine_reads_table(src, direct)) {
+        if ((int)tbl.size() <= kArgTableWords && (ps.packed || (w->tuning.combine_nt & 3) == 3)) {
+            d.host_table = tbl.data();
+        } else if (int rc = upload_table(w, 1, tbl, cap, stream, &d_tbl)) {
+            return rc;
+        }
+    }
     // sized on every path, so that an eager call prepares the world for any recorded one of the same shape
     if (int rc = ensure_routes(w, (size_t)R * max_tokens * num_topk)) return rc;
     if (!direct) {

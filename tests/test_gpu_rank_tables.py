@@ -1,0 +1,66 @@
+"""Where a call's rank table comes from: kernel arguments (up to 288 words: 36 ranks of a dispatch, 32 of a combine),
+memory for larger worlds, or nowhere when every tensor is evenly spaced.  Two sets of tensors take turns on one world,
+so that every call finds another call's table behind it, on both sides of each limit, against the oracle."""
+import pytest
+import torch
+
+from mooncake_amd import _lib, ep
+from mooncake_amd.harness import WorldHarness
+from mooncake_amd.workloads import EPConfig, generate
+from tests.gpu_util import announce, compare_dispatch
+
+pytestmark = pytest.mark.gpu
+
+
+def _harness(cfg, world, seed, num_tokens):
+    h = WorldHarness(cfg, world=world, num_tokens=num_tokens)
+    h.data = generate(cfg, seed=seed)
+    h.load(h.data)
+    h.alloc_dispatch_outputs(poison=True)
+    h.alloc_combine_io()
+    h.expert_out.normal_(generator=torch.Generator(device="cuda").manual_seed(seed))
+    return h
+
+
+def _check(h, oracle, combined):
+    cfg = h.cfg
+    ref = oracle.dispatch(h.data["x"], h.data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
+    compare_dispatch(h, ref, check_poison=True)
+    want = oracle.combine(h.expert_out.cpu(), h.data["topk_idx"], h.data["topk_weights"], ref["src_info"],
+                          ref["layout_range"], h.num_tokens, cfg.max_tokens, cfg.num_experts)
+    for r, n in enumerate(h.num_tokens):
+        assert torch.equal(combined[r, :n].view(torch.int16), want[r, :n].view(torch.int16)), f"rank {r}"
+
+
+@pytest.mark.parametrize("uniform", [1, 0])
+@pytest.mark.parametrize("ragged", [False, True], ids=["full", "ragged"])
+@pytest.mark.parametrize("ranks", [1, 8, 9, 32, 33, 36, 37])
+def test_calls_take_turns_on_one_world(gpu_device, oracle, ranks, ragged, uniform):
+    cfg = EPConfig("tables", ranks, 8, 256, 2 * ranks, 2, True)
+    nt = [(r * 5) % 9 for r in range(ranks)] if ragged else None
+    announce(f"rank tables ranks={ranks} ragged={ragged} uniform={uniform}")
+    world = ep.World(ranks)
+    world.set_option("uniform", uniform)
+    world.set_option("fused_small", 0)
+    a, b = _harness(cfg, world, 1, nt), _harness(cfg, world, 2, nt)
+    for _ in range(2):
+        a.dispatch()
+        b.dispatch(phases=_lib.PHASE_LAYOUT)
+        b.dispatch(phases=_lib.PHASE_DATA)
+        b.dispatch(phases=_lib.PHASE_FINISH)
+        b.combine()                       # the last dispatch's handle
+        a.combine()                       # an older one
+        torch.cuda.synchronize()
+        for h in (a, b):
+            _check(h, oracle, h.combined.cpu())
+        plain = b.combined.clone()
+        b.expert_out.zero_()              # the packed combine must not look here
+        b.cast_back()
+        b.combine()
+        want = b.combined.clone()
+        b.combine_packed()
+        torch.cuda.synchronize()
+        for r, n in enumerate(b.num_tokens):
+            assert torch.equal(b.combined[r, :n].view(torch.int16), want[r, :n].view(torch.int16))
+        b.expert_out.normal_(generator=torch.Generator(device="cuda").manual_seed(2))
+        b.combined.copy_(plain)
