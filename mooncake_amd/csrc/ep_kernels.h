@@ -202,8 +202,7 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
                                 const RoutingScratch& sc, bool direct, const CombineSource& src, const void* d_zero_row,
                                 const float* d_factor, bool use_fp8, const Dims& d, const Tuning& t, hipStream_t stream);
 // packed rows below packed_recv_count -> bf16 rows times factor[expert]; max_rows bounds the world's valid rows
-// d_chunk_map: 16 bytes x (cast_back_chunks(max_rows, E) + 1) of scratch for the kernel's work list
-constexpr int kCastRows = 4;          // packed rows of one expert per work item of the cast-back kernel
+constexpr int kCastRows = 16;         // packed rows of one expert per work item of the cast-back kernel
 long long cast_back_chunks(long long max_rows, int num_experts);
 hipError_t launch_cast_back(const uint64_t* d_tbl, void* d_chunk_map, const float* d_factor, bool use_fp8,
                             long long max_rows, const Dims& d, hipStream_t stream);

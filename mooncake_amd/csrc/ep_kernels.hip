@@ -39,8 +39,8 @@
 //                   (mooncake_ep_kernel.cu:711-753); a selection counts while
 //                   topk_idx, as combine is given it, still names the expert
 //                   (:719-732).
-//   cast_chunks_kernel,  the consumer of the packed layout: valid rows back to
-//   cast_back_kernel     bf16, times a per-expert factor
+//   cast_back_kernel  the consumer of the packed layout: valid rows back to
+//                   bf16, times a per-expert factor
 //                   (per_token_cast_back, mooncake-wheel/tests/ep_test_utils.py:50-53;
 //                   the mock expert of mooncake-ep/tests/test_ep_grid.py:168-173).
 //   reduce_packed_kernel  combine fused with that consumer: reads dispatch's
@@ -1324,168 +1324,153 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
     }
 }
 
-// Work list of the cast-back kernel: which (expert, row chunk) each chunk
-// number is, from the packed_recv_count tensors alone; map[0].x is the number
-// of chunks.  Per block: a thread per expert fetches the count, one wave scans
-// ceil(count / kCastRows) over the experts in LDS, then a thread per chunk
-// finds its expert by bisection of the scanned begins.  It costs a launch, and
-// saves every block of the main kernel the same scan (a chain of dependent
-// loads) in front of its first row.
-constexpr int kCastWaves = 4;        // waves per block of the main kernel: kCastRows / kCastWaves rows each
-constexpr int kCastCols = 1024;
-constexpr int kCastMaxExperts = 4096;
-constexpr int kCastMapBlocks = 8;      // each repeats the scan (cheap) and writes an eighth of the entries
-
-__global__ __launch_bounds__(1024) void cast_chunks_kernel(const uint64_t* __restrict__ tbl, int4* __restrict__ map,
-                                                           int R, int E, int max_tokens, int max_chunks) {
-    __shared__ int lds_count[kCastMaxExperts];
-    __shared__ int lds_begin[kCastMaxExperts + 1];
-    const int lane = wave_lane();
-    const int L = E / R;
-    const int64_t RM = (int64_t)R * max_tokens;
-    for (int ee = threadIdx.x; ee < E; ee += blockDim.x) {
-        const int qq = ee / L;
-        const int32_t* cnt = (const int32_t*)tbl[XF_RECV_COUNT * R + qq];
-        int c = 0;
-        // a rank without tensors takes no part
-        if (cnt != nullptr && tbl[XF_RECV_X * R + qq] != 0 && tbl[XF_OUT * R + qq] != 0) c = cnt[ee - qq * L];
-        lds_count[ee] = c < 0 ? 0 : (c > RM ? (int)RM : c);
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        int carry = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int ee = e0 + lane;
-            const int n = (ee < E) ? (lds_count[ee] + kCastRows - 1) / kCastRows : 0;
-            const int incl = wave_scan_inclusive(n);
-            if (ee < E) lds_begin[ee] = carry + incl - n;
-            carry += __builtin_amdgcn_readlane(incl, 63);
-        }
-        if (lane == 0) {
-            lds_begin[E] = carry;
-            if (blockIdx.x == 0) map[0] = make_int4(carry < max_chunks ? carry : max_chunks, 0, 0, 0);
-        }
-    }
-    __syncthreads();
-    const int total = lds_begin[E] < max_chunks ? lds_begin[E] : max_chunks;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        // the last expert whose first chunk number is <= i (experts without rows share their successor's begin)
-        int lo = 0, hi = E;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (lds_begin[mid] <= i) lo = mid; else hi = mid;
-        }
-        map[1 + i] = make_int4(lo, i - lds_begin[lo], lds_count[lo], 0);
-    }
-}
-
 // A block takes one chunk (kCastRows consecutive packed rows of one expert)
-// times kCastCols columns, so only rows below packed_recv_count cost anything;
-// each of its kCastWaves waves converts one row of the chunk.  A lane owns two
-// pieces of 8 elements half the block's width apart: per piece 8 payload bytes
-// and one scale (fp8; the scales of a row sit R*max floats apart in the
-// column-major layout, and the four chunks that share their 64-byte sectors
-// run next to each other on one XCD) or 16 payload bytes (bf16), and one
-// 16-byte store that is contiguous across the wave.  No LDS.
-template <bool FP8>
-__global__ __launch_bounds__(kCastWaves * 64) void cast_back_kernel(const uint64_t* __restrict__ tbl,
-                                                         const int4* __restrict__ map,
+// times kCastCols columns, so only rows below packed_recv_count cost anything.
+// Which expert the block's chunk number belongs to follows from the counts
+// alone, and every block finds it by itself: a thread adds up ceil(count /
+// kCastRows) over a run of experts, the block scans the sums, and the thread
+// whose run holds the number says which.  That is one load and two barriers in
+// front of the first row, where a work list cost a launch (5 us) and a load.
+//
+// Each of the kCastWaves waves converts kCastRows / kCastWaves consecutive rows,
+// all their loads in flight together (with one row per wave the kernel was held
+// up by its own latency: 252 -> 237 us for 65 536 fp8 rows of 7168, 232 with the
+// output written through the L2).  A lane owns two pieces of 8 elements half the
+// block's width apart: per piece and row 8 payload bytes (fp8) or 16 (bf16), one
+// 16-byte store that is contiguous across the wave, and for all four rows one
+// 16-byte load of scales, which lie next to each other in the column-major
+// layout - a block's 16 rows are a 64-byte sector of it, so no sector is fetched
+// twice.  Whole cycles with the output stored this way / streamed / plainly:
+// 8 x 256 tokens fp8 144.8 / 150.4 / - us, 32 x 128 271.9 / 276.7 / -, 8 x 1024
+// 533.0 / 533.3 / 538.1, Mixtral 107.5 / 105.8 / 108.3; the payload, read once,
+// is better loaded with the streaming hint (bf16, 8 x 512: 187 against 201).
+constexpr int kCastWaves = 4;
+constexpr int kCastCols = 1024;
+
+template <bool FP8, int TW>
+__global__ __launch_bounds__(kCastWaves * 64) void cast_back_kernel(const uint64_t* __restrict__ tbl_mem, RankPtr counts,
                                                          const float* __restrict__ factor, int R, int E, int H,
-                                                         int max_tokens, int parts, int max_chunks) {
+                                                         int max_tokens, int parts, ArgTable<TW> arg_tbl) {
+    const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
+    __shared__ int lds_wave[kCastWaves];
+    __shared__ int lds_item[3];
     const int lane = wave_lane();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // Blocks go round-robin over the 8 XCDs, each with an L2 of its own.  The four chunks that share
-    // 64-byte sectors of scales (16 consecutive rows of one group) are therefore given to four blocks
-    // of the same XCD, next to each other in launch order: block = (set / 8 * 4 + chunk % 4) * 8 + set % 8,
-    // with set = (chunk / 4) * parts + part.
-    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
-    const int set = (seq >> 2) * 8 + xcd;
-    const int part = set % parts;
-    const int target = (set / parts) * 4 + (seq & 3);
+    const int target = blockIdx.x / parts, part = blockIdx.x - target * parts;
     const int L = E / R;
     const int64_t RM = (int64_t)R * max_tokens;
-    const int total = map[0].x;
-    const int4 item = map[1 + (target < max_chunks ? target : 0)];
-    if (target >= total) return;            // block-uniform
-    const int e = __builtin_amdgcn_readfirstlane(item.x);
-    const int chunk = __builtin_amdgcn_readfirstlane(item.y);
-    const int count = __builtin_amdgcn_readfirstlane(item.z);
+
+    // this thread's run of experts
+    const int run = (E + kCastWaves * 64 - 1) / (kCastWaves * 64);
+    const int e_first = threadIdx.x * run;
+    auto valid_rows = [&](int ee) -> int {
+        if (ee >= E) return 0;
+        const int qq = ee / L;
+        const uint64_t cnt = rank_ptr(tbl, counts, XF_RECV_COUNT, R, qq);
+        // a rank without tensors takes no part (evenly spaced counts are those of ranks that all do)
+        if (counts.base == 0 && (cnt == 0 || tbl[XF_RECV_X * R + qq] == 0 || tbl[XF_OUT * R + qq] == 0)) return 0;
+        const int c = load_i32(cnt + (uint64_t)(ee - qq * L) * 4);
+        return c < 0 ? 0 : (c > RM ? (int)RM : c);
+    };
+    int chunks = 0;
+    for (int i = 0; i < run; ++i) chunks += (valid_rows(e_first + i) + kCastRows - 1) / kCastRows;
+    const int incl = wave_scan_inclusive(chunks);
+    if (lane == 63) lds_wave[wave] = incl;
+    if (threadIdx.x == 0) lds_item[0] = -1;
+    __syncthreads();
+    int begin = incl - chunks;
+#pragma unroll
+    for (int w = 0; w < kCastWaves - 1; ++w) begin += w < wave ? lds_wave[w] : 0;
+    if (begin <= target && target < begin + chunks) {
+        for (int i = 0; i < run; ++i) {
+            const int c = valid_rows(e_first + i), n = (c + kCastRows - 1) / kCastRows;
+            if (target < begin + n) {
+                lds_item[0] = e_first + i;
+                lds_item[1] = target - begin;
+                lds_item[2] = c;
+                break;
+            }
+            begin += n;
+        }
+    }
+    __syncthreads();
+    const int e = __builtin_amdgcn_readfirstlane(lds_item[0]);
+    if (e < 0) return;                      // beyond the last chunk
+    const int row0 = __builtin_amdgcn_readfirstlane(lds_item[1]) * kCastRows + wave * (kCastRows / kCastWaves);
+    const int count = __builtin_amdgcn_readfirstlane(lds_item[2]);
+    if (row0 >= count) return;              // wave-uniform
 
     const int q = e / L, le = e - q * L;
     const int G = H / 128;
     const int col0 = part * kCastCols;
     const int ncols = (H - col0 < kCastCols) ? (H - col0) : kCastCols;
-    const int row0 = chunk * kCastRows;
     const float f = factor != nullptr ? factor[e] : 1.0f;
-    const uint8_t* in = (const uint8_t*)tbl[XF_RECV_X * R + q];
-    uint8_t* out = (uint8_t*)tbl[XF_OUT * R + q];
+    const uint64_t in = tbl[XF_RECV_X * R + q], out = tbl[XF_OUT * R + q];
 
     // A lane owns two pieces of 8 elements, half a block's width apart, so that each
     // of its two 16-byte stores lands in a run of 1 KB written by the wave as a whole.
     // Piece p covers columns col0 + p * 512 + lane * 8 .. + 7; 16 lanes share a scale group.
     constexpr int kHalf = kCastCols / 2;
+    constexpr int kWaveRows = kCastRows / kCastWaves;
+    static_assert(kWaveRows == 4, "the scales of a wave's rows are one 16-byte load");
+    const int64_t grow = (int64_t)le * RM + row0;
+    uint4 v[kWaveRows][2];
+    // (four floats at any 4-byte address: where R * max_tokens is no multiple of four a row's scales start anywhere)
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    f4 sv[2];
     bool on[2];
-    int64_t in_off[2], out_off[2];
-    const float* scale_col[2];
+    int col[2];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-        const int col = p * kHalf + lane * 8;
-        on[p] = col < ncols;
-        const int c = on[p] ? col : 0;
-        in_off[p] = (int64_t)(col0 + c) * (FP8 ? 1 : 2);
-        out_off[p] = (int64_t)(col0 + c) * 2;
-        scale_col[p] = FP8 ? (const float*)tbl[XF_RECV_SCALES * R + q] + ((int64_t)le * G + (col0 + c) / 128) * RM
-                           : nullptr;
-    }
-
-    constexpr int kWaveRows = kCastRows / kCastWaves;
-    constexpr int kBatch = kWaveRows < 8 ? kWaveRows : 8;   // rows whose loads are in flight together
-    const int64_t row_base = (int64_t)le * RM;
-    for (int b = 0; b < kWaveRows; b += kBatch) {
-        const int r_first = row0 + wave * kWaveRows + b;
-        if (r_first >= count) break;
-        uint4 v[kBatch][2];
-        float sv[kBatch][2];
+        const int c = p * kHalf + lane * 8;
+        on[p] = c < ncols;
+        col[p] = col0 + (on[p] ? c : 0);
+        if (FP8) {
+            const uint64_t column = tbl[XF_RECV_SCALES * R + q] + (uint64_t)(((int64_t)le * G + col[p] / 128) * RM) * 4;
+            if (row0 + kWaveRows <= RM) {
+                sv[p] = *(const MCEP_GLOBAL f4*)(uintptr_t)(column + (uint64_t)row0 * 4);
+            } else {
 #pragma unroll
-        for (int i = 0; i < kBatch; ++i) {
-            const int row = r_first + i < count ? r_first + i : r_first;
-            const uint8_t* src = in + (row_base + row) * H * (FP8 ? 1 : 2);
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                if (FP8) {
-                    const uint2 w = *(const uint2*)(src + in_off[p]);
-                    v[i][p] = make_uint4(w.x, w.y, 0u, 0u);
-                    sv[i][p] = scale_col[p][row];
-                } else {
-                    v[i][p] = load16<true>(src + in_off[p]);
-                }
+                for (int i = 0; i < kWaveRows; ++i)
+                    sv[p][i] = load_f32(column + (uint64_t)(row0 + (row0 + i < count ? i : 0)) * 4);
             }
         }
 #pragma unroll
-        for (int i = 0; i < kBatch; ++i) {
-            if (r_first + i >= count) break;       // wave-uniform
-            uint8_t* dst = out + (row_base + r_first + i) * H * 2;
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                uint32_t o[4];
-                if (FP8) {
-                    typedef float f2 __attribute__((ext_vector_type(2)));
-                    const f2 a0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].x, false);
-                    const f2 a1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].x, true);
-                    const f2 a2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].y, false);
-                    const f2 a3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].y, true);
-                    const float sc = sv[i][p];
-                    o[0] = scale_round_twice(a0.x, a0.y, sc, f);
-                    o[1] = scale_round_twice(a1.x, a1.y, sc, f);
-                    o[2] = scale_round_twice(a2.x, a2.y, sc, f);
-                    o[3] = scale_round_twice(a3.x, a3.y, sc, f);
-                } else {
-                    const uint32_t w[4] = {v[i][p].x, v[i][p].y, v[i][p].z, v[i][p].w};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) o[j] = pack_bf16_rne(bf16_lo(w[j]) * f, bf16_hi(w[j]) * f);
-                }
-                if (on[p]) store16<false>(dst + out_off[p], make_uint4(o[0], o[1], o[2], o[3]));
+        for (int i = 0; i < kWaveRows; ++i) {
+            const int64_t row = grow + (row0 + i < count ? i : 0);
+            const uint64_t src = in + (uint64_t)(row * H + col[p]) * (FP8 ? 1 : 2);
+            if (FP8) {
+                const u32x2 w = __builtin_nontemporal_load((const MCEP_GLOBAL u32x2*)(uintptr_t)src);
+                v[i][p] = make_uint4(w.x, w.y, 0u, 0u);
+            } else {
+                v[i][p] = load16<true>((const void*)src);
             }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kWaveRows; ++i) {
+        if (row0 + i >= count) break;       // wave-uniform
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            uint32_t o[4];
+            if (FP8) {
+                typedef float f2 __attribute__((ext_vector_type(2)));
+                const f2 a0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].x, false);
+                const f2 a1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].x, true);
+                const f2 a2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].y, false);
+                const f2 a3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v[i][p].y, true);
+                const float sc = sv[p][i];
+                o[0] = scale_round_twice(a0.x, a0.y, sc, f);
+                o[1] = scale_round_twice(a1.x, a1.y, sc, f);
+                o[2] = scale_round_twice(a2.x, a2.y, sc, f);
+                o[3] = scale_round_twice(a3.x, a3.y, sc, f);
+            } else {
+                const uint32_t w[4] = {v[i][p].x, v[i][p].y, v[i][p].z, v[i][p].w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = pack_bf16_rne(bf16_lo(w[j]) * f, bf16_hi(w[j]) * f);
+            }
+            const uint64_t dst = out + (uint64_t)(grow + i) * (uint64_t)H * 2;
+            if (on[p]) store16_row<kStoreThrough>(dst, col[p] * 2, make_uint4(o[0], o[1], o[2], o[3]), H * 2);
         }
     }
 }
@@ -1918,26 +1903,34 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
 #undef MCEP_P4
 }
 
-hipError_t launch_cast_back(const uint64_t* d_tbl, void* d_chunk_map, const float* d_factor, bool use_fp8,
+hipError_t launch_cast_back(const uint64_t* d_tbl, void* /*scratch: none needed*/, const float* d_factor, bool use_fp8,
                             long long max_rows, const Dims& d, hipStream_t stream) {
     const int parts = (d.H + kCastCols - 1) / kCastCols;
-    const long long chunks = cast_back_chunks(max_rows, d.E);
-    const long long total = chunks * parts;
-    if (total <= 0) return hipSuccess;
-    if (total > 0x7fffffffll || d.E > kCastMaxExperts) return hipErrorInvalidValue;
-    int4* map = (int4*)d_chunk_map;
-    hipLaunchKernelGGL(cast_chunks_kernel, dim3(kCastMapBlocks), dim3(1024), 0, stream, d_tbl, map, d.R, d.E, d.max_tokens,
-                       (int)chunks);
-    // sets of four chunks times parts, rounded up to whole rounds over the 8 XCDs
-    const long long sets = (chunks + 3) / 4 * parts;
-    const long long blocks = (sets + 7) / 8 * 8 * 4;
+    const long long blocks = cast_back_chunks(max_rows, d.E) * parts;
+    if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffffll) return hipErrorInvalidValue;
-    if (use_fp8)
-        hipLaunchKernelGGL(cast_back_kernel<true>, dim3((unsigned)blocks), dim3(kCastWaves * 64), 0, stream, d_tbl, map,
-                           d_factor, d.R, d.E, d.H, d.max_tokens, parts, (int)chunks);
-    else
-        hipLaunchKernelGGL(cast_back_kernel<false>, dim3((unsigned)blocks), dim3(kCastWaves * 64), 0, stream, d_tbl,
-                           map, d_factor, d.R, d.E, d.H, d.max_tokens, parts, (int)chunks);
+    // The table is in the arguments, with the counts' address and spacing beside it where they are even: one
+    // dependent load less in front of every block.
+    constexpr int kWords = (int)XF_COUNT * 32;
+    const int words = (int)XF_COUNT * d.R;
+    if (d.host_table != nullptr && words > kWords) return hipErrorInvalidValue;
+    RankPtr counts;
+    if (d.host_table != nullptr) {
+        const uint64_t* c = d.host_table + (size_t)XF_RECV_COUNT * d.R;
+        bool even = true;
+        const int64_t stride = d.R > 1 ? (int64_t)(c[1] - c[0]) : 0;
+        for (int r = 0; r < d.R; ++r)
+            even = even && c[r] != 0 && c[r] == c[0] + (uint64_t)(stride * r) && d.host_table[XF_RECV_X * d.R + r] != 0;
+        if (even) counts = RankPtr{c[0], stride};
+    }
+#define MCEP_CAST(FP8, TW)                                                                                          \
+    hipLaunchKernelGGL((cast_back_kernel<FP8, TW>), dim3((unsigned)blocks), dim3(kCastWaves * 64), 0, stream, d_tbl, \
+                       counts, d_factor, d.R, d.E, d.H, d.max_tokens, parts, arg_table<TW>(d.host_table, words))
+    if (use_fp8 && d.host_table != nullptr) MCEP_CAST(true, kWords);
+    else if (use_fp8) MCEP_CAST(true, 0);
+    else if (d.host_table != nullptr) MCEP_CAST(false, kWords);
+    else MCEP_CAST(false, 0);
+#undef MCEP_CAST
     return hipGetLastError();
 }
 

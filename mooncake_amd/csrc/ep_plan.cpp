@@ -1,6 +1,6 @@
 // Host-side planning shared by the runtime and the kernel launchers: how a world's selections are cut
-// into units, what the count kernel needs of LDS, how many work items the cast-back kernel's list can
-// hold.  Plain C++ (no device code), so that the runtime's bookkeeping can also be built and exercised on
+// into units, what the count kernel needs of LDS, how many work items the cast-back kernel has to
+// cover.  Plain C++ (no device code), so that the runtime's bookkeeping can also be built and exercised on
 // a machine without a GPU.
 #include "ep_kernels.h"
 
@@ -39,8 +39,9 @@ bool combine_reads_table(const CombineSource& src, bool direct) {
 }
 
 long long cast_back_chunks(long long max_rows, int num_experts) {
-    // every row is in one chunk, and each expert has at most one partly filled chunk
-    return (max_rows + kCastRows - 1) / kCastRows + num_experts;
+    // every row is in one chunk, each expert has at most one partly filled chunk, and no chunk is empty
+    const long long chunks = max_rows / kCastRows + num_experts;
+    return chunks < max_rows ? chunks : max_rows;
 }
 
 }  // namespace mcep

@@ -199,6 +199,10 @@ class World:
                   stream_ptr: int) -> None:
         """Valid packed rows -> bf16 rows (fp8 payload times its scales; bf16 payload when
         recv_scales_ptrs is None), times expert_factor[expert] when a factor array is given."""
+        if self._native is not None:
+            self._native.cast_back(recv_x_ptrs, recv_scales_ptrs, recv_count_ptrs, expert_factor_ptr, out_ptrs, hidden,
+                                   num_topk, num_max_dispatch_tokens_per_rank, num_experts, stream_ptr)
+            return
         u = _lib.u64_array
         _lib.check(_lib.lib().mc_ep_world_cast_back(
             self._h, u(recv_x_ptrs), u(recv_scales_ptrs) if recv_scales_ptrs is not None else None,
