@@ -725,126 +725,180 @@ __global__ __launch_bounds__(512) void pack_bf16_kernel(const uint64_t* __restri
 // ---------------------------------------------------------------------------
 // When the whole world names a few thousand selections (a decode step of one rank, or of a few), the
 // three launches above cost more than the bytes they move: each is close to the floor of an empty
-// kernel.  Here every wave rebuilds the routing it needs by itself, from the ranks' index lists, so one
+// kernel.  Here every block rebuilds the routing it needs by itself, from the ranks' index lists, so one
 // launch does everything - as the reference's dispatch is one launch (mooncake_ep_kernel.cu:138-470).
-// The row of a selection is the number of earlier selections (source rank ascending, then token, then
-// k) that name the same expert: a data wave reads the lists of the earlier ranks and its own rank's up
-// to its token (16-byte loads, two entries per lane, a few KB out of L2) and counts matches for its
-// token's K experts at once.  The first E waves count one expert each over the whole lists and write
-// recv_count and layout_range.  fp8 scales go straight into the column-major layout (4-byte stores 16 KB
-// apart: costly for a large world, nothing next to a launch here).  The rank table travels in the
-// kernel's arguments, so there is no table to upload; nothing is shared between waves, no LDS, no atomics.
-// The slab-0 wave of a token leaves selrow for a combine of the same handle.
-typedef long long i64x2 __attribute__((ext_vector_type(2)));
+// What bounds it is the chain of loads in front of the stores.  The row of a selection is the number of
+// earlier selections (source rank ascending, then token, then k) that name the same expert.  A block is one
+// token, a wave per 1024-element slab of it; its waves share out the lists of the earlier ranks, and of the own
+// rank up to the token, in rounds of kSmallListRound entries and count them into one LDS histogram of the experts
+// (one LDS addition per entry; comparing every entry with each of the token's experts by lane masks was bound by
+// those instructions: 10.4 against 8.5 us for 12 ragged ranks of 70 tokens).  The first round's loads leave before
+// the token's own experts are known, every other round's before the one in front of it is counted; a lane's loads
+// are single entries, so a list may start anywhere.  The first blocks take kSmallExperts experts each over the
+// whole lists, shared out in the same way, and write recv_count and layout_range.  Rows are written through the L2
+// (0.6 to 1.5 us faster than ordinary stores, whose write-back the end of the kernel waits for); fp8 scales go
+// straight into the column-major layout (4-byte stores 16 KB apart: costly for a large world, nothing next to a
+// launch here).  The rank table travels in the kernel's arguments, so there is no table to upload; nothing is
+// shared between blocks.  The slab-0 wave of a token leaves selrow for a combine of the same handle.
+// Kernel, when every wave counted all the lists by itself -> now: 1 x 128 tokens, hidden 7168, top-8, fp8 7.3 -> 6.3 us;
+// 4 x 128, 2048, top-4, bf16 7.1 -> 5.6; 1 x 384, 7168, top-8, fp8 14.1 -> 9.3.  Against count + pack + transpose, which
+// these took: 8 x 64, 4096, top-6, fp8 3.2 + 6.5 + 4.0 (and two gaps) -> 7.4; 12 ragged ranks of 70, 1152, top-5, fp8
+// 3.4 + 5.0 + 4.8 -> 8.5; 16 x 32 and 32 x 16, 7168, top-8, fp8 17 -> 12.2 and 14.6.
+constexpr int kSmallExperts = 8;
+constexpr int kSmallSpan = 4096;                    // experts a data block counts at a time (16 KB of LDS)
+constexpr int kSmallDepth = kSmallListRound / 64;   // entries per lane and round
 
-// counts, per lane, the entries of list[0, n) that equal each of ek[0..KMAX): list and n are wave-uniform;
-// entries outside [0, E) equal nothing (targets are in [0, E) or -2)
-template <int KMAX>
-__device__ __forceinline__ void count_list(uint64_t list, int n, int E, const int (&ek)[KMAX], int (&cnt)[KMAX],
-                                           int lane) {
-    constexpr int kDepth = 4;             // 16-byte loads in flight per lane
-    static_assert(kDepth * 128 == kSmallListRound, "the host prices a world in rounds of this many entries");
-    if ((list & 8) != 0 && n > 0) {
-        // a list that starts in the middle of a 16-byte unit (rank r's slice of a rank-major tensor with an
-        // odd number of entries per rank): its first entry by itself, pairs from there
-        if (lane == 0) {
-            const int64_t v = *(const MCEP_GLOBAL int64_t*)(uintptr_t)list;
-            const int k0 = (uint64_t)v < (uint64_t)E ? (int)v : -1;
-#pragma unroll
-            for (int k = 0; k < KMAX; ++k) cnt[k] += k0 == ek[k] ? 1 : 0;
-        }
-        list += 8;
-        n -= 1;
+// A wave's way through the ranks' index lists: every `waves`-th round of kSmallListRound entries of the lists of
+// ranks 0 .. last_rank, the last one only up to last_len.  Everything but the entries is wave-uniform.
+struct ListWalk {
+    const uint64_t* tbl;
+    uint64_t readable;                 // 8 bytes anywhere
+    int R, K, last_rank, last_len, parts, waves;
+    int rank, part;
+
+    __device__ __forceinline__ ListWalk(const uint64_t* table, uint64_t anything, int ranks, int k, int rank_end,
+                                        int len_end, int most, int n_waves, int wave)
+        : tbl(table), readable(anything), R(ranks), K(k), last_rank(rank_end), last_len(len_end),
+          parts((most + kSmallListRound - 1) / kSmallListRound), waves(n_waves), rank(0), part(wave) {
+        settle();
     }
-    for (int base = 0; base < n; base += kDepth * 128) {
-        i64x2 v[kDepth];
-#pragma unroll
-        for (int j = 0; j < kDepth; ++j) {
-            const int i = base + j * 128 + 2 * lane;
-            v[j] = i64x2{-1, -1};
-            if (i + 1 < n) v[j] = *(const MCEP_GLOBAL i64x2*)(uintptr_t)(list + (uint64_t)i * 8);
-            else if (i < n) v[j].x = *(const MCEP_GLOBAL int64_t*)(uintptr_t)(list + (uint64_t)i * 8);
-        }
-#pragma unroll
-        for (int j = 0; j < kDepth; ++j) {
-            const int k0 = (uint64_t)v[j].x < (uint64_t)E ? (int)v[j].x : -1;
-            const int k1 = (uint64_t)v[j].y < (uint64_t)E ? (int)v[j].y : -1;
-#pragma unroll
-            for (int k = 0; k < KMAX; ++k) cnt[k] += (k0 == ek[k] ? 1 : 0) + (k1 == ek[k] ? 1 : 0);
+    __device__ __forceinline__ void settle() {
+        while (part >= parts) {
+            part -= parts;
+            ++rank;
         }
     }
+    __device__ __forceinline__ bool more() const {
+        return rank < last_rank || (rank == last_rank && part * kSmallListRound < last_len);
+    }
+    // Asks for the next round's entries: how many there are (none or fewer: nothing to count) and whose they are.
+    // Nothing is loaded under a branch, so that a round's loads leave back to back and the round before it is not
+    // waited for: a lane beyond the last entry loads that one again, a round without entries something else.
+    __device__ __forceinline__ int fetch(int64_t (&v)[kSmallDepth], int* whose) {
+        const int lane = wave_lane();
+        const int r = rank < last_rank ? rank : last_rank;
+        const int tokens = (int)tbl[DF_NUM_TOKENS * R + r];
+        const uint64_t entries = tbl[DF_TOPK_IDX * R + r];
+        const int first = part * kSmallListRound;
+        const int n = more() ? (rank < last_rank ? tokens * K : last_len) - first : 0;
+        const uint64_t list = n > 0 ? entries + (uint64_t)first * 8 : readable;
+        const int last = n > 0 ? n - 1 : 0;
+#pragma unroll
+        for (int j = 0; j < kSmallDepth; ++j) {
+            const int i = j * 64 + lane;
+            v[j] = *(const MCEP_GLOBAL int64_t*)(uintptr_t)(list + (uint64_t)(i < last ? i : last) * 8);
+        }
+        *whose = r;
+        part += waves;
+        settle();
+        return n;
+    }
+};
+
+// Adds a round's n entries to the histogram of the experts first .. first + span - 1 in LDS; entries outside that range
+// (and so outside [0, E)) name nothing.
+__device__ __forceinline__ void count_round(const int64_t (&v)[kSmallDepth], int n, int first, int span, int* hist) {
+    const int lane = wave_lane();
+#pragma unroll
+    for (int j = 0; j < kSmallDepth; ++j) {
+        if (j * 64 >= n) break;
+        const uint64_t at = (uint64_t)(v[j] - (int64_t)first);
+        if (j * 64 + lane < n && at < (uint64_t)span) atomicAdd(&hist[(int)at], 1);
+    }
+    // every load of the round has arrived here: one still in flight into a register that the next round's addresses
+    // or entries take would have that round wait for this one's successor as well
+#pragma unroll
+    for (int j = 0; j < kSmallDepth; ++j) asm volatile("" ::"v"(v[j]));
 }
 
-__device__ __forceinline__ int wave_total(int v) { return __builtin_amdgcn_readlane(wave_scan_inclusive(v), 63); }
-
-// recv_count and layout_range of expert ee, by one wave: its selections in every rank's list
-__device__ __forceinline__ void small_expert(const SmallTable& tb, int R, int E, int K, int max_tokens, int ee) {
+// recv_count and layout_range of kSmallExperts experts from e0 on, by one block: their selections in every rank's list
+__device__ __forceinline__ void small_experts(const uint64_t* tbl, const int32_t* selrow, int R, int E, int K,
+                                              int max_tokens, int Tgrid, int e0, int wave, int waves) {
+    __shared__ int lds_cnt[kSmallRanks * kSmallExperts];
     const int lane = wave_lane();
-    const int L = E / R, q = ee / L, le = ee - q * L;
+    ListWalk walk(tbl, (uint64_t)(uintptr_t)selrow, R, K, R - 1, (int)tbl[DF_NUM_TOKENS * R + R - 1] * K, Tgrid * K, waves,
+                  wave);
+    int64_t v[2][kSmallDepth];
+    int whose[2] = {0, 0}, n[2];
+    bool go = walk.more();
+    n[0] = walk.fetch(v[0], &whose[0]);
+    for (int i = threadIdx.x; i < kSmallRanks * kSmallExperts; i += blockDim.x) lds_cnt[i] = 0;
+    __syncthreads();
+    auto take = [&](int i) {                                      // counts round i while the other one is on its way
+        const bool another = walk.more();
+        n[1 - i] = walk.fetch(v[1 - i], &whose[1 - i]);
+        count_round(v[i], n[i], e0, E - e0 < kSmallExperts ? E - e0 : kSmallExperts, lds_cnt + whose[i] * kSmallExperts);
+        return another;
+    };
+    if (go)
+        for (;;) {
+            if (!take(0)) break;
+            if (!take(1)) break;
+        }
+    __syncthreads();
+
+    const int L = E / R;
     const int64_t RM = (int64_t)R * max_tokens;
     const int cap = (int)(RM < 0x7fffffff ? RM : 0x7fffffff);   // rows past a block's capacity are dropped
-    const int target[1] = {ee};
-    int run = 0, mine_b = 0, mine_e = 0;
-    for (int rr = 0; rr < R; ++rr) {
-        int c[1] = {0};
-        count_list<1>(tb.v[DF_TOPK_IDX * R + rr], (int)tb.v[DF_NUM_TOKENS * R + rr] * K, E, target, c, lane);
-        const int total = wave_total(c[0]);
-        if (lane == rr) {
-            mine_b = run;
-            mine_e = run + total;
+    for (int k = wave; k < kSmallExperts && e0 + k < E; k += waves) {
+        const int ee = e0 + k, q = ee / L, le = ee - q * L;
+        const int c = lane < R ? lds_cnt[lane * kSmallExperts + k] : 0;
+        const int end = wave_scan_inclusive(c), begin = end - c;
+        const int total = __builtin_amdgcn_readlane(end, 63);
+        if (tbl[DF_RECV_X * R + q] == 0) continue;              // the rank takes no part and receives nothing
+        if (lane == 0) *(MCEP_GLOBAL int32_t*)(uintptr_t)(tbl[DF_RECV_COUNT * R + q] + (uint64_t)le * 4) = total < cap ? total : cap;
+        if (lane < R) {
+            const int b = begin < cap ? begin : cap, b2 = end < cap ? end : cap;
+            // count in the low half, begin in the high half; an empty pair is 0
+            *(MCEP_GLOBAL int64_t*)(uintptr_t)(tbl[DF_LAYOUT_RANGE * R + q] + (uint64_t)(le * R + lane) * 8) =
+                (b2 > b) ? (((int64_t)b << 32) | (int64_t)(b2 - b)) : 0;
         }
-        run += total;
-    }
-    const uint64_t recv_x = tb.v[DF_RECV_X * R + q];              // 0: the rank takes no part and receives nothing
-    if (recv_x == 0) return;
-    if (lane == 0) ((int32_t*)tb.v[DF_RECV_COUNT * R + q])[le] = run < cap ? run : cap;
-    if (lane < R) {
-        const int b = mine_b < cap ? mine_b : cap, b2 = mine_e < cap ? mine_e : cap;
-        // count in the low half, begin in the high half; an empty pair is 0
-        ((int64_t*)tb.v[DF_LAYOUT_RANGE * R + q])[(int64_t)le * R + lane] =
-            (b2 > b) ? (((int64_t)b << 32) | (int64_t)(b2 - b)) : 0;
     }
 }
 
-template <int KMAX, bool FP8, bool NATIVE>
-__global__ __launch_bounds__(256) void dispatch_small_kernel(SmallTable tb, int32_t* __restrict__ selrow, int R, int E,
-                                                              int K, int max_tokens, int H, int slabs, int Tgrid,
-                                                              int total_tasks) {
+template <bool FP8, bool NATIVE, int TW>
+__global__ __launch_bounds__(kSmallWaves * 64) void dispatch_small_kernel(ArgTable<TW> tb, int32_t* __restrict__ selrow,
+                                                                          int R, int E, int K, int max_tokens, int H,
+                                                                          int slabs, int Tgrid, int expert_blocks) {
     const int lane = wave_lane();
-    int task = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
-    if (task >= total_tasks) return;
-    if (task < E) {
-        small_expert(tb, R, E, K, max_tokens, task);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    if ((int)blockIdx.x < expert_blocks) {
+        small_experts(tb.v, selrow, R, E, K, max_tokens, Tgrid, blockIdx.x * kSmallExperts, wave, waves);
         return;
     }
-    task -= E;
-    const int n = task / slabs, s = task - n * slabs;
+    const int n = blockIdx.x - expert_blocks;
     const int r = n / Tgrid, t = n - r * Tgrid;
-    if (t >= (int)tb.v[DF_NUM_TOKENS * R + r]) return;
-    const char* xtok = (const char*)tb.v[DF_X * R + r] + (int64_t)t * H * 2;
-    const uint64_t own_list = tb.v[DF_TOPK_IDX * R + r];
+    const int T = (int)tb.v[DF_NUM_TOKENS * R + r];
+    const uint64_t own_list = tb.v[DF_TOPK_IDX * R + r], own_x = tb.v[DF_X * R + r];
+    asm volatile("" ::"s"(T), "s"(own_list), "s"(own_x));         // (one wait for the three)
+    if (t >= T) return;                                           // the whole block
+    const char* xtok = (const char*)own_x + (int64_t)t * H * 2;
 
     // the payload loads first: everything below hides behind them
     constexpr int kSlabBytes = 2048;
-    const int elem0 = s * 1024 + lane * (FP8 ? 16 : 8);          // bf16: the first of two 512-element halves
-    uint4 a = make_uint4(0, 0, 0, 0), b = a;
+    uint4 a, b;
     bool act_a, act_b;
-    if (FP8) {
-        act_a = act_b = elem0 < H;
-        if (act_a) {
-            a = load16<false>(xtok + (int64_t)elem0 * 2);
-            b = load16<false>(xtok + (int64_t)elem0 * 2 + 16);
-        }
-    } else {
+    int elem0;
+    auto load_slab = [&](int s) {
+        elem0 = s * 1024 + lane * (FP8 ? 16 : 8);                // bf16: the first of two 512-element halves
         act_a = elem0 < H;
-        act_b = elem0 + 512 < H;
+        act_b = FP8 ? act_a : elem0 + 512 < H;
+        a = b = make_uint4(0, 0, 0, 0);
         if (act_a) a = load16<false>(xtok + (int64_t)elem0 * 2);
-        if (act_b) b = load16<false>(xtok + (int64_t)elem0 * 2 + kSlabBytes / 2);
-    }
+        if (act_b) b = load16<false>(xtok + (int64_t)elem0 * 2 + (FP8 ? 16 : kSlabBytes / 2));
+    };
+    load_slab(wave);
 
-    // the token's K experts, one per lane, and each as a wave-uniform target
+    // the token's K experts, one per lane, and the first round of the lists in front of it
     const int li = lane < K ? lane : 0;
     const int64_t e64 = *(const MCEP_GLOBAL int64_t*)(uintptr_t)(own_list + (uint64_t)((int64_t)t * K + li) * 8);
+    const auto lists = [&] { return ListWalk(tb.v, own_list, R, K, r, t * K, Tgrid * K, waves, wave); };
+    ListWalk walk = lists();
+    int64_t v[2][kSmallDepth];
+    int whose = 0, n_round[2];
+    bool go = walk.more();
+    n_round[0] = walk.fetch(v[0], &whose);
+
     const bool valid = lane < K && (uint64_t)e64 < (uint64_t)E;
     const int e = valid ? (int)e64 : 0;
     const int L = E / R, q = e / L, le = e - q * L;
@@ -852,24 +906,39 @@ __global__ __launch_bounds__(256) void dispatch_small_kernel(SmallTable tb, int3
     const uint64_t base = tb.v[DF_RECV_X * R + q];
     const uint64_t info = tb.v[DF_SRC_INFO * R + q];
     const uint64_t sbase = FP8 ? tb.v[DF_RECV_SCALES * R + q] : 0;
-    const int target = valid ? e : -2;
-    int ek[KMAX], cnt[KMAX];
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-        ek[k] = __builtin_amdgcn_readlane(target, k);
-        cnt[k] = 0;
-    }
-    // selections of earlier ranks, then of this rank's earlier tokens
-    for (int rr = 0; rr < r; ++rr)
-        count_list<KMAX>(tb.v[DF_TOPK_IDX * R + rr], (int)tb.v[DF_NUM_TOKENS * R + rr] * K, E, ek, cnt, lane);
-    count_list<KMAX>(own_list, t * K, E, ek, cnt, lane);
+    extern __shared__ int lds_hist[];                             // [min(E, kSmallSpan)]
     int slot = 0;
+    for (int first = 0;;) {                                       // (once, unless there are more experts than kSmallSpan)
+        const int span = E - first < kSmallSpan ? E - first : kSmallSpan;
+        for (int i = threadIdx.x; i < span; i += blockDim.x) lds_hist[i] = 0;
+        __syncthreads();
+        auto take = [&](int i) {                                  // counts round i while the other one is on its way
+            const bool another = walk.more();
+            n_round[1 - i] = walk.fetch(v[1 - i], &whose);
+            count_round(v[i], n_round[i], first, span, lds_hist);
+            return another;
+        };
+        if (go)
+            for (;;) {
+                if (!take(0)) break;
+                if (!take(1)) break;
+            }
+        __syncthreads();
+        if (valid && e >= first && e - first < span) slot = lds_hist[e - first];
+        first += span;
+        if (first >= E) break;
+        // the lists again, for the next span (the last round's successor, never counted, has to have arrived)
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-        const int total = wave_total(cnt[k]);
-        // plus the token's own earlier selections of the same expert (a repeated expert gets a row per occurrence)
-        if (lane == k) slot += total;
-        if (lane > k && ek[k] == target) slot += 1;
+        for (int j = 0; j < kSmallDepth; ++j) asm volatile("" ::"v"(v[0][j]), "v"(v[1][j]));
+        walk = lists();
+        go = walk.more();
+        n_round[0] = walk.fetch(v[0], &whose);
+        __syncthreads();                                          // this span has been read
+    }
+    // plus the token's own earlier selections of the same expert (a repeated expert gets a row per occurrence)
+    for (int k = 0; k + 1 < K; ++k) {
+        const int earlier = __builtin_amdgcn_readlane(valid ? e : -1, k);
+        if (lane > k && earlier == e) slot += 1;
     }
     const int64_t RM = (int64_t)R * max_tokens;
     const bool ok = valid && slot < RM && base != 0;
@@ -879,28 +948,31 @@ __global__ __launch_bounds__(256) void dispatch_small_kernel(SmallTable tb, int3
         row = base + (uint64_t)grow * (uint64_t)H * (FP8 ? 1 : 2);
         if (FP8) srow = sbase + (uint64_t)((int64_t)le * (H >> 7) * RM + slot) * 4;
     }
-    if (s == 0 && lane < K) {
+    if (wave == 0 && lane < K) {
         // where the selection went, for a combine of this dispatch's handle: expert * R*max + row, or -1
         selrow[((int64_t)r * max_tokens + t) * K + lane] = ok ? (int)((int64_t)e * RM + slot) : -1;
-        if (ok) ((int32_t*)info)[grow] = t;
+        if (ok) *(MCEP_GLOBAL int32_t*)(uintptr_t)(info + (uint64_t)grow * 4) = t;
     }
 
-    if (FP8) {
-        float scale_inv;
-        const uint4 out = quantise16<NATIVE>(a, b, &scale_inv);
-        const uint64_t goff = (uint64_t)((int64_t)(elem0 >> 7) * RM) * 4;
-        for (int k = 0; k < K; ++k) {
-            const uint64_t dst = read_lane_u64(row, k);
-            if (dst == 0) continue;
-            if (act_a) store16<false>((void*)(dst + elem0), out);
-            if (act_a && (lane & 7) == 0) *(MCEP_GLOBAL float*)(uintptr_t)(read_lane_u64(srow, k) + goff) = scale_inv;
-        }
-    } else {
-        for (int k = 0; k < K; ++k) {
-            const uint64_t dst = read_lane_u64(row, k);
-            if (dst == 0) continue;
-            if (act_a) store16<false>((void*)(dst + (int64_t)elem0 * 2), a);
-            if (act_b) store16<false>((void*)(dst + (int64_t)elem0 * 2 + kSlabBytes / 2), b);
+    for (int s = wave; s < slabs; s += waves) {                  // (once, unless hidden is above 8192)
+        if (s != wave) load_slab(s);
+        if (FP8) {
+            float scale_inv;
+            const uint4 out = quantise16<NATIVE>(a, b, &scale_inv);
+            const uint64_t goff = (uint64_t)((int64_t)(elem0 >> 7) * RM) * 4;
+            for (int k = 0; k < K; ++k) {
+                const uint64_t dst = read_lane_u64(row, k);
+                if (dst == 0) continue;
+                if (act_a) store16_row<kStoreThrough>(dst, elem0, out, H);
+                if (act_a && (lane & 7) == 0) *(MCEP_GLOBAL float*)(uintptr_t)(read_lane_u64(srow, k) + goff) = scale_inv;
+            }
+        } else {
+            for (int k = 0; k < K; ++k) {
+                const uint64_t dst = read_lane_u64(row, k);
+                if (dst == 0) continue;
+                if (act_a) store16_row<kStoreThrough>(dst, elem0 * 2, a, H * 2);
+                if (act_b) store16_row<kStoreThrough>(dst, elem0 * 2 + kSlabBytes / 2, b, H * 2);
+            }
         }
     }
 }
@@ -1728,31 +1800,32 @@ hipError_t launch_pack(const uint64_t* d_tbl, const RoutingScratch& sc, const Di
     return hipGetLastError();
 }
 
-template <int KMAX>
-static hipError_t launch_dispatch_small_t(const SmallTable& tb, int32_t* d_selrow, const Dims& d, bool use_fp8,
-                                          const Tuning& t, hipStream_t stream) {
+hipError_t launch_dispatch_small(const SmallTable& tb, int32_t* d_selrow, const Dims& d, bool use_fp8, const Tuning& t,
+                                 hipStream_t stream) {
+    if (d.R > kSmallRanks || d.Tgrid <= 0 || d_selrow == nullptr) return hipErrorInvalidValue;
     const int slabs = (d.H + 1023) / 1024;
-    const long long total = (long long)d.E + (long long)d.R * d.Tgrid * slabs;
+    const int expert_blocks = (d.E + kSmallExperts - 1) / kSmallExperts;
+    const long long total = (long long)expert_blocks + (long long)d.R * d.Tgrid;
     if (total > 0x7fffffffll) return hipErrorInvalidValue;
-    constexpr int wpb = 4;
-    const dim3 grid((unsigned)((total + wpb - 1) / wpb)), block(wpb * 64);
-#define MCEP_SMALL(FP8, NATIVE)                                                                              \
-    hipLaunchKernelGGL((dispatch_small_kernel<KMAX, FP8, NATIVE>), grid, block, 0, stream, tb, d_selrow, d.R, \
-                       d.E, d.K, d.max_tokens, d.H, slabs, d.Tgrid, (int)total)
+    const dim3 grid((unsigned)total), block(small_block_waves(d.H) * 64);
+    const size_t lds = (size_t)(d.E < kSmallSpan ? d.E : kSmallSpan) * sizeof(int);
+    // (the fewer argument bytes the cheaper the launch, as for the count kernel)
+    constexpr int kFew = (int)DF_COUNT * 8, kMany = (int)DF_COUNT * kSmallRanks;
+    const int words = (int)DF_COUNT * d.R;
+#define MCEP_SMALL_TABLE(FP8, NATIVE, TW)                                                                              \
+    hipLaunchKernelGGL((dispatch_small_kernel<FP8, NATIVE, TW>), grid, block, lds, stream, arg_table<TW>(tb.v, words), \
+                       d_selrow, d.R, d.E, d.K, d.max_tokens, d.H, slabs, d.Tgrid, expert_blocks)
+#define MCEP_SMALL(FP8, NATIVE)                                 \
+    do {                                                        \
+        if (words <= kFew) MCEP_SMALL_TABLE(FP8, NATIVE, kFew); \
+        else MCEP_SMALL_TABLE(FP8, NATIVE, kMany);              \
+    } while (0)
     if (!use_fp8) MCEP_SMALL(false, false);
     else if (t.fp8_arith == 1) MCEP_SMALL(true, true);
     else MCEP_SMALL(true, false);
 #undef MCEP_SMALL
+#undef MCEP_SMALL_TABLE
     return hipGetLastError();
-}
-
-hipError_t launch_dispatch_small(const SmallTable& tb, int32_t* d_selrow, const Dims& d, bool use_fp8, const Tuning& t,
-                                 hipStream_t stream) {
-    if (d.R > kSmallRanks || d.Tgrid <= 0 || d_selrow == nullptr) return hipErrorInvalidValue;
-    if (d.K <= 2) return launch_dispatch_small_t<2>(tb, d_selrow, d, use_fp8, t, stream);
-    if (d.K <= 4) return launch_dispatch_small_t<4>(tb, d_selrow, d, use_fp8, t, stream);
-    if (d.K <= 8) return launch_dispatch_small_t<8>(tb, d_selrow, d, use_fp8, t, stream);
-    return launch_dispatch_small_t<16>(tb, d_selrow, d, use_fp8, t, stream);
 }
 
 hipError_t launch_resolve(const uint64_t* d_tbl, CombineRoute* d_routes, uint32_t stamp, bool packed, const Dims& d,

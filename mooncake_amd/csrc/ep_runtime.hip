@@ -546,14 +546,18 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         selections += (long long)num_tokens[r] * num_topk;
         list_rounds += ((long long)num_tokens[r] * num_topk + kSmallListRound - 1) / kSmallListRound;
     }
-    // A world that names few selections is dispatched in one launch, every wave rebuilding the routing it
+    // A world that names few selections is dispatched in one launch, every block rebuilding the routing it
     // needs from the index lists (dispatch_small_kernel); the rank table then travels in kernel arguments.
-    // What that costs grows with the rounds of index-list entries a late wave reads one after another (every
-    // rank's list is at least one round); measured against the launches it saves - two for an fp8 payload,
-    // one for bf16 - it pays up to six rounds and four.
+    // What that costs grows with the rounds of index-list entries a wave of a late token reads one after another
+    // (every rank's list is at least one round; a block's payload waves share them out), which is weighed against
+    // the launches it saves - two for an fp8 payload, one for bf16: up to six rounds and four.  At six rounds a wave
+    // the one launch takes 8.5 us (12 ranks, two payload waves, fp8) where the three kernels and the gaps between
+    // them take 15.
     const int rounds_limit = w->tuning.fused_small_rounds >= 0 ? w->tuning.fused_small_rounds : (use_fp8 ? 6 : 4);
-    const bool fused = w->tuning.fused_small != 0 && phases == MC_EP_PHASE_ALL && R <= kSmallRanks && tgrid > 0 &&
-                       selections <= (long long)w->tuning.fused_small_max && list_rounds <= (long long)rounds_limit;
+    const long long wave_rounds = (list_rounds + small_waves(hidden) - 1) / small_waves(hidden);
+    const bool fused = w->tuning.fused_small != 0 && phases == MC_EP_PHASE_ALL && tgrid > 0 && R <= kSmallRanks &&
+                       R <= kSmallWaveRanks * small_waves(hidden) &&
+                       selections <= (long long)w->tuning.fused_small_max && wave_rounds <= (long long)rounds_limit;
     DeviceGuard guard(w->device);
     w->launches = 0;
     struct Tally {                                // the option "last_dispatch_launches", on every way out
@@ -614,7 +618,8 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         if (int rc = capture_of(stream, &cap)) return rc;
         RecordingScope recording(cap.active);
         if (int rc = order_begin(w, stream, cap)) return rc;
-        if (int rc = ensure_scratch(w, &w->d_selrow, &w->selrow_cap, (size_t)R * max_tokens * num_topk)) return rc;
+        // (two entries at least: dispatch_small_kernel may read 8 bytes there)
+        if (int rc = ensure_scratch(w, &w->d_selrow, &w->selrow_cap, (size_t)R * max_tokens * num_topk + 1)) return rc;
         if (!fused) {
             // (the one-launch dispatch keeps no routing state but selrow, and needs no table in memory)
             if (int rc = ensure_scratch(w, &w->d_ucount, &w->ucount_cap, UE)) return rc;

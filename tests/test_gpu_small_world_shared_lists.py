@@ -1,0 +1,43 @@
+"""The one-launch dispatch where the waves of a block share the index lists out: several slabs per token (so several
+waves and more than 8 ranks), lists around the 512-entry rounds the waves take in turn, more slabs than a block has
+waves, more experts than its histogram holds at a time.  Whole numbers and bytes: everything equals the oracle's."""
+import pytest
+
+from mooncake_amd.workloads import EPConfig, generate
+from tests import gpu_util
+from tests.gpu_util import announce, compare_dispatch, run_dispatch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    EPConfig("ranks_12_two_slabs", 12, 68, 1152, 108, 5, True),      # 12 lists of 340 entries on four waves
+    EPConfig("ranks_16_two_slabs", 16, 8, 2048, 32, 3, False),       # the most ranks two slabs take
+    EPConfig("ranks_32_eight_slabs", 32, 16, 7424, 64, 8, True),     # the most ranks there are
+    EPConfig("rounds_512_513", 3, 171, 1152, 24, 3, False),          # 513 entries: a round and one entry
+    EPConfig("rounds_6_of_512", 1, 384, 4096, 64, 8, True),          # one list, six whole rounds
+    EPConfig("slabs_9", 2, 12, 9216, 16, 4, True),                   # a slab more than a block has waves
+    EPConfig("slabs_18_bf16", 2, 5, 17536, 16, 4, False),
+    EPConfig("experts_4096", 4, 16, 1152, 4096, 8, True),            # a whole histogram, and one with a remainder
+    EPConfig("experts_8200", 4, 16, 1152, 8200, 8, False),
+    EPConfig("hot", 8, 64, 4096, 64, 6, True, routing="zipf", masked_fraction=0.2),
+]
+
+
+@pytest.mark.parametrize("cfg", CASES, ids=[c.name for c in CASES])
+@pytest.mark.parametrize("is_ragged", [False, True], ids=["full", "ragged"])
+def test_shared_lists_match_oracle(gpu_device, oracle, cfg, is_ragged):
+    T = cfg.tokens_per_rank
+    nt = [T - r * 7 % (T + 1) for r in range(cfg.num_ranks)] if is_ragged else None
+    announce(f"one-launch dispatch, shared lists {cfg} ragged={nt}")
+    data = generate(cfg, seed=61)
+    if is_ragged:
+        data["topk_idx"][0, ::5, -1] = data["topk_idx"][0, ::5, 0]    # repeated experts
+        data["topk_idx"][-1, 0, 0] = 2 ** 32 + 1                      # and a number no expert has
+    gpu_util.DEFAULT_OPTIONS["fused_small_rounds"] = 1 << 20
+    try:
+        h = run_dispatch(cfg, data, num_tokens=nt, poison=True)
+    finally:
+        gpu_util.DEFAULT_OPTIONS.pop("fused_small_rounds", None)
+    assert h.world.get_option("last_dispatch_launches") == 1
+    ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
+    compare_dispatch(h, ref, check_poison=True)
