@@ -4,17 +4,29 @@
 // EventHandle, Buffer with the bound names and argument order of the reference, and
 // _benchmark_legacy_buffer with its three structs
 // (mooncake-ep/benchmarks/legacy_buffer_perf.cpp:151-199).  Everything goes through
-// the C ABI of include/mooncake_ep_hip.h; no torch type appears here either - device
-// addresses and streams are integers, as in the reference's bindings.
+// the C ABI of include/mooncake_ep_hip.h; in what the reference binds no torch type
+// appears here either - device addresses and streams are integers, as there.
+//
+// Buffer.dispatch_tensors and combine_tensors are the exception: the reference wrapper's
+// checks, its outputs and the call itself in one native step, for the Python `Buffer`
+// above (a rank's dispatch took 4.1 us of host time through Python and a combine 5.2,
+// nearly all of it tensor attributes, torch.empty and the pool's look-up).
 //
 // What the reference does not have: World (the expert-parallel world as logical ranks
 // of one GPU; Buffer takes the one it belongs to as an optional fifth argument and
 // otherwise joins a process-wide world of its num_ranks) and the whole-world calls.
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ops/empty.h>
+#include <ATen/ops/ones.h>
+#include <c10/core/Storage.h>
+#include <c10/core/TensorImpl.h>
 #include <pybind11/functional.h>
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
 #include <atomic>
+#include <climits>
 #include <cstdint>
 #include <deque>
 #include <functional>
@@ -124,8 +136,102 @@ int without_gil(F&& f) {
     return f();
 }
 
+// the reference wrapper's checks are Python assertions (mooncake_ep_buffer.py:378-393, :554-567, :616-640)
+#define MC_CHECK(cond)                                 \
+    do {                                               \
+        if (!(cond)) {                                 \
+            PyErr_SetString(PyExc_AssertionError, #cond); \
+            throw py::error_already_set();             \
+        }                                              \
+    } while (0)
+
+const at::Tensor& tensor_of(const py::handle& h) {
+    if (!THPVariable_Check(h.ptr())) throw py::type_error("a torch.Tensor expected");
+    return THPVariable_Unpack(h.ptr());
+}
+
+py::object wrap_tensor(at::Tensor t) {
+    PyObject* o = THPVariable_Wrap(std::move(t));
+    if (o == nullptr) throw py::error_already_set();
+    return py::reinterpret_steal<py::object>(o);
+}
+
+// torch.empty, with its own exception where memory runs out
+at::Tensor empty(c10::IntArrayRef sizes, at::ScalarType type, const at::Device& device) {
+    try {
+        return at::empty(sizes, at::TensorOptions().dtype(type).device(device));
+    } catch (const c10::OutOfMemoryError& e) {
+        py::object type = py::module_::import("torch").attr("OutOfMemoryError");
+        PyErr_SetString(type.ptr(), e.what_without_backtrace());
+        throw py::error_already_set();
+    }
+}
+
+// sizes travel as int from here on; a larger one is refused as pybind11 refuses it
+int as_int(int64_t v) {
+    if (v < INT_MIN || v > INT_MAX) throw py::type_error("size out of range");
+    return (int)v;
+}
+
+uint64_t address(const at::Tensor& t) { return (uint64_t)(uintptr_t)t.data_ptr(); }
+
+// The outputs of earlier dispatches, offered again under the rule of the Python `_OutputPool`: a set is free when
+// nothing but the pool refers to any of its storages (tensors, views and dtype reinterpretations of one all do).
+// Kept are the storages, not the tensors: every call gets tensors of its own.  Sets are kept per shape, type, device
+// and current stream, at most kSets of them per key; a caller that keeps every output alive pools nothing.
+class OutputPool {
+   public:
+    struct Spec {
+        std::vector<int64_t> sizes;
+        at::ScalarType type;
+        std::vector<int64_t> strides = {};   // empty: contiguous
+    };
+    using Key = std::tuple<int64_t, int64_t, int64_t, bool, int, uint64_t>;
+
+    std::vector<at::Tensor> take(const Key& key, const std::vector<Spec>& specs, const at::Device& device) {
+        std::vector<Set>& sets = sets_[key];
+        const auto idle = [&](const Set& set) {
+            for (size_t i = 0; i < specs.size(); ++i)
+                if (set[i].use_count() != 1 || set[i].nbytes() != bytes(specs[i])) return false;
+            return true;
+        };
+        Set fresh;
+        const Set* set = nullptr;
+        for (size_t i = 0; i < sets.size() && set == nullptr; ++i)
+            if (idle(sets[i])) set = &sets[i];
+        if (set == nullptr) {
+            // outputs are not cleared: rows at and beyond packed_recv_count stay unwritten
+            for (const Spec& s : specs) fresh.push_back(empty(s.sizes, s.type, device).storage());
+            if (sets.size() < kSets) sets.push_back(fresh);
+            set = &fresh;
+        }
+        std::vector<at::Tensor> out;
+        out.reserve(specs.size());
+        for (size_t i = 0; i < specs.size(); ++i) {
+            const auto dispatch_key = c10::computeDispatchKey(specs[i].type, c10::nullopt, device);
+            at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(
+                c10::Storage((*set)[i]), c10::DispatchKeySet(dispatch_key), c10::scalarTypeToTypeMeta(specs[i].type));
+            if (specs[i].strides.empty()) t.unsafeGetTensorImpl()->set_sizes_contiguous(specs[i].sizes);
+            else t.unsafeGetTensorImpl()->set_sizes_and_strides(specs[i].sizes, specs[i].strides);
+            out.push_back(std::move(t));
+        }
+        return out;
+    }
+
+   private:
+    static constexpr size_t kSets = 4;
+    using Set = std::vector<c10::Storage>;
+    std::map<Key, std::vector<Set>> sets_;
+    static size_t bytes(const Spec& s) {
+        size_t n = c10::elementSize(s.type);
+        for (int64_t d : s.sizes) n *= (size_t)d;
+        return n;
+    }
+};
+
 // MooncakeEpBuffer, mooncake_ep_buffer.h:66-194
 struct Buffer {
+    OutputPool outputs;
     mc_ep_buffer_t* h = nullptr;
     WorldPtr world;
     int rank = 0, num_ranks = 0;
@@ -194,6 +300,114 @@ struct Buffer {
         retain(1, rc, keep_alive);
         check(rc);
         return wrap(ev, hook, world);
+    }
+
+    // the rank's view of live ranks: the caller's, or (none given, or one of another size) all of them
+    at::Tensor active_or_default(const py::object& active_ranks, const at::Tensor& like) const {
+        if (!active_ranks.is_none()) {
+            const at::Tensor& active = tensor_of(active_ranks);
+            MC_CHECK(active.dim() == 1 && active.is_contiguous());
+            MC_CHECK(active.scalar_type() == at::kInt);
+            if (active.numel() == num_ranks) return active;
+        }
+        return at::ones({num_ranks}, at::TensorOptions().dtype(at::kInt).device(like.device()));
+    }
+
+    // -> (event, hook, (x, topk_idx, active_ranks, packed_recv_x, scales or None, count, src_info, layout_range))
+    py::tuple dispatch_tensors(py::object x_, py::object topk_idx_, py::object active_ranks_, int max_tokens,
+                               int num_experts, int timeout_us, bool use_fp8, bool async, bool return_recv_hook,
+                               uint64_t stream_ptr) {
+        const at::Tensor &x = tensor_of(x_), &topk_idx = tensor_of(topk_idx_);
+        MC_CHECK(x.dim() == 2 && x.is_contiguous());
+        MC_CHECK(x.scalar_type() == at::kBFloat16);
+        MC_CHECK(topk_idx.dim() == 2 && topk_idx.is_contiguous());
+        MC_CHECK(topk_idx.scalar_type() == at::kLong);
+        const int64_t num_tokens = x.size(0), hidden = x.size(1);
+        MC_CHECK(num_tokens == topk_idx.size(0));
+        MC_CHECK(num_tokens <= max_tokens);
+        MC_CHECK(hidden % 16 == 0 && hidden % 128 == 0);
+        MC_CHECK(num_experts % num_ranks == 0);
+        const at::Tensor active = active_or_default(active_ranks_, x);
+        const int64_t local = num_experts / num_ranks, rm = (int64_t)num_ranks * max_tokens;
+        if (use_fp8) MC_CHECK(rm % 4 == 0);
+
+        std::vector<OutputPool::Spec> specs{{{local, rm, hidden}, use_fp8 ? at::kFloat8_e4m3fn : at::kBFloat16},
+                                            {{local}, at::kInt},
+                                            {{local, rm}, at::kInt},
+                                            {{local, (int64_t)num_ranks}, at::kLong}};
+        // column-major per expert: [L, H/128, R*max] storage viewed as [L, R*max, H/128]
+        if (use_fp8) specs.push_back({{local, rm, hidden / 128}, at::kFloat, {hidden / 128 * rm, 1, rm}});
+        std::vector<at::Tensor> outs =
+            outputs.take({local, rm, hidden, use_fp8, x.device().index(), stream_ptr}, specs, x.device());
+        const uint64_t recv_x = address(outs[0]), count = address(outs[1]), info = address(outs[2]),
+                       range = address(outs[3]), scales = use_fp8 ? address(outs[4]) : 0;
+        py::object active_obj = active_ranks_;
+        if (active_ranks_.is_none() || !active.is_same(tensor_of(active_ranks_))) active_obj = wrap_tensor(active);
+        const int num_topk = as_int(topk_idx.size(1));
+        const uint64_t x_ptr = address(x), idx_ptr = address(topk_idx), active_ptr = address(active);
+        py::tuple kept = py::make_tuple(
+            std::move(x_), std::move(topk_idx_), std::move(active_obj), wrap_tensor(std::move(outs[0])),
+            use_fp8 ? wrap_tensor(std::move(outs[4])) : py::object(py::none()), wrap_tensor(std::move(outs[1])),
+            wrap_tensor(std::move(outs[2])), wrap_tensor(std::move(outs[3])));
+        CallResult r = dispatch(x_ptr, idx_ptr, active_ptr, as_int(num_tokens), as_int(hidden), num_topk, max_tokens,
+                                num_experts, timeout_us, use_fp8, recv_x, scales, count, info, range, async,
+                                return_recv_hook, stream_ptr, kept);
+        return py::make_tuple(std::move(std::get<0>(r)), std::move(std::get<1>(r)), std::move(kept));
+    }
+
+    // -> (event, hook, (x, topk_idx, topk_weights, active_ranks, src_info, layout_range, combined_x))
+    py::tuple combine_tensors(py::object x_, py::object topk_idx_, py::object topk_weights_, py::object active_ranks_,
+                              py::object src_info_, py::object layout_range_, int max_tokens, int hidden,
+                              int num_experts, int timeout_us, py::object out_, bool async, bool return_recv_hook,
+                              uint64_t stream_ptr) {
+        const at::Tensor &x = tensor_of(x_), &topk_idx = tensor_of(topk_idx_), &topk_weights = tensor_of(topk_weights_);
+        const at::Tensor &src_info = tensor_of(src_info_), &layout_range = tensor_of(layout_range_);
+        MC_CHECK(x.dim() == 3 && x.is_contiguous());
+        MC_CHECK(x.scalar_type() == at::kBFloat16);
+        MC_CHECK(topk_idx.dim() == 2 && topk_idx.is_contiguous());
+        MC_CHECK(topk_idx.scalar_type() == at::kLong);
+        MC_CHECK(topk_weights.dim() == 2 && topk_weights.is_contiguous());
+        MC_CHECK(topk_weights.scalar_type() == at::kFloat);
+        const at::Tensor active = active_or_default(active_ranks_, x);
+        const int64_t local = num_experts / num_ranks;
+        MC_CHECK(x.size(0) == local);
+        MC_CHECK(x.size(1) == (int64_t)num_ranks * max_tokens);
+        MC_CHECK(x.size(2) == hidden);
+        MC_CHECK(hidden % 16 == 0 && hidden % 128 == 0);
+        MC_CHECK(topk_idx.sizes() == topk_weights.sizes());
+        const int64_t num_tokens = topk_weights.size(0);
+        MC_CHECK(num_tokens <= max_tokens);
+        MC_CHECK(src_info.dim() == 2 && src_info.is_contiguous());
+        MC_CHECK(src_info.scalar_type() == at::kInt);
+        MC_CHECK(src_info.size(0) == x.size(0));
+        MC_CHECK(layout_range.dim() == 2 && layout_range.is_contiguous());
+        MC_CHECK(layout_range.scalar_type() == at::kLong);
+        MC_CHECK(layout_range.size(0) == local);
+        MC_CHECK(layout_range.size(1) == num_ranks);
+        at::Tensor combined;
+        if (!out_.is_none()) {
+            combined = tensor_of(out_);
+            MC_CHECK(combined.dim() == 2 && combined.is_contiguous());
+            MC_CHECK(combined.size(0) == num_tokens);
+            MC_CHECK(combined.size(1) == hidden);
+            MC_CHECK(combined.scalar_type() == at::kBFloat16);
+        } else {
+            combined = empty({num_tokens, hidden}, at::kBFloat16, x.device());
+            out_ = wrap_tensor(combined);
+        }
+        py::object active_obj = active_ranks_;
+        if (active_ranks_.is_none() || !active.is_same(tensor_of(active_ranks_))) active_obj = wrap_tensor(active);
+        const uint64_t x_ptr = address(x), idx_ptr = address(topk_idx), weights_ptr = address(topk_weights),
+                       info_ptr = address(src_info), range_ptr = address(layout_range), active_ptr = address(active),
+                       out_ptr = address(combined);
+        const int num_topk = as_int(topk_weights.size(1));
+        py::tuple kept = py::make_tuple(std::move(x_), std::move(topk_idx_), std::move(topk_weights_),
+                                        std::move(active_obj), std::move(src_info_), std::move(layout_range_),
+                                        std::move(out_));
+        CallResult r = combine(x_ptr, idx_ptr, weights_ptr, info_ptr, range_ptr, active_ptr, as_int(local), as_int(num_tokens),
+                               hidden, num_topk, max_tokens, num_experts, timeout_us, false, out_ptr, async,
+                               return_recv_hook, stream_ptr, kept);
+        return py::make_tuple(std::move(std::get<0>(r)), std::move(std::get<1>(r)), std::move(kept));
     }
 
     std::pair<int, int> pending_calls() const {
@@ -447,6 +661,9 @@ PYBIND11_MODULE(_ep, m) {
         .def("sync_nvlink_ipc_handles", [](Buffer&, py::object, py::object) {})
         .def("pending_calls", &Buffer::pending_calls)
         .def("retained", &Buffer::retained, "(dispatch, combine) keep_alive objects still held")
+        // what the Python `Buffer`'s dispatch and combine are made of (positional arguments)
+        .def("dispatch_tensors", &Buffer::dispatch_tensors)
+        .def("combine_tensors", &Buffer::combine_tensors)
         // the reference's argument lists (ep_py.cpp:43-44), positional; keep_alive is this module's addition
         .def("dispatch", &Buffer::dispatch, py::arg("x_ptr"), py::arg("topk_idx_ptr"), py::arg("active_ranks_ptr"),
              py::arg("num_tokens"), py::arg("hidden"), py::arg("num_topk"),

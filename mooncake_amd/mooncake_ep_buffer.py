@@ -41,6 +41,7 @@ def _native_current_stream_ptr() -> int:
 
 _storage_use_count = getattr(torch._C, "_storage_Use_Count", None)
 _getrefcount = sys.getrefcount
+_Tensor = torch.Tensor
 _BF16, _I64, _I32, _F32, _FP8 = torch.bfloat16, torch.int64, torch.int32, torch.float32, torch.float8_e4m3fn
 
 
@@ -194,6 +195,10 @@ class Buffer:
         # posted: each call hands its tensors to the runtime (`keep_alive`), which holds them until it
         # has enqueued the call's round, however far ahead of its peers this rank runs.
         self._outputs = _OutputPool()
+        # The compiled module takes whole calls on plain torch tensors; what it does not take (its ctypes stand-in,
+        # tensor subclasses) goes through the Python statements of the same checks below.
+        self._dispatch_tensors = getattr(self.runtime, "dispatch_tensors", None) if _FAST_STREAM else None
+        self._combine_tensors = getattr(self.runtime, "combine_tensors", None) if _FAST_STREAM else None
         self.connect()
 
     @staticmethod
@@ -232,6 +237,18 @@ class Buffer:
                  use_fp8: Optional[bool] = None, async_finish: bool = False, return_recv_hook: bool = False,
                  ) -> Tuple[Union[Tuple[torch.Tensor, torch.Tensor], torch.Tensor], torch.Tensor, Tuple,
                             EventOverlap, Callable]:
+        native = self._dispatch_tensors
+        if native is not None and type(x) is _Tensor and type(topk_idx) is _Tensor and \
+                (active_ranks is None or type(active_ranks) is _Tensor):
+            # the checks, the outputs and the call below, in the compiled module
+            event, hook, kept = native(x, topk_idx, active_ranks, num_max_dispatch_tokens_per_rank, num_experts,
+                                       timeout_us, use_fp8 is None or bool(use_fp8), async_finish, return_recv_hook,
+                                       _raw_stream(_raw_device()))
+            _, _, _, recv_x, scales, count, src_info, layout_range = kept
+            return (recv_x if scales is None else (recv_x, scales), count,
+                    (src_info, layout_range, num_max_dispatch_tokens_per_rank, x.shape[1], num_experts),
+                    EventOverlap(event, kept if async_finish else None),
+                    None if hook is None else self._hook_keeping(hook, kept))
         # the reference's checks (:378-393), on each tensor's shape tuple: this wrapper is all host time
         xs, ts, group_size = x.shape, topk_idx.shape, self.group_size
         assert len(xs) == 2 and x.is_contiguous()
@@ -299,6 +316,16 @@ class Buffer:
                 ) -> Tuple[torch.Tensor, EventOverlap, Callable]:
         if zero_copy:
             raise NotImplementedError(_ZERO_COPY_COMBINE_UNSUPPORTED)
+        native = self._combine_tensors
+        if native is not None and type(x) is _Tensor and type(topk_idx) is _Tensor and \
+                type(topk_weights) is _Tensor and (active_ranks is None or type(active_ranks) is _Tensor) and \
+                type(handle[0]) is _Tensor and type(handle[1]) is _Tensor and (out is None or type(out) is _Tensor):
+            src_info, layout_range, num_max_dispatch_tokens_per_rank, hidden, num_experts = handle
+            event, hook, kept = native(x, topk_idx, topk_weights, active_ranks, src_info, layout_range,
+                                       num_max_dispatch_tokens_per_rank, hidden, num_experts, timeout_us, out,
+                                       async_finish, return_recv_hook, _raw_stream(_raw_device()))
+            return (kept[6], EventOverlap(event, kept if async_finish else None),
+                    None if hook is None else self._hook_keeping(hook, kept))
         # the reference's checks (:554-567, :616-640), on each tensor's shape tuple
         xs, ts, ws, group_size = x.shape, topk_idx.shape, topk_weights.shape, self.group_size
         assert len(xs) == 3 and x.is_contiguous()
