@@ -94,7 +94,9 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
 /* Options ("pack_waves", "pack_nt", "uniform", "routing_sum", "combine_direct",
  * "combine_chunks", "combine_waves", "combine_nt", "combine_occupancy",
  * "packed_map": tuning knobs
- * for measurement sweeps; "fused_small": 1 (default) dispatches a world of at
+ * for measurement sweeps; "combine_search_tokens" (default 256): a combine of a
+ * handle that is not the last dispatch's is one launch while no rank combines
+ * more tokens than this, two beyond (0: always two); "fused_small": 1 (default) dispatches a world of at
  * most "fused_small_max" (default 4096) selections and 8 ranks per 1024
  * hidden elements (32 ranks in all) in one kernel launch - provided the ranks'
  * index lists make at most "fused_small_rounds" rounds of 512 entries, each

@@ -136,7 +136,9 @@ struct CombineSource {
     RankPtr x;              // the rows combine reads (expert outputs, or the packed payload)
     RankPtr scales;         // packed combine of an fp8 payload
     RankPtr active;
+    RankPtr src_info, layout_range;   // the handle, when the reduce kernels look rows up in it
     bool packed_fp8 = false;   // `scales` is read
+    bool search = false;       // rows are looked up in the handle (not: in the last dispatch's state, or in routes)
     int tokens = -1;
 };
 
@@ -162,6 +164,8 @@ struct Tuning {
     int fp8_arith = 0;         // fp8 scale arithmetic: 0 = the reference's PyTorch statement as CPU PyTorch runs it,
                                // 1 = the reference kernel's own (see pack_fp8_kernel)
     int combine_direct = 1;    // reuse the last dispatch's routing state when combine gets that dispatch's handle
+    int combine_search_tokens = 256;   // any other handle is searched by the reduce kernel itself while no rank combines
+                               // more tokens than this; beyond, a resolve launch turns it into routes
     int combine_chunks = 0;    // 16-byte chunks per lane in the combine kernel (1 or 2); 0: by top-k
     int combine_waves = 4;     // waves per block in the combine kernel
     int combine_nt = 3;        // bit 0: streaming loads, bit 1: streaming stores

@@ -33,7 +33,8 @@
 //   resolve_kernel  combine's handle (src_info, layout_range) -> source row and
 //                   weight of each (token, k) (data flow of
 //                   mooncake_ep_kernel.cu:611-637); only for a handle that is
-//                   not the last dispatch's.
+//                   not the last dispatch's, of ranks with many tokens (the
+//                   reduce kernels look rows of smaller ones up by themselves).
 //   reduce_kernel   per token: fp32 fused multiply-add over its top-k expert
 //                   rows in k order, round to nearest even bf16
 //                   (mooncake_ep_kernel.cu:711-753); a selection counts while
@@ -1081,15 +1082,79 @@ __device__ __forceinline__ DirectRow direct_row(const uint64_t* __restrict__ tbl
     return d;
 }
 
+// Where the reduce kernels find a token's rows.
+//   kFromRoutes    in the routes that the resolve kernel left;
+//   kFromDispatch  in the last dispatch's routing state (direct_row);
+//   kFromHandle    in the handle itself (search_row): no resolve launch (6.8 us for 32 x 64 tokens), but two more
+//                  dependent loads in front of every wave's payload.
+enum : int { kFromRoutes = 0, kFromDispatch = 1, kFromHandle = 2 };
+
+// Lanes that work on one of a token's selections: one, or under kFromHandle an equal share of the wave.
+template <int FROM, int KMAX>
+constexpr int lanes_per_selection() {
+    return FROM != kFromHandle ? 1 : 64 / (KMAX <= 1 ? 1 : (KMAX <= 2 ? 2 : (KMAX <= 4 ? 4 : (KMAX <= 8 ? 8 : 16))));
+}
+
+// The row of a selection from the handle as combine is given it: LPS lanes scan the rows that the selection's expert
+// got from the token's rank (layout_range) for the token (src_info), four loads per lane in flight.  With several such
+// rows - the token names the expert more than once - the last one counts, as in the resolve kernel and the oracle.
+// A malformed range, a rank without tensors and an expert outside [0, E) have no row.
+template <int LPS>
+__device__ __forceinline__ DirectRow search_row(const uint64_t* __restrict__ tbl, const CombineSource& cs, int R, int E,
+                                                int K, int max_tokens, int r, int t, int lane) {
+    static_assert(LPS >= 4, "the maximum over a selection's lanes starts with quads");
+    const int slot = lane / LPS, j = lane - slot * LPS;
+    const int64_t RM = (int64_t)R * max_tokens;
+    const int L = E / R;
+    const uint64_t active = rank_ptr(tbl, cs.active, CF_ACTIVE, R, r);
+    const uint64_t idx_row = rank_ptr(tbl, cs.topk_idx, CF_TOPK_IDX, R, r) + (uint64_t)((int64_t)t * K) * 8;
+    const int64_t now = *(const MCEP_GLOBAL int64_t*)(uintptr_t)(idx_row + (uint64_t)(slot < K ? slot : 0) * 8);
+    const bool valid = slot < K && now >= 0 && now < (int64_t)E;
+    DirectRow d;
+    d.e = valid ? (int)now : 0;
+    d.q = d.e / L;
+    d.le = d.e - d.q * L;
+    d.base = rank_ptr(tbl, cs.x, CF_X, R, d.q);
+    const uint64_t ranges = rank_ptr(tbl, cs.layout_range, CF_LAYOUT_RANGE, R, d.q);
+    const uint64_t infos = rank_ptr(tbl, cs.src_info, CF_SRC_INFO, R, d.q);
+    int begin = 0, count = 0;
+    if (valid && d.base != 0 && ranges != 0 && infos != 0) {
+        const int64_t lr = *(const MCEP_GLOBAL int64_t*)(uintptr_t)(ranges + (uint64_t)(d.le * R + r) * 8);
+        begin = (int)(lr >> 32);
+        count = (int)(lr & 0xffffffffll);
+        if (begin < 0 || count <= 0 || (int64_t)begin + count > RM) begin = count = 0;   // empty or malformed
+    }
+    d.live = load_i32(active + (uint64_t)d.q * 4);
+    const uint64_t rows = infos + (uint64_t)((int64_t)d.le * RM + begin) * 4;
+    int found = -1;
+    for (int i = j; i < count; i += 4 * LPS) {
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = load_i32(rows + (uint64_t)(i + u * LPS < count ? i + u * LPS : i) * 4);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * LPS < count && v[u] == t) found = i + u * LPS;
+    }
+    auto larger = [](int a, int b) { return a > b ? a : b; };
+    found = larger(found, __builtin_amdgcn_mov_dpp(found, 0xB1, 0xF, 0xF, true));                  // quad_perm [1,0,3,2]
+    found = larger(found, __builtin_amdgcn_mov_dpp(found, 0x4E, 0xF, 0xF, true));                  // quad_perm [2,3,0,1]
+    if (LPS >= 8) found = larger(found, __builtin_amdgcn_mov_dpp(found, 0x141, 0xF, 0xF, true));   // row_half_mirror
+    if (LPS >= 16) found = larger(found, __builtin_amdgcn_mov_dpp(found, 0x140, 0xF, 0xF, true));  // row_mirror
+    if (LPS >= 32) found = larger(found, __shfl_xor(found, 16));
+    if (LPS >= 64) found = larger(found, __shfl_xor(found, 32));
+    d.has = found >= 0;
+    d.slot = begin + (d.has ? found : 0);
+    d.grow = (int64_t)d.le * RM + d.slot;
+    return d;
+}
+
 // One wave per (token, slab of CH * 512 elements).  Lanes 0..K-1 find the K
 // source rows (a masked, inactive or unknown selection reads a zero row with
 // weight 0, which leaves the fp32 accumulator unchanged), then every lane
 // issues all KMAX * CH 16-byte loads before the first multiply-add.
-//   DIRECT   the handle is the one the last dispatch produced: rows come from
-//            that dispatch's routing state, no resolve kernel has run;
-//   !DIRECT  rows come from the routes the resolve kernel left.
+//   FROM     where the rows are looked up
 //   TW       words of the rank table in the arguments; 0: in memory, or not needed (every tensor evenly spaced).
-template <int KMAX, int CH, bool NTL, bool NTS, bool DIRECT, int TW>
+template <int KMAX, int CH, bool NTL, bool NTS, int FROM, int TW>
 __global__ __launch_bounds__(512) void reduce_kernel(const uint64_t* __restrict__ tbl_mem,
                                                       const CombineRoute* __restrict__ routes, uint32_t stamp,
                                                       RoutingScratch sc, CombineSource cs,
@@ -1108,12 +1173,15 @@ __global__ __launch_bounds__(512) void reduce_kernel(const uint64_t* __restrict_
     uint64_t src = (uint64_t)zero_row;
     float w = 0.0f;
     int live = 1;
-    if (DIRECT) {
+    constexpr int kLanes = lanes_per_selection<FROM, KMAX>();      // selection k's row ends up in lane k * kLanes
+    if (FROM != kFromRoutes) {
         // the caller's top-k rows exist only for t < T
         if (t >= T) return;
         const uint64_t w_row = rank_ptr(tbl, cs.topk_weights, CF_TOPK_W, R, r) + (uint64_t)((int64_t)t * K) * 4;
-        const float wl = load_f32(w_row + (uint64_t)(lane < K ? lane : 0) * 4);
-        const DirectRow d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, lane);
+        const float wl = load_f32(w_row + (uint64_t)(lane / kLanes < K ? lane / kLanes : 0) * 4);
+        DirectRow d;
+        if constexpr (FROM == kFromHandle) d = search_row<kLanes>(tbl, cs, R, E, K, max_tokens, r, t, lane);
+        else d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, lane);
         if (d.has && d.base != 0) {
             src = d.base + (uint64_t)d.grow * (uint64_t)H * 2;
             w = wl;
@@ -1144,18 +1212,18 @@ __global__ __launch_bounds__(512) void reduce_kernel(const uint64_t* __restrict_
     float wk[KMAX];
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
-        const uint64_t p = read_lane_u64(src, k);
+        const uint64_t p = read_lane_u64(src, k * kLanes);
 #pragma unroll
         for (int c = 0; c < CH; ++c) v[k][c] = load16<NTL>((const void*)(p + off[c]));
     }
     // An expert on a rank the token's owner sees as inactive is skipped (mooncake_ep_kernel.cu:729-732):
     // its row was fetched before that was known, so the row is dropped here (it may hold anything) and
     // the weight is zero, as for a selection that went nowhere.
-    if (DIRECT && live == 0) w = 0.0f;
+    if (FROM != kFromRoutes && live == 0) w = 0.0f;
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
-        wk[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k));
-        if (DIRECT && __builtin_amdgcn_readlane(live, k) == 0) {
+        wk[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k * kLanes));
+        if (FROM != kFromRoutes && __builtin_amdgcn_readlane(live, k * kLanes) == 0) {
 #pragma unroll
             for (int c = 0; c < CH; ++c) v[k][c] = make_uint4(0, 0, 0, 0);
         }
@@ -1230,7 +1298,7 @@ __device__ __forceinline__ uint32_t scale_round_twice(float a, float b, float s,
 // variant ran 5 % slower.  (Sixteen rows in flight do not fit that budget.)
 //   CH  bf16 payloads only: 16-byte chunks per lane and row, 512 elements apart (two when there are few
 //       rows per token, as in reduce_kernel: half as many waves, each with as many loads in flight)
-template <int KMAX, bool FP8, bool FACTOR, bool DIRECT, int CH, int TW>
+template <int KMAX, bool FP8, bool FACTOR, int FROM, int CH, int TW>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ? 8 : 4, 8))) void reduce_packed_kernel(const uint64_t* __restrict__ tbl_mem,
                                                              const CombineRoute* __restrict__ routes, uint32_t stamp,
                                                              RoutingScratch sc, CombineSource cs,
@@ -1277,15 +1345,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
     uint64_t src = (uint64_t)zero_row, ssrc = (uint64_t)zero_row;
     float w = 0.0f, f = 1.0f;
     int sstride = 0;                     // bytes between a row's consecutive scale groups (0: the zero row)
-    int live = 1;                        // DIRECT: loaded here, looked at after the payload loads are issued
+    int live = 1;                        // loaded here, looked at after the payload loads are issued (not: kFromRoutes)
+    constexpr int kLanes = lanes_per_selection<FROM, KMAX>();      // selection k's row ends up in lane k * kLanes
     {
         int e = 0, slot = 0;
         bool ok = false;
         float wl = 0.0f;
-        if (DIRECT) {
+        if (FROM != kFromRoutes) {
             const uint64_t w_row = rank_ptr(tbl, cs.topk_weights, CF_TOPK_W, R, r) + (uint64_t)((int64_t)t * K) * 4;
-            wl = load_f32(w_row + (uint64_t)(lane < K ? lane : 0) * 4);
-            const DirectRow d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, lane);
+            wl = load_f32(w_row + (uint64_t)(lane / kLanes < K ? lane / kLanes : 0) * 4);
+            DirectRow d;
+            if constexpr (FROM == kFromHandle) d = search_row<kLanes>(tbl, cs, R, E, K, max_tokens, r, t, lane);
+            else d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, lane);
             ok = d.has;
             e = d.e;
             slot = d.slot;
@@ -1329,12 +1400,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
     float sv[KMAX], wk[KMAX], fk[KMAX];
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
-        const uint64_t p = read_lane_u64(src, k);
+        const uint64_t p = read_lane_u64(src, k * kLanes);
 #pragma unroll
         for (int c = 0; c < CH; ++c) v[k][c] = load16<true>((const void*)(p + poff[c]));
         if (FP8) {
-            const uint64_t sp = read_lane_u64(ssrc, k);
-            const int st = __builtin_amdgcn_readlane(sstride, k);
+            const uint64_t sp = read_lane_u64(ssrc, k * kLanes);
+            const int st = __builtin_amdgcn_readlane(sstride, k * kLanes);
             sv[k] = load_f32(sp + (uint64_t)((int64_t)group * st));
         } else {
             sv[k] = 1.0f;
@@ -1342,15 +1413,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
     }
 
     // a row of a rank the token's owner sees as inactive was fetched before that was known: drop it
-    if (DIRECT && live == 0) w = 0.0f;
+    if (FROM != kFromRoutes && live == 0) w = 0.0f;
     // the expert's factor was loaded behind the row table, like `live`: looked at only now, when the payload
     // loads are on their way
     asm volatile("" : "+v"(f));
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
-        fk[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), k));
-        wk[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k));
-        if (DIRECT && __builtin_amdgcn_readlane(live, k) == 0) {
+        fk[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), k * kLanes));
+        wk[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k * kLanes));
+        if (FROM != kFromRoutes && __builtin_amdgcn_readlane(live, k * kLanes) == 0) {
 #pragma unroll
             for (int c = 0; c < CH; ++c) v[k][c] = make_uint4(0, 0, 0, 0);
             sv[k] = 0.0f;
@@ -1859,7 +1930,7 @@ struct ReduceLaunch {
 };
 }  // namespace
 
-template <int KMAX, int CH, bool DIRECT>
+template <int KMAX, int CH, int FROM>
 static hipError_t launch_reduce_t(const ReduceLaunch& rl, const Dims& d, const Tuning& t, hipStream_t stream) {
     const int slabs = (d.H + CH * 512 - 1) / (CH * 512);
     const long long total = (long long)d.R * d.Tgrid * slabs;
@@ -1873,20 +1944,25 @@ static hipError_t launch_reduce_t(const ReduceLaunch& rl, const Dims& d, const T
     // the 32 the hardware would run (fewer rows being walked at once), a little at top-11 and top-16; 12
     // waves no longer cover the latency.  With fewer rows per wave it wants all 32 (top-3: 39.6 us against
     // 41.1 at 20).  The limit is imposed with unused dynamic LDS: a CU's 160 KiB hold so many blocks and no more.
-    const int occupancy = t.combine_occupancy >= 0 ? t.combine_occupancy : (d.K >= 7 ? 20 : 0);
+    // Rows from the handle: all 32, which hide the two loads more in front of each wave's payload (whole cycles at 20 /
+    // 24 / 32 waves: 32 x 128 tokens of top-8 149.0 / 144.4 / 144.4 us, with Zipf routing 159.2 / 149.2 / 146.4).
+    const int occupancy = t.combine_occupancy >= 0 ? t.combine_occupancy : (d.K >= 7 && FROM != kFromHandle ? 20 : 0);
     const size_t pad = occupancy_pad_bytes(occupancy, wpb);
     const int words = (int)CF_COUNT * d.R;
-    const bool in_args = d.host_table != nullptr && combine_reads_table(rl.src, DIRECT);
-    if (in_args && (words > kArgTableWords || !(ntl && nts))) return hipErrorInvalidValue;
+    const bool in_args = d.host_table != nullptr && combine_reads_table(rl.src, FROM == kFromDispatch);
+    // (variants for the table in the arguments, and for rows from the handle, exist with the streaming hints only)
+    if ((in_args && words > kArgTableWords) || ((in_args || FROM == kFromHandle) && !(ntl && nts))) return hipErrorInvalidValue;
 #define MCEP_REDUCE(A, B, TW)                                                                                    \
-    hipLaunchKernelGGL((reduce_kernel<KMAX, CH, A, B, DIRECT, TW>), dim3(blocks), dim3(wpb * 64), pad, stream,   \
+    hipLaunchKernelGGL((reduce_kernel<KMAX, CH, A, B, FROM, TW>), dim3(blocks), dim3(wpb * 64), pad, stream,   \
                        rl.d_tbl, rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row, d.R, d.E, d.K,             \
                        d.max_tokens, d.H, slabs, d.Tgrid, (int)total, arg_table<TW>(d.host_table, words))
     if (in_args) MCEP_REDUCE(true, true, kArgTableWords);
     else if (ntl && nts) MCEP_REDUCE(true, true, 0);
-    else if (ntl) MCEP_REDUCE(true, false, 0);
-    else if (nts) MCEP_REDUCE(false, true, 0);
-    else MCEP_REDUCE(false, false, 0);
+    else if constexpr (FROM != kFromHandle) {
+        if (ntl) MCEP_REDUCE(true, false, 0);
+        else if (nts) MCEP_REDUCE(false, true, 0);
+        else MCEP_REDUCE(false, false, 0);
+    }
 #undef MCEP_REDUCE
     return hipGetLastError();
 }
@@ -1899,10 +1975,12 @@ hipError_t launch_reduce(const uint64_t* d_tbl, const CombineRoute* d_routes, ui
     const int ch = t.combine_chunks > 0 ? (t.combine_chunks >= 2 ? 2 : 1) : (d.K <= 4 ? 2 : 1);
 #define MCEP_K(KMAX)                                                                                   \
     do {                                                                                               \
-        if (direct) return ch == 2 ? launch_reduce_t<KMAX, 2, true>(rl, d, t, stream)                  \
-                                   : launch_reduce_t<KMAX, 1, true>(rl, d, t, stream);                 \
-        return ch == 2 ? launch_reduce_t<KMAX, 2, false>(rl, d, t, stream)                             \
-                       : launch_reduce_t<KMAX, 1, false>(rl, d, t, stream);                            \
+        if (direct) return ch == 2 ? launch_reduce_t<KMAX, 2, kFromDispatch>(rl, d, t, stream)         \
+                                   : launch_reduce_t<KMAX, 1, kFromDispatch>(rl, d, t, stream);        \
+        if (src.search) return ch == 2 ? launch_reduce_t<KMAX, 2, kFromHandle>(rl, d, t, stream)       \
+                                       : launch_reduce_t<KMAX, 1, kFromHandle>(rl, d, t, stream);      \
+        return ch == 2 ? launch_reduce_t<KMAX, 2, kFromRoutes>(rl, d, t, stream)                       \
+                       : launch_reduce_t<KMAX, 1, kFromRoutes>(rl, d, t, stream);                      \
     } while (0)
     if (d.K <= 1) MCEP_K(1);
     if (d.K <= 2) MCEP_K(2);
@@ -1914,7 +1992,7 @@ hipError_t launch_reduce(const uint64_t* d_tbl, const CombineRoute* d_routes, ui
 #undef MCEP_K
 }
 
-template <int KMAX, bool FP8, bool FACTOR, bool DIRECT, int CH = 1>
+template <int KMAX, bool FP8, bool FACTOR, int FROM, int CH = 1>
 static hipError_t launch_reduce_packed_t(const ReduceLaunch& rl, const float* d_factor, const Dims& d, const Tuning& t,
                                          hipStream_t stream) {
     const int slab = FP8 ? 1024 : 512 * CH;
@@ -1934,10 +2012,10 @@ static hipError_t launch_reduce_packed_t(const ReduceLaunch& rl, const float* d_
     }
     if (blocks > 0x7fffffffll) return hipErrorInvalidValue;
     const int words = (int)CF_COUNT * d.R;
-    const bool in_args = d.host_table != nullptr && combine_reads_table(rl.src, DIRECT);
+    const bool in_args = d.host_table != nullptr && combine_reads_table(rl.src, FROM == kFromDispatch);
     if (in_args && words > kArgTableWords) return hipErrorInvalidValue;
 #define MCEP_PACKED(TW)                                                                                             \
-    hipLaunchKernelGGL((reduce_packed_kernel<KMAX, FP8, FACTOR, DIRECT, CH, TW>), dim3((unsigned)blocks),           \
+    hipLaunchKernelGGL((reduce_packed_kernel<KMAX, FP8, FACTOR, FROM, CH, TW>), dim3((unsigned)blocks),           \
                        dim3(wpb * 64), 0, stream, rl.d_tbl, rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row,    \
                        d_factor, d.R, d.E, d.K, d.max_tokens, d.H, slabs, d.Tgrid, group_blocks,                    \
                        arg_table<TW>(d.host_table, words))
@@ -1953,8 +2031,9 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
     const ReduceLaunch rl{d_tbl, d_routes, stamp, sc, src, d_zero_row};
     const bool fac = d_factor != nullptr;
 #define MCEP_P4(KMAX, FP8, FACTOR)                                                                   \
-    (direct ? launch_reduce_packed_t<KMAX, FP8, FACTOR, true>(rl, d_factor, d, t, stream)            \
-            : launch_reduce_packed_t<KMAX, FP8, FACTOR, false>(rl, d_factor, d, t, stream))
+    (direct       ? launch_reduce_packed_t<KMAX, FP8, FACTOR, kFromDispatch>(rl, d_factor, d, t, stream) \
+     : src.search ? launch_reduce_packed_t<KMAX, FP8, FACTOR, kFromHandle>(rl, d_factor, d, t, stream)   \
+                  : launch_reduce_packed_t<KMAX, FP8, FACTOR, kFromRoutes>(rl, d_factor, d, t, stream))
 #define MCEP_PK(KMAX)                                                                                \
     do {                                                                                             \
         if (use_fp8) return fac ? MCEP_P4(KMAX, true, true) : MCEP_P4(KMAX, true, false);            \
@@ -1962,8 +2041,9 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
     } while (0)
     // a bf16 payload with few rows per token: two chunks per lane, as in the combine kernel
 #define MCEP_P2(KMAX, FACTOR)                                                                        \
-    (direct ? launch_reduce_packed_t<KMAX, false, FACTOR, true, 2>(rl, d_factor, d, t, stream)       \
-            : launch_reduce_packed_t<KMAX, false, FACTOR, false, 2>(rl, d_factor, d, t, stream))
+    (direct       ? launch_reduce_packed_t<KMAX, false, FACTOR, kFromDispatch, 2>(rl, d_factor, d, t, stream) \
+     : src.search ? launch_reduce_packed_t<KMAX, false, FACTOR, kFromHandle, 2>(rl, d_factor, d, t, stream)   \
+                  : launch_reduce_packed_t<KMAX, false, FACTOR, kFromRoutes, 2>(rl, d_factor, d, t, stream))
     const int ch = t.combine_chunks > 0 ? (t.combine_chunks >= 2 ? 2 : 1) : (d.K <= 4 ? 2 : 1);
     if (!use_fp8 && ch == 2 && d.K <= 2) return fac ? MCEP_P2(2, true) : MCEP_P2(2, false);
     if (!use_fp8 && ch == 2 && d.K <= 4) return fac ? MCEP_P2(4, true) : MCEP_P2(4, false);

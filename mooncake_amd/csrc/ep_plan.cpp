@@ -33,7 +33,8 @@ void plan_units(Dims& d, const Tuning& t) {
 bool combine_reads_table(const CombineSource& src, bool direct) {
     if (src.tokens < 0 || src.out.base == 0) return true;
     // rows come as addresses from the routes, except that the packed combine looks its tensors up either way
-    if (!direct) return src.x.base == 0 || (src.packed_fp8 && src.scales.base == 0);
+    if (!direct && src.search && (src.src_info.base == 0 || src.layout_range.base == 0)) return true;
+    if (!direct && !src.search) return src.x.base == 0 || (src.packed_fp8 && src.scales.base == 0);
     return src.topk_idx.base == 0 || src.topk_weights.base == 0 || src.active.base == 0 || src.x.base == 0 ||
            (src.packed_fp8 && src.scales.base == 0);
 }

@@ -773,6 +773,18 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     src.packed_fp8 = ps.scales != nullptr;
     src.active = uniform_ptr(active_ranks, R, uni);
     src.tokens = uniform_tokens(num_tokens, R, uni);
+    // A handle that is not the last dispatch's: every wave of the reduce kernel looks its token's rows up in it while
+    // an expert cannot have many rows of one rank, whatever the routing; beyond that a resolve launch turns the handle
+    // into routes first.  Whole cycles, resolved / searched: 32 x 64 tokens, hidden 7168, top-8, fp8, rows given
+    // 86.8 / 81.1 us (81.4 when the last dispatch's state is there), Zipf(1.2) routing 84.2 / 79.1; 32 x 128 150.7 /
+    // 144.4 and 150.7 / 146.4; 16 x 256, hidden 4096, bf16 101.4 / 95.7 and 106.9 / 104.3; 8 x 256, 7168, Zipf 88.0 /
+    // 85.6, where the hottest experts' 256 rows of a rank are what the lead shrinks by.
+    src.search = !direct && phases == MC_EP_PHASE_ALL && tgrid <= w->tuning.combine_search_tokens &&
+                 (ps.packed || (w->tuning.combine_nt & 3) == 3);
+    if (src.search) {
+        src.src_info = uniform_ptr(src_info, R, uni);
+        src.layout_range = uniform_ptr(layout_range, R, uni);
+    }
     // The rank table: not needed when every tensor is evenly spaced, else in the kernels' arguments (a recorded call
     // then carries its own), in memory only for worlds too large for that and for the streaming hints that have no
     // such variant.
@@ -786,7 +798,7 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     }
     // sized on every path, so that an eager call prepares the world for any recorded one of the same shape
     if (int rc = ensure_routes(w, (size_t)R * max_tokens * num_topk)) return rc;
-    if (!direct) {
+    if (!direct && !src.search) {
         if (phases & MC_EP_PHASE_LAYOUT) {
             w->stamp += 1;
             // every replay of a recorded call carries the same stamp: clear the routes so that none of an
@@ -1185,6 +1197,7 @@ static int* option_slot(Tuning& t, const char* name) {
     if (!strcmp(name, "uniform")) return &t.uniform;
     if (!strcmp(name, "fp8_arith")) return &t.fp8_arith;
     if (!strcmp(name, "comm_stream")) return &t.comm_stream;
+    if (!strcmp(name, "combine_search_tokens")) return &t.combine_search_tokens;
     if (!strcmp(name, "combine_direct")) return &t.combine_direct;
     if (!strcmp(name, "combine_chunks")) return &t.combine_chunks;
     if (!strcmp(name, "packed_map")) return &t.packed_map;
