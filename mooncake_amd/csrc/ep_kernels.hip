@@ -261,16 +261,30 @@ __device__ __forceinline__ void prefix_expert(const uint64_t* __restrict__ tbl, 
                                               int max_tokens, int upr, int U, int ee, int* pre) {
     const int lane = wave_lane();
     int carry = 0;
-    for (int u0 = 0; u0 < U; u0 += 64) {
-        const int u = u0 + lane;
-        const int c = (u < U) ? sc.ucount[(int64_t)u * E + ee] : 0;
-        const int incl = wave_scan_inclusive(c);
-        if (u < U) {
-            const int excl = carry + incl - c;
-            sc.ubegin[(int64_t)u * E + ee] = excl;
-            pre[u] = excl;
+    // 64 * kAhead units at a time, their loads all in flight before the first scan: one after another they were the
+    // kernel's time (1024 units of 64 experts: 10.6 -> 7.8 us; what is left is one line per lane and access)
+    constexpr int kAhead = 8;
+    for (int u0 = 0; u0 < U; u0 += 64 * kAhead) {
+        int counts[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            const int u = u0 + j * 64 + lane;
+            counts[j] = 0;
+            if (u0 + j * 64 < U) counts[j] = sc.ucount[(int64_t)(u < U ? u : U - 1) * E + ee];
         }
-        carry += __builtin_amdgcn_readlane(incl, 63);
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            if (u0 + j * 64 >= U) break;
+            const int u = u0 + j * 64 + lane;
+            const int c = u < U ? counts[j] : 0;
+            const int incl = wave_scan_inclusive(c);
+            if (u < U) {
+                const int excl = carry + incl - c;
+                sc.ubegin[(int64_t)u * E + ee] = excl;
+                pre[u] = excl;
+            }
+            carry += __builtin_amdgcn_readlane(incl, 63);
+        }
     }
     if (lane == 0) pre[U] = carry;
     // the same wave wrote pre[] and reads it below: a wave's LDS accesses complete in order

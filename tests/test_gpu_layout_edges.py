@@ -1,4 +1,5 @@
-"""Edges of the layout kernels against the oracle, bit for bit: scale counts per row around the 16 that a wave of the
+"""Edges of the layout kernels against the oracle, bit for bit: worlds with as many units of 256 selections as a wave of
+the prefix pass loads at a time (512), one more and one fewer, and scale counts per row around the 16 that a wave of the
 scale transposition takes (whole, with a remainder of whole and of partial 16-byte pieces)."""
 import pytest
 
@@ -13,6 +14,12 @@ def check(oracle, cfg, nt=None, **options):
     h = run_dispatch(cfg, data, num_tokens=nt, poison=True, options={"fused_small": 0, **options})
     ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
     compare_dispatch(h, ref, check_poison=True)
+
+
+@pytest.mark.parametrize("units", [511, 512, 513])
+def test_prefix_over_many_units(gpu_device, oracle, units):
+    announce(f"prefix pass over {units} units")
+    check(oracle, EPConfig("units", 1, units * 32 - 3, 128, 8, 8, False))
 
 
 @pytest.mark.parametrize("groups", [15, 16, 17, 20, 32, 36])
