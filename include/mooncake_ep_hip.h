@@ -97,11 +97,12 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * for measurement sweeps; "combine_search_tokens" (default 256): a combine of a
  * handle that is not the last dispatch's is one launch while no rank combines
  * more tokens than this, two beyond (0: always two); "fused_small": 1 (default) dispatches a world of at
- * most "fused_small_max" (default 4096) selections and 8 ranks per 1024
- * hidden elements (32 ranks in all) in one kernel launch - provided the ranks'
- * index lists make at most "fused_small_rounds" rounds of 512 entries, each
- * list counted by itself and the rounds shared out over a wave per 1024 hidden
- * elements, up to 8 (default -1: 6 for an fp8 payload, 4 for bf16) - and 0
+ * most "fused_small_max" (default 4096) selections and 8 ranks per wave of a
+ * block (32 ranks in all) in one kernel launch - provided the ranks' index
+ * lists make at most "fused_small_rounds" rounds of 512 entries per wave, each
+ * list counted by itself (default -1: 6 for an fp8 payload, 4 for bf16); a
+ * block has a wave per 1024 hidden elements, 4 to 8 of them, and counts as one
+ * wave up to 512 - and 0
  * always takes the count / pack / scale-transpose launches;
  * "last_dispatch_launches", "last_combine_launches": read them to learn how
  * many kernels the world's last dispatch / combine call enqueued (a rank-table

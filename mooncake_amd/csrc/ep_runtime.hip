@@ -549,10 +549,11 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     // A world that names few selections is dispatched in one launch, every block rebuilding the routing it
     // needs from the index lists (dispatch_small_kernel); the rank table then travels in kernel arguments.
     // What that costs grows with the rounds of index-list entries a wave of a late token reads one after another
-    // (every rank's list is at least one round; a block's payload waves share them out), which is weighed against
-    // the launches it saves - two for an fp8 payload, one for bf16: up to six rounds and four.  At six rounds a wave
-    // the one launch takes 8.5 us (12 ranks, two payload waves, fp8) where the three kernels and the gaps between
-    // them take 15.
+    // (every rank's list is at least one round; a block's waves share them out), which is weighed against the
+    // launches it saves - two for an fp8 payload, one for bf16: up to six rounds a wave and four.  Dispatches apart /
+    // in one, us: fp8, one to six rounds 10.3 / 4.5 (hidden 256) to 12.2 / 8.6 (24 ranks of 20 tokens, 3072), eight
+    // 13.0 / 11.2 (32 ranks of 16, 4096); bf16, two rounds 8.9 / 7.1 (8 ranks of 64, 2048), four 9.0 / 8.1, eight
+    // 8.9 / 8.6.
     const int rounds_limit = w->tuning.fused_small_rounds >= 0 ? w->tuning.fused_small_rounds : (use_fp8 ? 6 : 4);
     const long long wave_rounds = (list_rounds + small_waves(hidden) - 1) / small_waves(hidden);
     const bool fused = w->tuning.fused_small != 0 && phases == MC_EP_PHASE_ALL && tgrid > 0 && R <= kSmallRanks &&

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     EPConfig("ranks_12_two_slabs", 12, 68, 1152, 108, 5, True),      # 12 lists of 340 entries on four waves
-    EPConfig("ranks_16_two_slabs", 16, 8, 2048, 32, 3, False),       # the most ranks two slabs take
+    EPConfig("ranks_32_four_waves", 32, 8, 640, 32, 3, False),       # the most ranks there are, on the fewest waves
     EPConfig("ranks_32_eight_slabs", 32, 16, 7424, 64, 8, True),     # the most ranks there are
     EPConfig("rounds_512_513", 3, 171, 1152, 24, 3, False),          # 513 entries: a round and one entry
     EPConfig("rounds_6_of_512", 1, 384, 4096, 64, 8, True),          # one list, six whole rounds
@@ -41,3 +41,19 @@ def test_shared_lists_match_oracle(gpu_device, oracle, cfg, is_ragged):
     assert h.world.get_option("last_dispatch_launches") == 1
     ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
     compare_dispatch(h, ref, check_poison=True)
+
+
+def test_size_rule_per_wave(gpu_device, oracle):
+    """Up to six rounds a wave for fp8 and four for bf16: four waves up to hidden 4096, a wave per 1024 elements above."""
+    announce("one-launch dispatch, the size rule per wave")
+    for cfg, one in ((EPConfig("fp8_24_lists", 24, 4, 1152, 24, 2, True), True),
+                     (EPConfig("fp8_25_lists", 25, 4, 1152, 25, 2, True), False),
+                     (EPConfig("bf16_16_lists", 16, 4, 640, 16, 2, False), True),
+                     (EPConfig("bf16_17_lists", 17, 4, 640, 17, 2, False), False),
+                     (EPConfig("fp8_30_lists_5_waves", 30, 4, 4224, 30, 2, True), True),
+                     (EPConfig("fp8_31_lists_5_waves", 31, 4, 4224, 31, 2, True), False)):
+        data = generate(cfg, seed=62)
+        h = run_dispatch(cfg, data, poison=True)
+        assert (h.world.get_option("last_dispatch_launches") == 1) == one, cfg.name
+        ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
+        compare_dispatch(h, ref, check_poison=True)
