@@ -1506,6 +1506,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
 // is better loaded with the streaming hint (bf16, 8 x 512: 187 against 201).
 constexpr int kCastWaves = 4;
 constexpr int kCastCols = 1024;
+constexpr int kCastMaxExperts = 4096;
 
 template <bool FP8, int TW>
 __global__ __launch_bounds__(kCastWaves * 64) void cast_back_kernel(const uint64_t* __restrict__ tbl_mem, RankPtr counts,
@@ -2078,7 +2079,8 @@ hipError_t launch_cast_back(const uint64_t* d_tbl, void* /*scratch: none needed*
     const int parts = (d.H + kCastCols - 1) / kCastCols;
     const long long blocks = cast_back_chunks(max_rows, d.E) * parts;
     if (blocks <= 0) return hipSuccess;
-    if (blocks > 0x7fffffffll) return hipErrorInvalidValue;
+    // (every block looks at all the counts, which is meant for no more than this many)
+    if (blocks > 0x7fffffffll || d.E > kCastMaxExperts) return hipErrorInvalidValue;
     // The table is in the arguments, with the counts' address and spacing beside it where they are even: one
     // dependent load less in front of every block.
     constexpr int kWords = (int)XF_COUNT * 32;

@@ -61,3 +61,19 @@ def test_chunk_edges(gpu_device, oracle, shape, use_fp8):
                 assert bool((got[r].view(torch.int16) == FILL).all()), f"rank {r} takes no part but was written"
             else:
                 assert torch.equal(got[r].view(torch.int16), want[r].view(torch.int16)), f"rank {r}"
+
+
+@pytest.mark.parametrize("experts", [4096, 4098])
+def test_more_experts_than_a_block_looks_through(gpu_device, experts):
+    cfg = EPConfig("experts", 2, 1, 128, experts, 1, False)
+    announce(f"cast back with {experts} experts")
+    h = WorldHarness(cfg)
+    h.alloc_dispatch_outputs(poison=False)
+    h.alloc_combine_io()
+    h.recv_count.zero_()
+    if experts <= 4096:
+        h.cast_back(None)
+    else:
+        with pytest.raises(RuntimeError):
+            h.cast_back(None)
+    torch.cuda.synchronize()
