@@ -571,9 +571,11 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         if (int rc = finish_round(w, w->unfinished.get())) return rc;
     Dims d{R, num_experts, num_topk, hidden, max_tokens, tgrid};
     plan_units(d, w->tuning);
-    // the count kernel keeps per-wave counts and prefixes of every expert in LDS
-    MC_ASSERT(fused || count_lds_bytes(d) <= kMaxCountLdsBytes);
-    MC_ASSERT(fused || d.units() <= kMaxUnits);
+    // The count kernel keeps per-wave counts and prefixes of every expert in LDS.  A world whose lists a wave could count
+    // alone needs none of it; any other one has to fit, also where the rule above happens to give it one launch.
+    const bool alone = fused && R <= kSmallWaveRanks && list_rounds <= (long long)rounds_limit;
+    MC_ASSERT(alone || count_lds_bytes(d) <= kMaxCountLdsBytes);
+    MC_ASSERT(alone || d.units() <= kMaxUnits);
     const size_t UE = (size_t)d.units() * num_experts;
     const size_t stage_floats = use_fp8 ? (size_t)R * max_tokens * (hidden / 128) : 0;
 

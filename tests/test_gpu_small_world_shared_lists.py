@@ -57,3 +57,14 @@ def test_size_rule_per_wave(gpu_device, oracle):
         assert (h.world.get_option("last_dispatch_launches") == 1) == one, cfg.name
         ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
         compare_dispatch(h, ref, check_poison=True)
+
+
+def test_what_no_path_but_this_could_take(gpu_device):
+    """More experts than the count kernel's LDS holds: taken while one wave could count the lists, refused beyond."""
+    announce("one-launch dispatch, more experts than the other path takes")
+    cfg = EPConfig("few_lists", 4, 16, 1152, 8200, 8, True)
+    h = run_dispatch(cfg, generate(cfg, seed=63), poison=False)
+    assert h.world.get_option("last_dispatch_launches") == 1
+    cfg = EPConfig("many_lists", 10, 4, 1152, 8200, 8, True)
+    with pytest.raises(RuntimeError):
+        run_dispatch(cfg, generate(cfg, seed=63), poison=False)
