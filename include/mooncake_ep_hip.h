@@ -96,13 +96,16 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * "packed_map": tuning knobs
  * for measurement sweeps; "combine_search_tokens" (default 256): a combine of a
  * handle that is not the last dispatch's is one launch while no rank combines
- * more tokens than this, two beyond (0: always two); "fused_small": 1 (default) dispatches a world of at
- * most "fused_small_max" (default 4096) selections and 8 ranks per wave of a
- * block (32 ranks in all) in one kernel launch - provided the ranks' index
- * lists make at most "fused_small_rounds" rounds of 512 entries per wave, each
- * list counted by itself (default -1: 6 for an fp8 payload, 4 for bf16); a
- * block has a wave per 1024 hidden elements, 4 to 8 of them, and counts as one
- * wave up to 512 - and 0
+ * more tokens than this, two beyond (0: always two); "fused_small": 1 (default) dispatches a
+ * small world in one kernel launch - at most "fused_small_max" (default 4096)
+ * selections, and few rounds of 512 index-list entries: up to 8 ranks whose
+ * lists make at most "fused_small_rounds" rounds, each list counted by itself
+ * (default -1: 6 for an fp8 payload, 4 for bf16), or, above 512 hidden
+ * elements, at most that many per wave of a block and at most 8 ranks per wave
+ * (32 in all), where a block has a wave per 1024 hidden elements, 4 to 8 of
+ * them, and goes through as many rounds of every rank as the longest list has;
+ * by default it may then be at most 16384 (bf16: 8192) rounds for all tokens
+ * together - and 0
  * always takes the count / pack / scale-transpose launches;
  * "last_dispatch_launches", "last_combine_launches": read them to learn how
  * many kernels the world's last dispatch / combine call enqueued (a rank-table

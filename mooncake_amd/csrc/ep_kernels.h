@@ -62,17 +62,13 @@ struct TableChunk {
 // round of its own).
 constexpr int kSmallRanks = 32;
 constexpr int kSmallWaveRanks = 8;
-constexpr int kSmallListRound = 512;  // index-list entries a wave of dispatch_small_kernel has in flight at a time
+constexpr int kSmallListRound = 512;  // index-list entries a wave of the one-launch dispatch has in flight at a time
 constexpr int kSmallWaves = 8;        // most waves a block of dispatch_small_kernel has
 // its waves per block (a block is one token): one per 1024-element slab, at least four, so that a block of few slabs does
 // not wait for long lists
 constexpr int small_block_waves(int hidden) {
     return (hidden + 1023) / 1024 > kSmallWaves ? kSmallWaves : (hidden > 4096 ? (hidden + 1023) / 1024 : 4);
 }
-// The waves that the size rule shares the lists out over.  Rows of half a slab and less keep the line that was drawn
-// when a wave counted alone: the one launch would pay beyond it too (7 lists of 16 entries, hidden 256, fp8: 10.3 us
-// apart, 4.5 in one), but which of these calls take how many launches is relied on.
-constexpr int small_waves(int hidden) { return hidden <= 512 ? 1 : small_block_waves(hidden); }
 struct SmallTable {
     uint64_t v[(int)DF_COUNT * kSmallRanks];
 };
@@ -178,8 +174,8 @@ struct Tuning {
     int comm_stream = 0;       // 1: per-rank rounds always run on the world's communication stream
     int fused_small = 1;       // dispatch of a small world (see dispatch_small_kernel) in one launch
     int fused_small_max = 4096;   // ... when the world names at most this many selections
-    int fused_small_rounds = -1;  // ... in at most this many rounds of kSmallListRound index-list entries per wave of a
-                                  // block (small_waves), each rank's list counted by itself; -1: 6 for an fp8 payload, 4 for bf16
+    int fused_small_rounds = -1;  // ... in at most this many rounds of kSmallListRound index-list entries per wave
+                                  // (plan_small); -1: what measurement chose
     int last_dispatch_launches = 0;   // read-only in spirit: kernels the world's last dispatch / combine call enqueued
     int last_combine_launches = 0;    // (a rank-table upload counts; launches of other phases' calls do not)
     int blocking = 0;          // 1: a per-rank call returns only when its round has been launched (a thread per rank)
@@ -188,8 +184,14 @@ struct Tuning {
 };
 
 // Chooses the unit plan for a shape (summed when allowed, the shape permits and there are tokens).
-// (plan_units, combine_reads_table, count_lds_bytes and cast_back_chunks are host arithmetic: ep_plan.cpp.)
+// (plan_units, plan_small, combine_reads_table, count_lds_bytes and cast_back_chunks are host arithmetic: ep_plan.cpp.)
 void plan_units(Dims& d, const Tuning& t);
+// Whether a dispatch of the world takes one launch (the sizes alone decide).
+struct SmallPlan {
+    bool fused = false;
+    bool single = false;       // few enough lists that a wave counting alone could take them
+};
+SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t);
 // Whether the reduce kernels look anything up in the rank table: nothing when every tensor they touch is evenly spaced.
 bool combine_reads_table(const CombineSource& src, bool direct);
 

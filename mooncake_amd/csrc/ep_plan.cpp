@@ -30,6 +30,39 @@ void plan_units(Dims& d, const Tuning& t) {
     d.plan = p;
 }
 
+SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t) {
+    long long tokens = 0, lists = 0;           // tokens; rounds of kSmallListRound entries, each rank's list by itself
+    int most = 0;
+    for (int r = 0; r < R; ++r) {
+        tokens += num_tokens[r];
+        lists += ((long long)num_tokens[r] * K + kSmallListRound - 1) / kSmallListRound;
+        if (num_tokens[r] > most) most = num_tokens[r];
+    }
+    SmallPlan p;
+    if (t.fused_small == 0 || most == 0 || tokens * K > (long long)t.fused_small_max) return p;
+    const bool chosen = t.fused_small_rounds >= 0;      // the option replaces the measured lines
+    const long long limit = chosen ? t.fused_small_rounds : (use_fp8 ? 6 : 4);
+    const int waves = small_block_waves(hidden);
+    p.single = R <= kSmallWaveRanks && lists <= limit;
+    if (p.single) {
+        p.fused = true;
+        return p;
+    }
+    // The waves of a block share the lists, and go through as many rounds of every rank as the longest list has.  Two
+    // prices, against the launches saved (two for fp8, one for bf16).  The rounds a wave of a late token reads one after
+    // another; dispatches apart / in one, us: fp8, one to six 10.3 / 4.5 to 12.2 / 8.6 (24 ranks of 20 tokens, hidden
+    // 3072), eight 13.0 / 11.2 (32 ranks of 16, 4096); 12 ranks of 8 and one of 256 top-8 tokens, twelve 12.0 / 14.7; bf16,
+    // two 8.9 / 7.1 (8 ranks of 64, 2048), four 9.0 / 8.1.  And the rounds of all tokens together, which fill the chip: top-4,
+    // 1024 tokens of one rank (8192) fp8 11.1 / 7.9, bf16 8.1 / 7.5 at hidden 1024 and 13.3 / 9.1, 11.5 / 9.2 at 4096;
+    // top-2, 2048 tokens (16384) 11.4 / 10.1 and 16.0 / 12.4, bf16 8.1 / 9.6 and 13.6 / 12.9, with one hot expert in eight
+    // 11.5 / 13.1, 8.4 / 12.4; top-1, 4096 tokens (32768) 12.5 / 15.1 and 19.6 / 18.3, hot 12.8 / 33.3.  Rows of half a slab
+    // and less have not been measured over that range, and stay with the separate launches.
+    const long long walked = (long long)R * (((long long)most * K + kSmallListRound - 1) / kSmallListRound);
+    p.fused = hidden > 512 && R <= kSmallRanks && R <= kSmallWaveRanks * waves &&
+              (walked + waves - 1) / waves <= limit && (chosen || tokens * walked <= (use_fp8 ? 16384 : 8192));
+    return p;
+}
+
 bool combine_reads_table(const CombineSource& src, bool direct) {
     if (src.tokens < 0 || src.out.base == 0) return true;
     // rows come as addresses from the routes, except that the packed combine looks its tensors up either way

@@ -523,7 +523,6 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         MC_ASSERT(recv_scales != nullptr);
     }
     int tgrid = 0;
-    long long selections = 0, list_rounds = 0;
     // the rank table: on the stack, so that the allocation-free variant touches no heap either
     uint64_t tbl[(size_t)DF_COUNT * MC_EP_MAX_QP_COUNT];
     const size_t tbl_words = (size_t)DF_COUNT * R;
@@ -543,22 +542,12 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         tbl[DF_LAYOUT_RANGE * R + r] = layout_range[r];
         tbl[DF_NUM_TOKENS * R + r] = (uint64_t)num_tokens[r];
         if (num_tokens[r] > tgrid) tgrid = num_tokens[r];
-        selections += (long long)num_tokens[r] * num_topk;
-        list_rounds += ((long long)num_tokens[r] * num_topk + kSmallListRound - 1) / kSmallListRound;
     }
-    // A world that names few selections is dispatched in one launch, every block rebuilding the routing it
-    // needs from the index lists (dispatch_small_kernel); the rank table then travels in kernel arguments.
-    // What that costs grows with the rounds of index-list entries a wave of a late token reads one after another
-    // (every rank's list is at least one round; a block's waves share them out), which is weighed against the
-    // launches it saves - two for an fp8 payload, one for bf16: up to six rounds a wave and four.  Dispatches apart /
-    // in one, us: fp8, one to six rounds 10.3 / 4.5 (hidden 256) to 12.2 / 8.6 (24 ranks of 20 tokens, 3072), eight
-    // 13.0 / 11.2 (32 ranks of 16, 4096); bf16, two rounds 8.9 / 7.1 (8 ranks of 64, 2048), four 9.0 / 8.1, eight
-    // 8.9 / 8.6.
-    const int rounds_limit = w->tuning.fused_small_rounds >= 0 ? w->tuning.fused_small_rounds : (use_fp8 ? 6 : 4);
-    const long long wave_rounds = (list_rounds + small_waves(hidden) - 1) / small_waves(hidden);
-    const bool fused = w->tuning.fused_small != 0 && phases == MC_EP_PHASE_ALL && tgrid > 0 && R <= kSmallRanks &&
-                       R <= kSmallWaveRanks * small_waves(hidden) &&
-                       selections <= (long long)w->tuning.fused_small_max && wave_rounds <= (long long)rounds_limit;
+    // A world that names few selections is dispatched in one launch, which rebuilds the routing it needs from the index
+    // lists (dispatch_small_kernel); the rank table then travels in kernel arguments.
+    const SmallPlan small = phases == MC_EP_PHASE_ALL ? plan_small(num_tokens, R, num_topk, hidden, use_fp8 != 0, w->tuning)
+                                                      : SmallPlan{};
+    const bool fused = small.fused;
     DeviceGuard guard(w->device);
     w->launches = 0;
     struct Tally {                                // the option "last_dispatch_launches", on every way out
@@ -573,9 +562,9 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     plan_units(d, w->tuning);
     // The count kernel keeps per-wave counts and prefixes of every expert in LDS.  A world whose lists a wave could count
     // alone needs none of it; any other one has to fit, also where the rule above happens to give it one launch.
-    const bool alone = fused && R <= kSmallWaveRanks && list_rounds <= (long long)rounds_limit;
-    MC_ASSERT(alone || count_lds_bytes(d) <= kMaxCountLdsBytes);
-    MC_ASSERT(alone || d.units() <= kMaxUnits);
+    const bool single = fused && small.single;
+    MC_ASSERT(single || count_lds_bytes(d) <= kMaxCountLdsBytes);
+    MC_ASSERT(single || d.units() <= kMaxUnits);
     const size_t UE = (size_t)d.units() * num_experts;
     const size_t stage_floats = use_fp8 ? (size_t)R * max_tokens * (hidden / 128) : 0;
 

@@ -68,3 +68,24 @@ def test_what_no_path_but_this_could_take(gpu_device):
     cfg = EPConfig("many_lists", 10, 4, 1152, 8200, 8, True)
     with pytest.raises(RuntimeError):
         run_dispatch(cfg, generate(cfg, seed=63), poison=False)
+
+
+def test_size_rule_prices_the_rounds_that_are_walked(gpu_device, oracle):
+    """A wave goes through as many rounds of every rank as the longest list has, and every token goes through them: very
+    uneven lists and thousands of tokens with one or two selections each take the separate launches."""
+    announce("one-launch dispatch, the size rule for uneven lists and many tokens")
+    cases = [
+        (EPConfig("8_ranks_one_long", 8, 440, 1024, 64, 8, True), [440] + [10] * 7, False),     # 8 x 7 rounds on 4 waves
+        (EPConfig("12_ranks_last_long", 12, 256, 1024, 48, 8, True), [8] * 11 + [256], False),
+        (EPConfig("4_ranks_one_long", 4, 320, 1024, 64, 8, True), [320, 8, 8, 8], True),        # 4 x 5 on 4 waves
+        (EPConfig("top1_4096", 1, 4096, 640, 8, 1, True), None, False),                         # 32768 rounds in all
+        (EPConfig("top2_2048", 1, 2048, 640, 8, 2, True), None, True),                          # 16384
+        (EPConfig("top2_2048_bf16", 1, 2048, 640, 8, 2, False), None, False),
+        (EPConfig("top4_1024_bf16", 1, 1024, 640, 8, 4, False), None, True),                    # 8192
+    ]
+    for cfg, nt, one in cases:
+        data = generate(cfg, seed=67)
+        h = run_dispatch(cfg, data, num_tokens=nt, poison=True)
+        assert (h.world.get_option("last_dispatch_launches") == 1) == one, cfg.name
+        ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
+        compare_dispatch(h, ref, check_poison=True)
