@@ -186,9 +186,10 @@ struct Tuning {
 // Chooses the unit plan for a shape (summed when allowed, the shape permits and there are tokens).
 // (plan_units, plan_small, combine_reads_table, count_lds_bytes and cast_back_chunks are host arithmetic: ep_plan.cpp.)
 void plan_units(Dims& d, const Tuning& t);
-// Whether a dispatch of the world takes one launch (the sizes alone decide).
+// Whether a dispatch of the world takes one launch (the sizes alone decide), and which of the two kernels.
 struct SmallPlan {
     bool fused = false;
+    bool alone = false;        // dispatch_alone_kernel: every wave counts by itself; else dispatch_small_kernel
     bool single = false;       // few enough lists that a wave counting alone could take them
 };
 SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t);
@@ -204,8 +205,8 @@ hipError_t launch_pack(const uint64_t* d_tbl, const RoutingScratch& sc, const Di
                        hipStream_t stream);
 // The whole dispatch of a small world in one launch (layout, payload, scales, src_info, counts, ranges, and
 // selrow for a combine of the same handle).  The caller has checked: R <= kSmallRanks, d.Tgrid > 0.
-hipError_t launch_dispatch_small(const SmallTable& tb, int32_t* d_selrow, const Dims& d, bool use_fp8, const Tuning& t,
-                                 hipStream_t stream);
+hipError_t launch_dispatch_small(const SmallTable& tb, int32_t* d_selrow, const Dims& d, bool use_fp8, bool alone,
+                                 const Tuning& t, hipStream_t stream);
 // packed: routes carry (expert, row) instead of a row address
 hipError_t launch_resolve(const uint64_t* d_tbl, CombineRoute* d_routes, uint32_t stamp, bool packed, const Dims& d,
                           const Tuning& t, hipStream_t stream);

@@ -46,6 +46,17 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
     p.single = R <= kSmallWaveRanks && lists <= limit;
     if (p.single) {
         p.fused = true;
+        // Every wave counting by itself (dispatch_alone_kernel): nothing to set up and no barrier, but each entry is
+        // compared with each of the token's K experts.  Dispatch, us, alone / shared: one round of one rank's list, 8
+        // tokens of hidden 7168, fp8, top-4 4.1 / 4.6, top-8 5.0 / 5.1 (hidden 4096 4.9 / 4.7); bf16, top-8 4.6 / 5.2 (4096
+        // 4.6 / 4.5), top-16 6.2 / 6.8.  More rounds: top-1, 2048 tokens of hidden 1024, fp8 6.0 / 8.2 (12.4 when nine
+        // tokens in ten name one expert, for whose LDS counter the shared count queues); top-2, 1024 tokens 5.6 / 6.2;
+        // top-4, 512 tokens 6.4 / 5.5.  Several ranks, top-1: 4 x 512 tokens 6.4 / 8.4, 2 x 256 4.6 / 4.9, but 4 x 64, where
+        // most of a round is missing, 5.6 / 4.3.
+        if (R == 1 && (long long)most * K <= kSmallListRound)
+            p.alone = K <= 4 || (K <= 8 && !use_fp8) || waves > 4;
+        else
+            p.alone = K <= 2 && (R == 1 || most * K >= 256);
         return p;
     }
     // The waves of a block share the lists, and go through as many rounds of every rank as the longest list has.  Two

@@ -544,7 +544,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         if (num_tokens[r] > tgrid) tgrid = num_tokens[r];
     }
     // A world that names few selections is dispatched in one launch, which rebuilds the routing it needs from the index
-    // lists (dispatch_small_kernel); the rank table then travels in kernel arguments.
+    // lists (dispatch_small_kernel, dispatch_alone_kernel); the rank table then travels in kernel arguments.
     const SmallPlan small = phases == MC_EP_PHASE_ALL ? plan_small(num_tokens, R, num_topk, hidden, use_fp8 != 0, w->tuning)
                                                       : SmallPlan{};
     const bool fused = small.fused;
@@ -657,7 +657,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     if (fused) {
         SmallTable st{};
         memcpy(st.v, tbl, tbl_words * sizeof(uint64_t));
-        MC_HIP(launch_dispatch_small(st, sc.selrow, d, use_fp8 != 0, w->tuning, stream));
+        MC_HIP(launch_dispatch_small(st, sc.selrow, d, use_fp8 != 0, small.alone, w->tuning, stream));
         w->launches += 1;
         if (!static_scratch) remember(true);
         return MC_EP_OK;

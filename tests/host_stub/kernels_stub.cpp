@@ -21,7 +21,7 @@ hipError_t launch_pack(const uint64_t*, const RoutingScratch&, const DispatchSou
                        const Tuning&, bool, bool, hipStream_t s) {
     return launched(s);
 }
-hipError_t launch_dispatch_small(const SmallTable&, int32_t*, const Dims&, bool, const Tuning&, hipStream_t s) {
+hipError_t launch_dispatch_small(const SmallTable&, int32_t*, const Dims&, bool, bool, const Tuning&, hipStream_t s) {
     return launched(s);
 }
 hipError_t launch_resolve(const uint64_t*, CombineRoute*, uint32_t, bool, const Dims&, const Tuning&, hipStream_t s) {
