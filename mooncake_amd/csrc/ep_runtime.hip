@@ -765,13 +765,19 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     src.packed_fp8 = ps.scales != nullptr;
     src.active = uniform_ptr(active_ranks, R, uni);
     src.tokens = uniform_tokens(num_tokens, R, uni);
-    // A handle that is not the last dispatch's: every wave of the reduce kernel looks its token's rows up in it while
-    // an expert cannot have many rows of one rank, whatever the routing; beyond that a resolve launch turns the handle
-    // into routes first.  Whole cycles, resolved / searched: 32 x 64 tokens, hidden 7168, top-8, fp8, rows given
-    // 86.8 / 81.1 us (81.4 when the last dispatch's state is there), Zipf(1.2) routing 84.2 / 79.1; 32 x 128 150.7 /
-    // 144.4 and 150.7 / 146.4; 16 x 256, hidden 4096, bf16 101.4 / 95.7 and 106.9 / 104.3; 8 x 256, 7168, Zipf 88.0 /
-    // 85.6, where the hottest experts' 256 rows of a rank are what the lead shrinks by.
-    src.search = !direct && phases == MC_EP_PHASE_ALL && tgrid <= w->tuning.combine_search_tokens &&
+    // A handle that is not the last dispatch's: every wave of the reduce kernel looks its token's rows up in it, or a
+    // resolve launch turns it into routes first.  A look-up scans the rows that the expert got from the token's rank: at
+    // most this many when the handle is that of the tokens combined now and no token names an expert twice (more scan
+    // longer, with the same result), and whatever the routing.  Whole cycles, resolved / searched: 32 x 64 tokens, hidden
+    // 7168, top-8, fp8, rows given 86.8 / 81.1 us (81.4 when the last dispatch's state is there), Zipf(1.2) routing 84.2 /
+    // 79.1; 32 x 128 150.7 / 144.4 and 150.7 / 146.4; 16 x 256, hidden 4096, bf16 101.4 / 95.7 and 106.9 / 104.3; 8 x 256,
+    // 7168, Zipf 88.0 / 85.6, where the hottest experts' 256 rows of a rank are what the lead shrinks by.
+    // From top-9 on a selection has half the lanes and the kernel fewer waves to hide the scan behind.  Combines alone, us,
+    // resolved / searched, nine tokens in ten on an eighth of 64 experts: top-9, 16 ranks of 96, 128 and 256 tokens, hidden
+    // 4096, 28.8 / 27.3, 35.5 / 36.2, 62.8 / 80.1; top-11, 8 of 256, hidden 7168, 67.1 / 78.5.
+    const int search_tokens = num_topk <= 8 ? w->tuning.combine_search_tokens
+                                            : (int)((long long)w->tuning.combine_search_tokens * 3 / 8);
+    src.search = !direct && phases == MC_EP_PHASE_ALL && tgrid <= search_tokens &&
                  (ps.packed || (w->tuning.combine_nt & 3) == 3);
     if (src.search) {
         src.src_info = uniform_ptr(src_info, R, uni);

@@ -78,3 +78,44 @@ def test_the_search_rule(gpu_device):
         h.combine()
         torch.cuda.synchronize()
         assert (h.world.get_option("last_combine_launches") == 1) == one
+
+
+def test_the_search_rule_from_top_9_on(gpu_device):
+    announce("combine: the rule for searched handles, many selections a token")
+    for K, T, one in ((8, 97, True), (9, 96, True), (9, 97, False), (16, 96, True), (16, 97, False)):
+        cfg = EPConfig("rule", 2, T, 128, 16, K, False)
+        h = run_dispatch(cfg, generate(cfg, seed=73), poison=False, options={"combine_direct": 0})
+        h.alloc_combine_io()
+        h.cast_back(None)
+        h.combine()
+        torch.cuda.synchronize()
+        assert (h.world.get_option("last_combine_launches") == 1) == one, (K, T)
+
+
+@pytest.mark.parametrize("tokens", [256, 0], ids=["searched", "resolved"])
+def test_ranges_longer_than_the_tokens_combined(gpu_device, oracle, tokens):
+    """A handle of many tokens, of which a few are combined; and ranges that repeated experts make longer than that."""
+    cfg = EPConfig("long_ranges", 2, 700, 256, 4, 2, True)
+    announce(f"combine of a few tokens of a long handle, search={tokens}")
+    data = generate(cfg, seed=74)
+    data["topk_idx"][1, ::2, 1] = data["topk_idx"][1, ::2, 0]
+    h = run_dispatch(cfg, data, poison=True, options={"combine_search_tokens": tokens})
+    factor = torch.arange(4).float() * 0.1 + 0.5
+    h.alloc_combine_io()
+    h.cast_back(factor)
+    torch.cuda.synchronize()
+    assert int((h.layout_range.cpu() & 0xffffffff).max()) > 300
+    h.num_tokens = [5, 256]
+    want = oracle.combine(h.expert_out.cpu(), data["topk_idx"], data["topk_weights"], h.src_info.cpu(),
+                          h.layout_range.cpu(), h.num_tokens, cfg.max_tokens, 4)
+    for packed in (False, True):
+        h.combined.fill_(7.0)
+        if packed:
+            h.combine_packed(factor)
+        else:
+            h.combine()
+        torch.cuda.synchronize()
+        assert (h.world.get_option("last_combine_launches") == 1) == (tokens > 0)
+        for r, n in enumerate(h.num_tokens):
+            assert torch.equal(h.combined[r, :n].cpu().view(torch.int16), want[r, :n].view(torch.int16)), f"rank {r}"
+            assert bool((h.combined[r, n:] == 7.0).all())
