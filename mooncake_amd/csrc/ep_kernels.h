@@ -164,8 +164,8 @@ struct Tuning {
                                // 1 = the reference kernel's own (see pack_fp8_kernel)
     int combine_direct = 1;    // reuse the last dispatch's routing state when combine gets that dispatch's handle
     int combine_search_tokens = 256;   // any other handle is searched by the reduce kernel itself while no rank combines
-                               // more tokens than this (from top-9 on: three eighths of it); beyond, a resolve launch
-                               // turns it into routes
+                               // more tokens than this (top-5 to top-7: three quarters of it, from top-9 on: three
+                               // eighths); beyond, a resolve launch turns it into routes
     int combine_chunks = 0;    // 16-byte chunks per lane in the combine kernel (1 or 2); 0: by top-k
     int combine_waves = 4;     // waves per block in the combine kernel
     int combine_nt = 3;        // bit 0: streaming loads, bit 1: streaming stores

@@ -772,11 +772,13 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     // 7168, top-8, fp8, rows given 86.8 / 81.1 us (81.4 when the last dispatch's state is there), Zipf(1.2) routing 84.2 /
     // 79.1; 32 x 128 150.7 / 144.4 and 150.7 / 146.4; 16 x 256, hidden 4096, bf16 101.4 / 95.7 and 106.9 / 104.3; 8 x 256,
     // 7168, Zipf 88.0 / 85.6, where the hottest experts' 256 rows of a rank are what the lead shrinks by.
-    // From top-9 on a selection has half the lanes and the kernel fewer waves to hide the scan behind.  Combines alone, us,
-    // resolved / searched, nine tokens in ten on an eighth of 64 experts: top-9, 16 ranks of 96, 128 and 256 tokens, hidden
-    // 4096, 28.8 / 27.3, 35.5 / 36.2, 62.8 / 80.1; top-11, 8 of 256, hidden 7168, 67.1 / 78.5.
-    const int search_tokens = num_topk <= 8 ? w->tuning.combine_search_tokens
-                                            : (int)((long long)w->tuning.combine_search_tokens * 3 / 8);
+    // From top-9 on a selection has half the lanes of top-8's to scan with, and from top-5 to top-7 top-8's with fewer
+    // payload rows to hide the scan behind.  Combines alone, us, resolved / searched, nine tokens in ten on an eighth of 64
+    // experts: top-9, 16 ranks of 96, 128 and 256 tokens, hidden 4096, 28.8 / 27.3, 35.5 / 36.2, 62.8 / 80.1; top-11, 8 of
+    // 256, hidden 7168, 67.1 / 78.5; top-8, 8 of 256, 53.7 / 52.4; Zipf, 8 of 256, top-5 37.4 / 39.2 (192: 29.1 / 29.6),
+    // top-7 47.3 / 48.6 (192: 36.9 / 35.4).
+    const int eighths = num_topk > 8 ? 3 : (num_topk >= 5 && num_topk <= 7 ? 6 : 8);
+    const int search_tokens = (int)((long long)w->tuning.combine_search_tokens * eighths / 8);
     src.search = !direct && phases == MC_EP_PHASE_ALL && tgrid <= search_tokens &&
                  (ps.packed || (w->tuning.combine_nt & 3) == 3);
     if (src.search) {
