@@ -612,8 +612,11 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         if (int rc = order_begin(w, stream, cap)) return rc;
         // (two entries at least: dispatch_small_kernel may read 8 bytes there)
         if (int rc = ensure_scratch(w, &w->d_selrow, &w->selrow_cap, (size_t)R * max_tokens * num_topk + 1)) return rc;
-        if (!fused) {
-            // (the one-launch dispatch keeps no routing state but selrow, and needs no table in memory)
+        // The one-launch dispatch keeps no routing state but selrow.  An eager one prepares the world for the separate
+        // launches all the same: a call of the same shape that is recorded later, with more tokens or in two parts, may
+        // need them and cannot grow scratch.  (Not where a wave could count the lists alone: such a world may be too
+        // large for the count kernel.)
+        if (!fused || (!small.single && !cap.active)) {
             if (int rc = ensure_scratch(w, &w->d_ucount, &w->ucount_cap, UE)) return rc;
             if (int rc = ensure_scratch(w, &w->d_ubegin, &w->ubegin_cap, UE)) return rc;
             if (int rc = ensure_scratch(w, &w->d_ucount_t, &w->ucount_t_cap, (size_t)num_experts * kMaxSummedUnits)) return rc;
@@ -624,6 +627,8 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
                 if (int rc = ensure_scale_stage(w, stage_floats)) return rc;
                 stage = w->d_scale_stage;
             }
+        }
+        if (!fused) {                             // (nor does it need the table in memory)
             const std::vector<uint64_t> tbl_vec(tbl, tbl + tbl_words);
             if (!cap.active && (phases & MC_EP_PHASE_LAYOUT) && (int)tbl_words <= kArgTableWords) {
                 // a new table goes up with the count kernel (a recorded call's is in its own slot instead: what a

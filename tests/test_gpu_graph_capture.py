@@ -127,3 +127,36 @@ def test_recording_refuses_to_grow_scratch_and_per_rank_calls(gpu_device):
     h.dispatch()
     torch.cuda.synchronize()
     assert int(h.recv_count.sum()) == int((h.topk_idx >= 0).sum())
+
+
+@pytest.mark.parametrize("two_parts", [False, True], ids=["more_tokens", "two_parts"])
+def test_a_one_launch_call_prepares_for_recording_the_others(gpu_device, oracle, two_parts):
+    """An eager dispatch of a few tokens (one launch, which needs hardly any scratch) is enough for a recorded one of the
+    same shape that takes the separate launches."""
+    cfg = EPConfig("graph_scratch", 12, 64, 1152, 24, 4, True)
+    announce(f"recorded after a one-launch call {cfg} two_parts={two_parts}")
+    world = ep.World(cfg.num_ranks)
+    few = WorldHarness(cfg, world=world, num_tokens=[3] * cfg.num_ranks)
+    few.load(generate(cfg, seed=90))
+    few.alloc_dispatch_outputs()
+    few.dispatch()
+    torch.cuda.synchronize()
+    assert world.get_option("last_dispatch_launches") == 1
+    world.set_option("fused_small_max", 12 * 64 * 4 - 1)         # so that all the tokens take the separate launches
+    data = generate(cfg, seed=91)
+    h = WorldHarness(cfg, world=world, num_tokens=[5] * cfg.num_ranks if two_parts else None)
+    h.load(data)
+    h.alloc_dispatch_outputs(poison=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        if two_parts:
+            h.dispatch(phases=1)
+            h.dispatch(phases=6)
+        else:
+            h.dispatch()
+    for _ in range(3):
+        g.replay()
+        few.dispatch()
+        torch.cuda.synchronize()
+        ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
+        compare_dispatch(h, ref, check_poison=True)
