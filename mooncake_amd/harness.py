@@ -15,6 +15,9 @@ import torch
 from . import _lib, ep
 from .workloads import EPConfig
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
 
 class WorldHarness:
     def __init__(self, cfg: EPConfig, device: str = "cuda", world: Optional[ep.World] = None,
@@ -29,7 +32,7 @@ class WorldHarness:
         self.recv_x = self.recv_scales_phys = self.recv_count = self.src_info = self.layout_range = None
         self.expert_out = self.combined = None
         self.active_ranks = torch.ones((R, R), dtype=torch.int32, device=self.device)
-        self._prepared = {}     # marshalled whole-world calls, keyed by (kind, present)
+        self._prepared = {}     # the latest marshalled whole-world calls, by everything that is marshalled (_key)
 
     # ------------------------------------------------------------------
     def load(self, data: Dict[str, torch.Tensor]) -> None:
@@ -72,9 +75,29 @@ class WorldHarness:
             return [0] * R
         return [t[r].data_ptr() if (present is None or present[r]) else 0 for r in range(R)]
 
+    # calls kept (a call's addresses; no tensor is kept)
+    _MOST_PREPARED = 64
+
+    def _key(self, kind: str, present: Optional[Sequence[int]], *tensors: Optional[torch.Tensor]) -> tuple:
+        """What a marshalled call was made from: a tensor that was replaced, or given other memory, is another call's."""
+        key = [kind, None if present is None else tuple(present), tuple(self.num_tokens)]
+        for t in tensors:
+            if t is not None:
+                key += (t.data_ptr(), t.stride(0))
+        return tuple(key)
+
+    def _keep(self, key: tuple, call):
+        while len(self._prepared) >= self._MOST_PREPARED:
+            del self._prepared[next(iter(self._prepared))]       # the oldest
+        self._prepared[key] = call
+        return call
+
     def _stream(self, stream: Optional[torch.cuda.Stream]) -> int:
-        s = stream if stream is not None else torch.cuda.current_stream(self.device)
-        return int(s.cuda_stream)
+        if stream is not None:
+            return int(stream.cuda_stream)
+        if _raw_stream is not None and _raw_device is not None:  # (0.2 us; asking for the stream object takes 3.2)
+            return int(_raw_stream(_raw_device() if self.device.index is None else self.device.index))
+        return int(torch.cuda.current_stream(self.device).cuda_stream)
 
     def dispatch(self, phases: int = _lib.PHASE_ALL, stream: Optional[torch.cuda.Stream] = None,
                  present: Optional[Sequence[int]] = None, noalloc: bool = False) -> None:
@@ -91,34 +114,33 @@ class WorldHarness:
                 self._ptrs(self.recv_count, R, present), self._ptrs(self.src_info, R, present),
                 self._ptrs(self.layout_range, R, present), self._stream(stream))
             return
-        key = ("dispatch", None if present is None else tuple(present), self.x.data_ptr(), self.recv_x.data_ptr())
+        key = self._key("dispatch", present, self.x, self.topk_idx, self.recv_x, self.recv_scales_phys, self.recv_count,
+                        self.src_info, self.layout_range)
         call = self._prepared.get(key)
         if call is None:
             nt = [n if (present is None or present[r]) else 0 for r, n in enumerate(self.num_tokens)]
-            call = self.world.prepare_dispatch(
+            call = self._keep(key, self.world.prepare_dispatch(
                 self._ptrs(self.x, R), self._ptrs(self.topk_idx, R), nt, c.hidden, c.num_topk, c.max_tokens,
                 c.num_experts, c.use_fp8, self._ptrs(self.recv_x, R, present),
                 self._ptrs(self.recv_scales_phys, R, present) if c.use_fp8 else None,
                 self._ptrs(self.recv_count, R, present), self._ptrs(self.src_info, R, present),
-                self._ptrs(self.layout_range, R, present))
-            self._prepared[key] = call
+                self._ptrs(self.layout_range, R, present)))
         call(self._stream(stream), phases)
 
     def combine(self, phases: int = _lib.PHASE_ALL, stream: Optional[torch.cuda.Stream] = None,
                 present: Optional[Sequence[int]] = None) -> None:
         c = self.cfg
         R = c.num_ranks
-        key = ("combine", None if present is None else tuple(present), self.expert_out.data_ptr(),
-               self.combined.data_ptr(), self.src_info.data_ptr())
+        key = self._key("combine", present, self.expert_out, self.topk_idx, self.topk_weights, self.src_info,
+                        self.layout_range, self.active_ranks, self.combined)
         call = self._prepared.get(key)
         if call is None:
             nt = [n if (present is None or present[r]) else 0 for r, n in enumerate(self.num_tokens)]
-            call = self.world.prepare_combine(
+            call = self._keep(key, self.world.prepare_combine(
                 self._ptrs(self.expert_out, R, present), self._ptrs(self.topk_idx, R),
                 self._ptrs(self.topk_weights, R), self._ptrs(self.src_info, R), self._ptrs(self.layout_range, R),
                 self._ptrs(self.active_ranks, R), nt, c.hidden, c.num_topk, c.max_tokens, c.num_experts,
-                self._ptrs(self.combined, R))
-            self._prepared[key] = call
+                self._ptrs(self.combined, R)))
         call(self._stream(stream), phases)
 
     def combine_packed(self, factor_per_expert: Optional[torch.Tensor] = None, phases: int = _lib.PHASE_ALL,
@@ -129,18 +151,17 @@ class WorldHarness:
         self._factor = None if factor_per_expert is None else \
             factor_per_expert.to(device=self.device, dtype=torch.float32).contiguous()
         fptr = 0 if self._factor is None else self._factor.data_ptr()
-        key = ("combine_packed", None if present is None else tuple(present), self.recv_x.data_ptr(),
-               self.combined.data_ptr(), self.src_info.data_ptr(), fptr)
+        key = (fptr, *self._key("combine_packed", present, self.recv_x, self.recv_scales_phys, self.topk_idx,
+                                self.topk_weights, self.src_info, self.layout_range, self.active_ranks, self.combined))
         call = self._prepared.get(key)
         if call is None:
             nt = [n if (present is None or present[r]) else 0 for r, n in enumerate(self.num_tokens)]
-            call = self.world.prepare_combine_packed(
+            call = self._keep(key, self.world.prepare_combine_packed(
                 self._ptrs(self.recv_x, R, present),
                 self._ptrs(self.recv_scales_phys, R, present) if c.use_fp8 else None, fptr,
                 self._ptrs(self.topk_idx, R), self._ptrs(self.topk_weights, R), self._ptrs(self.src_info, R),
                 self._ptrs(self.layout_range, R), self._ptrs(self.active_ranks, R), nt, c.hidden, c.num_topk,
-                c.max_tokens, c.num_experts, self._ptrs(self.combined, R))
-            self._prepared[key] = call
+                c.max_tokens, c.num_experts, self._ptrs(self.combined, R)))
         call(self._stream(stream), phases)
 
     # ------------------------------------------------------------------
