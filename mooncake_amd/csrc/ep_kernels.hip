@@ -2006,21 +2006,28 @@ static hipError_t launch_pack_t(Kern kern, const uint64_t* d_tbl, const RoutingS
 hipError_t launch_pack(const uint64_t* d_tbl, const RoutingScratch& sc, const DispatchSource& src, float* scale_stage,
                        const Dims& d, bool use_fp8, const Tuning& t, bool run_pack, bool run_finish,
                        hipStream_t stream) {
-    // Cache hints (bit 0: streaming loads; bit 1: streaming stores, bit 2: write-through stores).  What is measured is
+    // Cache hints (bit 0: streaming loads; bit 1: streaming stores, bit 2: write-through stores).  What is weighed is
     // the whole dispatch -> consumer -> combine cycle with the tensors of three cycles in rotation, because the stores
     // decide where the consumer finds the payload and who waits for its write-back.
-    //   fp8, 80 MiB of payload and more: streaming stores, ordinary loads.  235 MB (32 x 128 tokens, hidden 7168,
-    //     top-8): 167 -> 152 us the cycle with expert rows given, 129 -> 124 with the packed combine, 302 -> 296 with
-    //     the cast back in between; 115 MB: 90.7 -> 83.2, 76.2 -> 72.1, 161.6 -> 154.9; 57 MB: 51.0 -> 51.8,
-    //     41.7 -> 46.0, 90.9 -> 92.4, so below that the payload is left to the cache.
-    //   otherwise: write-through stores, and streaming loads from top-5 up.  bf16, 268 MB (16 x 256 tokens, hidden 4096,
-    //     top-8): 104.3 -> 102.7 when combine reads the payload (112.1 with streaming stores), 200.5 -> 198.3 with the
-    //     cast back in between, 120.4 -> 119.2 with expert rows given; fp8, 57 MB: 51.0 -> 49.6, 41.7 -> 41.5.
-    // A cache flush between the calls of a cycle hides what ordinary stores put off (their write-back falls into the
-    // flush) and so turns the first line around: it is right for callers whose calls follow each other.
-    constexpr long long kStreamBytes = 80ll << 20;
-    const bool stream_out = use_fp8 && (long long)d.R * d.Tgrid * d.K * d.H >= kStreamBytes;
-    const int nt = t.pack_nt >= 0 ? t.pack_nt : (stream_out ? 2 : (d.K > 4 ? 5 : 4));
+    //   fp8, 80 to 320 MiB of payload: streaming stores, ordinary loads.  224 MiB (32 x 128 tokens, hidden 7168, top-8),
+    //     streamed / written through with streaming loads: the cycle with expert rows given 145 / 156 us, with the cast back
+    //     in between 254 to 269 / 258 to 269, with the packed combine 119 / 121, dispatches alone 55 / 64; 112 MiB:
+    //     79 / 82, 132 to 138 / 134 to 137, 65 to 68 / 62 to 69, 32 / 35.  57 MiB: 47.3 / 45.7, 73.7 / 71.6, 43.1 / 41.2,
+    //     so below that the payload is left to the cache.  Above, the cache holds less and less of it either way, while
+    //     the streamed payload's reader loses: 448 MiB 280 to 292 / 288 to 290, 512 to 535 / 517 to 528, but packed 228 to
+    //     244 / 218 to 228, and top-4 275 to 280 / 258 to 263; 336 MiB packed 178 / 171.
+    //     A dispatch behind unrelated memory traffic does not gain: after 512 MiB have been read 224 MiB streamed take 62
+    //     to 71 us, depending on where the tensors lie, written through 60 (112 MiB 37 to 40 / 37); after 512 MiB have been
+    //     written 70 to 85 / 70 (41 to 46 / 39).  The line is for callers whose dispatches and combines follow each other.
+    //   otherwise: write-through stores, and streaming loads from top-5 up and for fp8 payloads above that line (top-4,
+    //     448 MiB, packed: 258 to 263 us the cycle against 267 to 269 with ordinary loads).  bf16, 256 MiB (16 x 256 tokens,
+    //     hidden 4096, top-8), plain stores / through: 98.0 / 96.6 when combine reads the payload (101.4 streamed), 186.2 /
+    //     183.5 with the cast back in between, 112.3 / 111.9 with expert rows given.
+    constexpr long long kStreamFrom = 80ll << 20, kStreamBelow = 320ll << 20;
+    const long long payload = (long long)d.R * d.Tgrid * d.K * d.H;          // bytes, of an fp8 payload
+    const bool stream_out = use_fp8 && payload >= kStreamFrom && payload < kStreamBelow;
+    const bool stream_in = d.K > 4 || (use_fp8 && payload >= kStreamBelow);
+    const int nt = t.pack_nt >= 0 ? t.pack_nt : (stream_out ? 2 : (stream_in ? 5 : 4));
     const bool ntl = (nt & 1) != 0;
     if (use_fp8 && scale_stage == nullptr) return hipErrorInvalidValue;
     hipError_t err = hipSuccess;
