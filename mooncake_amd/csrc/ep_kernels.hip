@@ -2009,13 +2009,14 @@ hipError_t launch_pack(const uint64_t* d_tbl, const RoutingScratch& sc, const Di
     // Cache hints (bit 0: streaming loads; bit 1: streaming stores, bit 2: write-through stores).  What is weighed is
     // the whole dispatch -> consumer -> combine cycle with the tensors of three cycles in rotation, because the stores
     // decide where the consumer finds the payload and who waits for its write-back.
-    //   fp8, 80 to 320 MiB of payload: streaming stores, ordinary loads.  224 MiB (32 x 128 tokens, hidden 7168, top-8),
+    //   fp8, 80 to 384 MiB of payload: streaming stores, ordinary loads.  224 MiB (32 x 128 tokens, hidden 7168, top-8),
     //     streamed / written through with streaming loads: the cycle with expert rows given 145 / 156 us, with the cast back
     //     in between 254 to 269 / 258 to 269, with the packed combine 119 / 121, dispatches alone 55 / 64; 112 MiB:
     //     79 / 82, 132 to 138 / 134 to 137, 65 to 68 / 62 to 69, 32 / 35.  57 MiB: 47.3 / 45.7, 73.7 / 71.6, 43.1 / 41.2,
-    //     so below that the payload is left to the cache.  Above, the cache holds less and less of it either way, while
-    //     the streamed payload's reader loses: 448 MiB 280 to 292 / 288 to 290, 512 to 535 / 517 to 528, but packed 228 to
-    //     244 / 218 to 228, and top-4 275 to 280 / 258 to 263; 336 MiB packed 178 / 171.
+    //     so below that the payload is left to the cache.  Above, the cache holds less and less of it either way, while a
+    //     streamed payload's reader loses: 336 MiB 218 / 223, 390 / 397, 178 / 171; 448 MiB, uniform, Zipf and nine tokens
+    //     in ten on an eighth of the experts, 281 to 298 / 282 to 299, 512 to 535 / 517 to 531, 228 to 244 / 218 to 231;
+    //     672 MiB 422 to 428 / 427 to 434, 778 to 790 / 775 to 788, 343 / 327 to 331.
     //     A dispatch behind unrelated memory traffic does not gain: after 512 MiB have been read 224 MiB streamed take 62
     //     to 71 us, depending on where the tensors lie, written through 60 (112 MiB 37 to 40 / 37); after 512 MiB have been
     //     written 70 to 85 / 70 (41 to 46 / 39).  The line is for callers whose dispatches and combines follow each other.
@@ -2023,7 +2024,7 @@ hipError_t launch_pack(const uint64_t* d_tbl, const RoutingScratch& sc, const Di
     //     448 MiB, packed: 258 to 263 us the cycle against 267 to 269 with ordinary loads).  bf16, 256 MiB (16 x 256 tokens,
     //     hidden 4096, top-8), plain stores / through: 98.0 / 96.6 when combine reads the payload (101.4 streamed), 186.2 /
     //     183.5 with the cast back in between, 112.3 / 111.9 with expert rows given.
-    constexpr long long kStreamFrom = 80ll << 20, kStreamBelow = 320ll << 20;
+    constexpr long long kStreamFrom = 80ll << 20, kStreamBelow = 384ll << 20;
     const long long payload = (long long)d.R * d.Tgrid * d.K * d.H;          // bytes, of an fp8 payload
     const bool stream_out = use_fp8 && payload >= kStreamFrom && payload < kStreamBelow;
     const bool stream_in = d.K > 4 || (use_fp8 && payload >= kStreamBelow);
