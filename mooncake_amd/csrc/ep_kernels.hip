@@ -2276,7 +2276,7 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
 #undef MCEP_P4
 }
 
-hipError_t launch_cast_back(const uint64_t* d_tbl, void* /*scratch: none needed*/, const float* d_factor, bool use_fp8,
+hipError_t launch_cast_back(const uint64_t* d_tbl, const float* d_factor, bool use_fp8,
                             long long max_rows, const Dims& d, hipStream_t stream) {
     const int parts = (d.H + kCastCols - 1) / kCastCols;
     const long long blocks = cast_back_chunks(max_rows, d.E) * parts;

@@ -1331,8 +1331,7 @@ int mc_ep_world_cast_back(mc_ep_world_t* w, const uint64_t* recv_x_ptrs, const u
     // valid rows of the world: at most one per selection, and no more than the layout holds
     long long max_rows = (long long)num_experts * R * max_tokens;
     if (num_topk > 0 && (long long)R * max_tokens * num_topk < max_rows) max_rows = (long long)R * max_tokens * num_topk;
-    MC_HIP(launch_cast_back(d_tbl, nullptr, (const float*)expert_factor_ptr, use_fp8, max_rows, d,
-                            stream));
+    MC_HIP(launch_cast_back(d_tbl, (const float*)expert_factor_ptr, use_fp8, max_rows, d, stream));
     return MC_EP_OK;
 }
 
