@@ -256,14 +256,13 @@ __global__ __launch_bounds__(UNIT) void count_kernel(uint64_t* __restrict__ tbl_
 // XCD's whole L2, which costs more than a launch.)
 constexpr int kPrefixWaves = 4;
 
-// The work of one wave for expert ee; pre is the wave's LDS row of U + 1 ints.
+// The work of one wave for expert ee; pre is the wave's LDS row of U + 1 ints.  64 * kAhead units at a time, their loads
+// all in flight before the first scan.
+template <int kAhead>
 __device__ __forceinline__ void prefix_expert(const uint64_t* __restrict__ tbl, const RoutingScratch& sc, int R, int E,
                                               int max_tokens, int upr, int U, int ee, int* pre) {
     const int lane = wave_lane();
     int carry = 0;
-    // 64 * kAhead units at a time, their loads all in flight before the first scan: one after another they were the
-    // kernel's time (1024 units of 64 experts: 10.6 -> 7.8 us; what is left is one line per lane and access)
-    constexpr int kAhead = 8;
     for (int u0 = 0; u0 < U; u0 += 64 * kAhead) {
         int counts[kAhead];
 #pragma unroll
@@ -313,6 +312,7 @@ __device__ __forceinline__ void prefix_expert(const uint64_t* __restrict__ tbl, 
     }
 }
 
+template <int kAhead>
 __global__ __launch_bounds__(kPrefixWaves * 64) void prefix_kernel(const uint64_t* __restrict__ tbl,
                                                                     RoutingScratch sc, int R, int E, int max_tokens,
                                                                     int upr, int U) {
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(kPrefixWaves * 64) void prefix_kernel(const uint64_
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ee = blockIdx.x * kPrefixWaves + wave;
     if (ee >= E) return;
-    prefix_expert(tbl, sc, R, E, max_tokens, upr, U, ee, lds_prefix + (size_t)wave * (U + 1));
+    prefix_expert<kAhead>(tbl, sc, R, E, max_tokens, upr, U, ee, lds_prefix + (size_t)wave * (U + 1));
 }
 
 // The packed row of one (token, k) selection, from the routing state, in two
@@ -654,7 +654,7 @@ __global__ __launch_bounds__(512) void pack_fp8_kernel(const uint64_t* __restric
         // the first E waves of the launch do the prefix pass (it needs the unit counts only)
         __shared__ int lds_pre[kMaxPackWaves * (kMaxSummedUnits + 1)];
         if (task < E) {
-            prefix_expert(tbl, sc, R, E, max_tokens, up.per_rank, up.total, task,
+            prefix_expert<1>(tbl, sc, R, E, max_tokens, up.per_rank, up.total, task,
                           lds_pre + (threadIdx.x >> 6) * (kMaxSummedUnits + 1));
             return;
         }
@@ -703,7 +703,7 @@ __global__ __launch_bounds__(512) void pack_bf16_kernel(const uint64_t* __restri
         // the first E waves of the launch do the prefix pass (it needs the unit counts only)
         __shared__ int lds_pre[kMaxPackWaves * (kMaxSummedUnits + 1)];
         if (task < E) {
-            prefix_expert(tbl, sc, R, E, max_tokens, up.per_rank, up.total, task,
+            prefix_expert<1>(tbl, sc, R, E, max_tokens, up.per_rank, up.total, task,
                           lds_pre + (threadIdx.x >> 6) * (kMaxSummedUnits + 1));
             return;
         }
@@ -1961,7 +1961,12 @@ hipError_t launch_count(const uint64_t* d_tbl, const RoutingScratch& sc, const D
     if (d.plan.carried) return hipSuccess;   // the prefix pass rides in the pack launch
     const size_t plds = (size_t)kPrefixWaves * (d.units() + 1) * sizeof(int);
     if (plds > 60 * 1024) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(prefix_kernel, dim3((d.E + kPrefixWaves - 1) / kPrefixWaves), dim3(kPrefixWaves * 64), plds,
+    // Eight pieces of the units' counts in flight where one after another they are the kernel's time; with 1024 experts and
+    // more there are waves enough to hide them, and the lines that each access touches are what bounds it.  Count and prefix
+    // launch, us, one / eight: 64 experts, 128, 256 and 1024 units 5.8 / 5.7, 6.9 / 6.2, 12.8 / 10.5; 512 experts 6.5 / 6.2,
+    // 8.1 / 7.5, 17.7 / 16.0; 1024 experts, 512 units 13.0 / 13.8; 2048, 256 14.2 / 15.1; 64 units, 256 experts 5.6 / 5.7.
+    const auto kern = d.units() > 64 && d.E < 1024 ? prefix_kernel<8> : prefix_kernel<1>;
+    hipLaunchKernelGGL(kern, dim3((d.E + kPrefixWaves - 1) / kPrefixWaves), dim3(kPrefixWaves * 64), plds,
                        stream, d_tbl, sc, d.R, d.E, d.max_tokens, d.units_per_rank(), d.units());
     return hipGetLastError();
 }

@@ -22,6 +22,13 @@ def test_prefix_over_many_units(gpu_device, oracle, units):
     check(oracle, EPConfig("units", 1, units * 32 - 3, 128, 8, 8, False))
 
 
+@pytest.mark.parametrize("units,experts", [(64, 1023), (65, 1023), (65, 1024), (130, 1024)])
+def test_prefix_pass_by_units_and_experts(gpu_device, oracle, units, experts):
+    """Both sides of the line between one and eight pieces of the counts in flight."""
+    announce(f"prefix pass over {units} units of {experts} experts")
+    check(oracle, EPConfig("units", 1, units * 64 - 3, 128, experts, 4, False), routing_sum=0)
+
+
 @pytest.mark.parametrize("groups", [15, 16, 17, 20, 32, 36])
 def test_scale_transposition_parts(gpu_device, oracle, groups):
     announce(f"scale transposition of {groups} groups")
