@@ -171,6 +171,15 @@ static ArgTable<N> arg_table(const uint64_t* words, int n) {
     return t;
 }
 
+// The first block of a kernel that got its table in the arguments puts it into memory for the calls after this one (not
+// when a recorded call runs: null).  Read from there it costs less: arguments lie in host memory, 0.5 us of a combine of
+// 3.4.
+template <int N>
+__device__ __forceinline__ void leave_table(uint64_t* tbl_mem, const ArgTable<N>& arg_tbl, int words) {
+    if (N > 0 && tbl_mem != nullptr && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < words; i += blockDim.x) tbl_mem[i] = arg_tbl.v[i];
+}
+
 // Clears `words` 32-bit words at each of n addresses carried in kernel
 // arguments: one launch where a per-rank hipMemsetAsync would be n launches.
 __global__ void clear_words_kernel(TableChunk chunk, int n, int words) {
@@ -1162,11 +1171,12 @@ __global__ __launch_bounds__(256) void dispatch_alone_kernel(ArgTable<(int)DF_CO
 // row's address and weight there.  Experts on ranks the owner sees as
 // inactive, and rows of ranks that take no part, leave no route.
 template <bool PACKED, int TW>
-__global__ __launch_bounds__(256) void resolve_kernel(const uint64_t* __restrict__ tbl_mem,
+__global__ __launch_bounds__(256) void resolve_kernel(uint64_t* __restrict__ tbl_mem,
                                                        CombineRoute* __restrict__ routes, uint32_t stamp, int R,
                                                        int E, int K, int H, int max_tokens, int total_tasks,
                                                        ArgTable<TW> arg_tbl) {
     const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
+    leave_table(tbl_mem, arg_tbl, (int)CF_COUNT * R);
     const int lane = wave_lane();
     const int task = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     if (task >= total_tasks) return;
@@ -1330,13 +1340,14 @@ __device__ __forceinline__ DirectRow search_row(const uint64_t* __restrict__ tbl
 //   FROM     where the rows are looked up
 //   TW       words of the rank table in the arguments; 0: in memory, or not needed (every tensor evenly spaced).
 template <int KMAX, int CH, bool NTL, bool NTS, int FROM, int TW>
-__global__ __launch_bounds__(512) void reduce_kernel(const uint64_t* __restrict__ tbl_mem,
+__global__ __launch_bounds__(512) void reduce_kernel(uint64_t* __restrict__ tbl_mem,
                                                       const CombineRoute* __restrict__ routes, uint32_t stamp,
                                                       RoutingScratch sc, CombineSource cs,
                                                       const void* __restrict__ zero_row, int R, int E, int K,
                                                       int max_tokens, int H, int slabs, int Tgrid,
                                                       int total_tasks, ArgTable<TW> arg_tbl) {
     const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
+    leave_table(tbl_mem, arg_tbl, (int)CF_COUNT * R);
     const int lane = wave_lane();
     const int task = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     if (task >= total_tasks) return;
@@ -1474,7 +1485,7 @@ __device__ __forceinline__ uint32_t scale_round_twice(float a, float b, float s,
 //   CH  bf16 payloads only: 16-byte chunks per lane and row, 512 elements apart (two when there are few
 //       rows per token, as in reduce_kernel: half as many waves, each with as many loads in flight)
 template <int KMAX, bool FP8, bool FACTOR, int FROM, int CH, int TW>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ? 8 : 4, 8))) void reduce_packed_kernel(const uint64_t* __restrict__ tbl_mem,
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ? 8 : 4, 8))) void reduce_packed_kernel(uint64_t* __restrict__ tbl_mem,
                                                              const CombineRoute* __restrict__ routes, uint32_t stamp,
                                                              RoutingScratch sc, CombineSource cs,
                                                              const void* __restrict__ zero_row,
@@ -1482,6 +1493,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
                                                              int max_tokens, int H, int slabs, int Tgrid,
                                                              int group_blocks, ArgTable<TW> arg_tbl) {
     const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
+    leave_table(tbl_mem, arg_tbl, (int)CF_COUNT * R);
     static_assert(!FP8 || CH == 1, "an fp8 payload is one 16-byte chunk of 16 elements per lane");
     constexpr int kSlab = FP8 ? 1024 : 512 * CH;
     constexpr int kChunkElems = FP8 ? 16 : 8;          // elements in a lane's 16-byte chunk
@@ -2134,7 +2146,8 @@ hipError_t launch_resolve(const uint64_t* d_tbl, CombineRoute* d_routes, uint32_
     const int words = (int)CF_COUNT * d.R;
     if (d.host_table != nullptr && words > kArgTableWords) return hipErrorInvalidValue;
 #define MCEP_RESOLVE(PACKED, TW)                                                                                   \
-    hipLaunchKernelGGL((resolve_kernel<PACKED, TW>), dim3(blocks), dim3(wpb * 64), 0, stream, d_tbl, d_routes, stamp, \
+    hipLaunchKernelGGL((resolve_kernel<PACKED, TW>), dim3(blocks), dim3(wpb * 64), 0, stream,       \
+                       const_cast<uint64_t*>(d_tbl), d_routes, stamp,                                                \
                        d.R, d.E, d.K, d.H, d.max_tokens, (int)total, arg_table<TW>(d.host_table, words))
     if (packed && d.host_table != nullptr) MCEP_RESOLVE(true, kArgTableWords);
     else if (packed) MCEP_RESOLVE(true, 0);
@@ -2179,7 +2192,8 @@ static hipError_t launch_reduce_t(const ReduceLaunch& rl, const Dims& d, const T
     if ((in_args && words > kArgTableWords) || ((in_args || FROM == kFromHandle) && !(ntl && nts))) return hipErrorInvalidValue;
 #define MCEP_REDUCE(A, B, TW)                                                                                    \
     hipLaunchKernelGGL((reduce_kernel<KMAX, CH, A, B, FROM, TW>), dim3(blocks), dim3(wpb * 64), pad, stream,   \
-                       rl.d_tbl, rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row, d.R, d.E, d.K,             \
+                       const_cast<uint64_t*>(rl.d_tbl), rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row,     \
+                       d.R, d.E, d.K,                                                                            \
                        d.max_tokens, d.H, slabs, d.Tgrid, (int)total, arg_table<TW>(d.host_table, words))
     if (in_args) MCEP_REDUCE(true, true, kArgTableWords);
     else if (ntl && nts) MCEP_REDUCE(true, true, 0);
@@ -2241,7 +2255,8 @@ static hipError_t launch_reduce_packed_t(const ReduceLaunch& rl, const float* d_
     if (in_args && words > kArgTableWords) return hipErrorInvalidValue;
 #define MCEP_PACKED(TW)                                                                                             \
     hipLaunchKernelGGL((reduce_packed_kernel<KMAX, FP8, FACTOR, FROM, CH, TW>), dim3((unsigned)blocks),           \
-                       dim3(wpb * 64), 0, stream, rl.d_tbl, rl.d_routes, rl.stamp, rl.sc, rl.src, rl.d_zero_row,    \
+                       dim3(wpb * 64), 0, stream, const_cast<uint64_t*>(rl.d_tbl), rl.d_routes, rl.stamp, rl.sc,    \
+                       rl.src, rl.d_zero_row,                                                                       \
                        d_factor, d.R, d.E, d.K, d.max_tokens, d.H, slabs, d.Tgrid, group_blocks,                    \
                        arg_table<TW>(d.host_table, words))
     if (in_args) MCEP_PACKED(kArgTableWords);

@@ -790,32 +790,39 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
         src.src_info = uniform_ptr(src_info, R, uni);
         src.layout_range = uniform_ptr(layout_range, R, uni);
     }
-    // The rank table: not needed when every tensor is evenly spaced, else in the kernels' arguments (a recorded call
-    // then carries its own), in memory only for worlds too large for that and for the streaming hints that have no
-    // such variant.
+    // The rank table: not needed when every tensor is evenly spaced; in memory when it is that of the last call that
+    // needed one; else in the kernels' arguments, and from there into memory (a recorded call carries its own and leaves
+    // the shared one alone).  Worlds too large for that, and the streaming hints that have no such variant, have it written
+    // by a launch of its own.
+    const bool resolves = !direct && !src.search && (phases & MC_EP_PHASE_LAYOUT);
+    const bool reads = (phases & MC_EP_PHASE_DATA) && combine_reads_table(src, direct);
     const uint64_t* d_tbl = nullptr;
-    if (!direct || combine_reads_table(src, direct)) {
-        if ((int)tbl.size() <= kArgTableWords && (ps.packed || (w->tuning.combine_nt & 3) == 3)) {
-            d.host_table = tbl.data();
-        } else if (int rc = upload_table(w, 1, tbl, cap, stream, &d_tbl)) {
-            return rc;
+    bool leaves = false;
+    if (!cap.active && (resolves || reads) && w->tbl_cache[1] == tbl) {
+        d_tbl = w->d_tbl[1];
+    } else if ((resolves || reads) && (int)tbl.size() <= kArgTableWords && (ps.packed || (w->tuning.combine_nt & 3) == 3)) {
+        d.host_table = tbl.data();
+        if (!cap.active) {
+            d_tbl = w->d_tbl[1];
+            leaves = true;
+            w->tbl_cache[1].clear();                      // until the launches have succeeded
         }
+    } else if (resolves || reads) {
+        if (int rc = upload_table(w, 1, tbl, cap, stream, &d_tbl)) return rc;
     }
     // sized on every path, so that an eager call prepares the world for any recorded one of the same shape
     if (int rc = ensure_routes(w, (size_t)R * max_tokens * num_topk)) return rc;
-    if (!direct && !src.search) {
-        if (phases & MC_EP_PHASE_LAYOUT) {
-            w->stamp += 1;
-            // every replay of a recorded call carries the same stamp: clear the routes so that none of an
-            // earlier replay passes for this one's
-            if (cap.active) {
-                MC_HIP(launch_fill_u32(w->d_routes, 0u, (size_t)R * max_tokens * num_topk * (sizeof(CombineRoute) / 4),
-                                       stream));
-                w->launches += 1;
-            }
-            MC_HIP(launch_resolve(d_tbl, w->d_routes, w->stamp, ps.packed, d, w->tuning, stream));
+    if (resolves) {
+        w->stamp += 1;
+        // every replay of a recorded call carries the same stamp: clear the routes so that none of an
+        // earlier replay passes for this one's
+        if (cap.active) {
+            MC_HIP(launch_fill_u32(w->d_routes, 0u, (size_t)R * max_tokens * num_topk * (sizeof(CombineRoute) / 4),
+                                   stream));
             w->launches += 1;
         }
+        MC_HIP(launch_resolve(d_tbl, w->d_routes, w->stamp, ps.packed, d, w->tuning, stream));
+        w->launches += 1;
     }
     if (phases & MC_EP_PHASE_DATA) w->launches += 1;
     if ((phases & MC_EP_PHASE_DATA) && ps.packed)
@@ -824,6 +831,7 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     else if (phases & MC_EP_PHASE_DATA)
         MC_HIP(launch_reduce(d_tbl, w->d_routes, w->stamp, routing_scratch(w), direct, src, w->d_zero_row, d,
                              w->tuning, stream));
+    if (leaves) w->tbl_cache[1] = tbl;
     return MC_EP_OK;
 }
 

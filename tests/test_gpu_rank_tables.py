@@ -64,3 +64,47 @@ def test_calls_take_turns_on_one_world(gpu_device, oracle, ranks, ragged, unifor
             assert torch.equal(b.combined[r, :n].view(torch.int16), want[r, :n].view(torch.int16))
         b.expert_out.normal_(generator=torch.Generator(device="cuda").manual_seed(2))
         b.combined.copy_(plain)
+
+
+@pytest.mark.parametrize("search", [256, 0], ids=["searched", "resolved"])
+@pytest.mark.parametrize("ranks", [3, 33])
+def test_a_table_left_in_memory_is_the_next_call_s(gpu_device, oracle, ranks, search):
+    """The same combine again finds its table in memory; a recorded one neither uses nor disturbs it."""
+    cfg = EPConfig("left", ranks, 8, 256, 2 * ranks, 2, True)
+    nt = [(r * 5) % 8 + 1 for r in range(ranks)]                # (uneven counts: the kernels read the table)
+    announce(f"rank table left in memory ranks={ranks} search={search}")
+    world = ep.World(ranks)
+    world.set_option("combine_search_tokens", search)
+    a, b = _harness(cfg, world, 3, nt), _harness(cfg, world, 4, nt)
+    factor = torch.rand(cfg.num_experts, device="cuda") + 0.5
+    for h in (a, b):
+        h.dispatch()
+        h.combine()
+        h.combine_packed(factor)
+    a.dispatch()
+    a.combine()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    recorded = torch.empty_like(b.combined)
+    with torch.cuda.graph(graph):
+        b.combine()
+        recorded.copy_(b.combined)
+    for turn in range(3):
+        for h in (a, a, b, b, a):
+            h.combined.fill_(7.0)
+            h.combine()
+            torch.cuda.synchronize()
+            _check(h, oracle, h.combined.cpu())
+            if turn:
+                recorded.fill_(7.0)
+                graph.replay()
+                torch.cuda.synchronize()
+                _check(b, oracle, recorded.cpu())
+            rows = h.expert_out.clone()
+            h.cast_back(factor)
+            h.combine()
+            want = h.combined.clone()
+            h.combine_packed(factor)
+            torch.cuda.synchronize()
+            assert torch.equal(h.combined.view(torch.int16), want.view(torch.int16))
+            h.expert_out.copy_(rows)
