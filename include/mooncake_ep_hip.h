@@ -96,8 +96,8 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * "packed_map": tuning knobs
  * for measurement sweeps; "combine_search_tokens" (default 256): a combine of a
  * handle that is not the last dispatch's is one launch while no rank combines
- * more tokens than this - three quarters of it from top-5 to top-7,
- * three eighths from top-9 on -, two beyond (0: always two); "fused_small": 1 (default) dispatches a
+ * more tokens than this - three eighths of it from top-5 to top-7,
+ * five at top-8, two from top-9 on -, two beyond (0: always two); "fused_small": 1 (default) dispatches a
  * small world in one kernel launch - at most "fused_small_max" (default 4096)
  * selections, and few rounds of 512 index-list entries: up to 8 ranks whose
  * lists make at most "fused_small_rounds" rounds, each list counted by itself

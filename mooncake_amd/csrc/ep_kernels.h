@@ -131,14 +131,16 @@ struct DispatchSource {
 };
 
 struct CombineSource {
+    // (read by every reduce kernel, in one piece: with `active` behind the scales, and so loaded by itself, combines of 550
+    // to 650 blocks took 0.15 us more, 5.1 against 5.0 for 2 x 1144 tokens of hidden 896, top-1)
     RankPtr topk_idx, topk_weights, out;
     RankPtr x;              // the rows combine reads (expert outputs, or the packed payload)
-    RankPtr scales;         // packed combine of an fp8 payload
     RankPtr active;
-    RankPtr src_info, layout_range;   // the handle, when the reduce kernels look rows up in it
+    int tokens = -1;
     bool packed_fp8 = false;   // `scales` is read
     bool search = false;       // rows are looked up in the handle (not: in the last dispatch's state, or in routes)
-    int tokens = -1;
+    RankPtr scales;         // packed combine of an fp8 payload
+    RankPtr src_info, layout_range;   // the handle, when the reduce kernels look rows up in it
 };
 
 struct Dims {
@@ -164,8 +166,8 @@ struct Tuning {
                                // 1 = the reference kernel's own (see pack_fp8_kernel)
     int combine_direct = 1;    // reuse the last dispatch's routing state when combine gets that dispatch's handle
     int combine_search_tokens = 256;   // any other handle is searched by the reduce kernel itself while no rank combines
-                               // more tokens than this (top-5 to top-7: three quarters of it, from top-9 on: three
-                               // eighths); beyond, a resolve launch turns it into routes
+                               // more tokens than this (top-5 to top-7: three eighths of it, top-8: five, from top-9 on:
+                               // two); beyond, a resolve launch turns it into routes
     int combine_chunks = 0;    // 16-byte chunks per lane in the combine kernel (1 or 2); 0: by top-k
     int combine_waves = 4;     // waves per block in the combine kernel
     int combine_nt = 3;        // bit 0: streaming loads, bit 1: streaming stores

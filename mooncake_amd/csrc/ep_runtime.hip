@@ -773,16 +773,15 @@ int world_combine_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_i
     // A handle that is not the last dispatch's: every wave of the reduce kernel looks its token's rows up in it, or a
     // resolve launch turns it into routes first.  A look-up scans the rows that the expert got from the token's rank: at
     // most this many when the handle is that of the tokens combined now and no token names an expert twice (more scan
-    // longer, with the same result), and whatever the routing.  Whole cycles, resolved / searched: 32 x 64 tokens, hidden
-    // 7168, top-8, fp8, rows given 86.8 / 81.1 us (81.4 when the last dispatch's state is there), Zipf(1.2) routing 84.2 /
-    // 79.1; 32 x 128 150.7 / 144.4 and 150.7 / 146.4; 16 x 256, hidden 4096, bf16 101.4 / 95.7 and 106.9 / 104.3; 8 x 256,
-    // 7168, Zipf 88.0 / 85.6, where the hottest experts' 256 rows of a rank are what the lead shrinks by.
-    // From top-9 on a selection has half the lanes of top-8's to scan with, and from top-5 to top-7 top-8's with fewer
-    // payload rows to hide the scan behind.  Combines alone, us, resolved / searched, nine tokens in ten on an eighth of 64
-    // experts: top-9, 16 ranks of 96, 128 and 256 tokens, hidden 4096, 28.8 / 27.3, 35.5 / 36.2, 62.8 / 80.1; top-11, 8 of
-    // 256, hidden 7168, 67.1 / 78.5; top-8, 8 of 256, 53.7 / 52.4; Zipf, 8 of 256, top-5 37.4 / 39.2 (192: 29.1 / 29.6),
-    // top-7 47.3 / 48.6 (192: 36.9 / 35.4).
-    const int eighths = num_topk > 8 ? 3 : (num_topk >= 5 && num_topk <= 7 ? 6 : 8);
+    // longer, with the same result), and whatever the routing.  The more selections a token has, the fewer lanes each has
+    // to scan with (top-9 and up four, top-5 to top-8 eight), and the more payload rows there are to hide the scan behind;
+    // from top-7 on the resolved combine also runs at the occupancy that suits it better.  Combines alone of the same
+    // tensors, us, resolved / searched, the slowest of 36 worlds (16 and 32 ranks, Zipf and incast routing) at the line and
+    // at 256 tokens: top-2 31.1 / 32.5 at 256 (the median world 14 % faster); top-5, 96 tokens 25.0 / 25.4, 256 42.0 / 51.7;
+    // top-7 32.0 / 31.5, 51.8 / 59.2; top-8, 160 tokens 55.1 / 55.5, 256 75.0 / 83.0; top-9, 64 tokens 27.4 / 27.8, 256
+    // 69.6 / 105.3; top-16 44.5 / 44.1, 169 / 209.  Whole cycles with tensors of their own each time: 32 x 64 tokens, hidden
+    // 7168, top-8, fp8, rows given 86.8 / 81.1 us, Zipf 84.2 / 79.1; 32 x 128 150.7 / 144.4 and 150.7 / 146.4.
+    const int eighths = num_topk <= 4 ? 8 : (num_topk < 8 ? 3 : (num_topk == 8 ? 5 : 2));
     const int search_tokens = (int)((long long)w->tuning.combine_search_tokens * eighths / 8);
     src.search = !direct && phases == MC_EP_PHASE_ALL && tgrid <= search_tokens &&
                  (ps.packed || (w->tuning.combine_nt & 3) == 3);

@@ -82,7 +82,8 @@ def test_the_search_rule(gpu_device):
 
 def test_the_search_rule_by_top_k(gpu_device):
     announce("combine: the rule for searched handles, by selections a token")
-    for K, T, one in ((4, 256, True), (5, 192, True), (5, 193, False), (7, 193, False), (8, 193, True), (9, 96, True), (9, 97, False), (16, 96, True), (16, 97, False)):
+    for K, T, one in ((4, 256, True), (5, 96, True), (5, 97, False), (7, 97, False), (8, 160, True), (8, 161, False),
+                      (9, 64, True), (9, 65, False), (16, 64, True), (16, 65, False)):
         cfg = EPConfig("rule", 2, T, 128, 16, K, False)
         h = run_dispatch(cfg, generate(cfg, seed=73), poison=False, options={"combine_direct": 0})
         h.alloc_combine_io()
