@@ -27,6 +27,16 @@ def gpu_device():
     return torch.device("cuda:0")
 
 
+@pytest.fixture(params=[256, 0], ids=["searched", "resolved"])
+def search_tokens(request):
+    """Runs a test once per way that a combine finds its rows in a handle: the reduce kernels search it (256), or a
+    resolve launch turns it into routes first (0)."""
+    from tests import gpu_util
+    gpu_util.DEFAULT_OPTIONS["combine_search_tokens"] = request.param
+    yield request.param
+    gpu_util.DEFAULT_OPTIONS.pop("combine_search_tokens", None)
+
+
 @pytest.fixture(params=[1, 0], ids=["one_launch", "three_launch"])
 def fused_small(request):
     """Runs a test once per dispatch path: worlds small enough for the one-launch dispatch take it (1), or

@@ -55,14 +55,16 @@ def oracle_two_step(oracle, cfg, data, nt, factor, active=None):
 @pytest.mark.parametrize("cfg", CASES, ids=[c.name for c in CASES])
 @pytest.mark.parametrize("is_ragged", [False, True], ids=["full", "ragged"])
 @pytest.mark.parametrize("with_factor", [True, False], ids=["factor", "nofactor"])
-@pytest.mark.parametrize("direct,packed_map", [(1, 1), (0, 1), (1, 0)], ids=["direct", "handle", "direct_rank_groups"])
+@pytest.mark.parametrize("direct,packed_map", [(1, 1), (0, 1), (1, 0), (-1, 1)],
+                         ids=["direct", "handle", "direct_rank_groups", "resolved"])
 def test_packed_combine_matches_oracle(gpu_device, oracle, cfg, is_ragged, with_factor, direct, packed_map):
     """packed_map: how the kernel's blocks are dealt to the XCDs (slabs owned by XCDs, or (rank, slab) groups)."""
     nt = ragged(cfg, is_ragged)
     announce(f"packed combine {cfg} ragged={nt} factor={with_factor} direct={direct} packed_map={packed_map}")
     data = generate(cfg, seed=21)
     h = run_dispatch(cfg, data, num_tokens=nt, poison=True,
-                     options={"combine_direct": direct, "packed_map": packed_map})
+                     options={"combine_direct": max(direct, 0), "packed_map": packed_map,
+                              "combine_search_tokens": 0 if direct < 0 else 256})
     factor = (torch.arange(cfg.num_experts).float() * 0.1 + 1.0) if with_factor else None
     h.alloc_combine_io()
     h.combined.fill_(7.0)
@@ -83,7 +85,7 @@ def test_packed_combine_matches_oracle(gpu_device, oracle, cfg, is_ragged, with_
 
 @pytest.mark.parametrize("chunks", [1, 2])
 @pytest.mark.parametrize("direct", [1, 0], ids=["direct", "handle"])
-def test_packed_combine_bf16_chunks_per_lane(gpu_device, oracle, chunks, direct):
+def test_packed_combine_bf16_chunks_per_lane(gpu_device, oracle, chunks, direct, search_tokens):
     """One or two 16-byte chunks per lane (option combine_chunks; by default two up to top-4) are the same function."""
     cfg = EPConfig("chunks_bf16", 4, 28, 2560, 16, 3, False, masked_fraction=0.2)
     announce(f"packed combine of a bf16 payload, combine_chunks={chunks} direct={direct}")
@@ -98,7 +100,7 @@ def test_packed_combine_bf16_chunks_per_lane(gpu_device, oracle, chunks, direct)
 
 
 @pytest.mark.parametrize("direct", [1, 0], ids=["direct", "handle"])
-def test_packed_combine_skips_inactive_ranks(gpu_device, oracle, direct):
+def test_packed_combine_skips_inactive_ranks(gpu_device, oracle, direct, search_tokens):
     cfg = EPConfig("inactive_packed", 4, 16, 1024, 16, 4, True)
     announce(f"packed combine with inactive ranks direct={direct}")
     data = generate(cfg, seed=22)

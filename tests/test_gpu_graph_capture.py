@@ -39,11 +39,13 @@ def _harness(cfg, world, seed):
 
 
 @pytest.mark.parametrize("use_fp8", [True, False])
-@pytest.mark.parametrize("one_graph", [True, False])
-def test_replays_match_the_oracle(gpu_device, oracle, use_fp8, one_graph):
+@pytest.mark.parametrize("one_graph,search", [(True, 256), (False, 256), (False, 0)],
+                         ids=["one_graph", "searched", "resolved"])
+def test_replays_match_the_oracle(gpu_device, oracle, use_fp8, one_graph, search):
     cfg = EPConfig("graph", 4, 48, 1024, 16, 4, use_fp8, masked_fraction=0.2)
-    announce(f"graph capture {cfg} one_graph={one_graph}")
+    announce(f"graph capture {cfg} one_graph={one_graph} search={search}")
     world = ep.World(cfg.num_ranks)
+    world.set_option("combine_search_tokens", search)
     h = _harness(cfg, world, seed=100)
     other = _harness(cfg, world, seed=200)          # eager traffic on the same world
     factor = (torch.arange(cfg.num_experts, dtype=torch.float32) * 0.1 + 1.0).to(gpu_device)
@@ -65,12 +67,14 @@ def test_replays_match_the_oracle(gpu_device, oracle, use_fp8, one_graph):
             h.cast_back(factor)
             h.combine()
         graphs = [g]
-    else:                                           # a combine recorded on its own resolves its handle
+    else:                                           # a combine recorded on its own looks its handle up
         for part in (lambda: (h.dispatch(), h.cast_back(factor)), h.combine):
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g):
                 part()
             graphs.append(g)
+        # in the reduce kernel, or through routes: cleared, resolved, read
+        assert world.get_option("last_combine_launches") == (1 if search else 3)
 
     for seed in (1, 2, 3):
         data = generate(cfg, seed=seed)

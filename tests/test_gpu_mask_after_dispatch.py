@@ -27,8 +27,8 @@ def mask_some(idx: torch.Tensor, fraction: float, seed: int) -> torch.Tensor:
 
 @pytest.mark.parametrize("cfg", CASES, ids=[c.name for c in CASES])
 @pytest.mark.parametrize("direct", [1, 0], ids=["direct", "handle"])
-def test_world_combine_after_masking_in_place(gpu_device, oracle, cfg, direct):
-    announce(f"mask 20 % of topk_idx between dispatch and combine {cfg} direct={direct}")
+def test_world_combine_after_masking_in_place(gpu_device, oracle, cfg, direct, search_tokens):
+    announce(f"mask 20 % of topk_idx between dispatch and combine {cfg} direct={direct} search={search_tokens}")
     data = generate(cfg, seed=31)
     h = run_dispatch(cfg, data, poison=False, options={"combine_direct": direct})
     nt = h.num_tokens
@@ -52,6 +52,7 @@ def test_world_combine_after_masking_in_place(gpu_device, oracle, cfg, direct):
     h.combined.fill_(7.0)
     h.combine()
     torch.cuda.synchronize()
+    assert h.world.get_option("last_combine_launches") == (1 if direct or search_tokens else 2)
     assert torch.equal(h.combined.cpu().view(torch.int16), want.view(torch.int16)), "combine"
     h.combined.fill_(7.0)
     h.combine_packed(factor)
@@ -60,11 +61,11 @@ def test_world_combine_after_masking_in_place(gpu_device, oracle, cfg, direct):
 
 
 @pytest.mark.parametrize("direct", [1, 0], ids=["direct", "handle"])
-def test_a_selection_pointed_at_another_expert_has_no_row(gpu_device, oracle, direct):
+def test_a_selection_pointed_at_another_expert_has_no_row(gpu_device, oracle, direct, search_tokens):
     """Out of contract in the reference (it would read a slot nobody wrote); here such a selection contributes
     nothing on either path - the handle holds no row of that token for the new expert."""
     cfg = EPConfig("repoint", 4, 32, 1024, 32, 4, False)
-    announce(f"re-pointed selections direct={direct}")
+    announce(f"re-pointed selections direct={direct} search={search_tokens}")
     data = generate(cfg, seed=32)
     h = run_dispatch(cfg, data, poison=False, options={"combine_direct": direct})
     nt = h.num_tokens
@@ -87,11 +88,12 @@ def test_a_selection_pointed_at_another_expert_has_no_row(gpu_device, oracle, di
 
 @pytest.mark.parametrize("direct", [1, 0], ids=["direct", "handle"])
 @pytest.mark.parametrize("use_fp8", [False, True], ids=["bf16", "fp8"])
-def test_buffer_combine_after_masking_in_place(gpu_device, oracle, direct, use_fp8):
+def test_buffer_combine_after_masking_in_place(gpu_device, oracle, direct, use_fp8, search_tokens):
     R, T, H, E, K = 4, 40, 2048, 32, 6
     announce(f"per-rank Buffer: mask topk_idx in place before combine direct={direct} fp8={use_fp8}")
     world, groups = LogicalGroup.make_world(R)
     world.set_option("combine_direct", direct)
+    world.set_option("combine_search_tokens", search_tokens)
     nbytes = Buffer.get_ep_buffer_size_hint(T, H, R, E)
     bufs = [Buffer(g, nbytes) for g in groups]
     cfg = EPConfig("buffer_mask", R, T, H, E, K, use_fp8)

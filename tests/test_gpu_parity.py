@@ -187,15 +187,17 @@ COMBINE_CASES = [
 
 @pytest.mark.parametrize("cfg", COMBINE_CASES, ids=[c.name for c in COMBINE_CASES])
 @pytest.mark.parametrize("is_ragged", [False, True], ids=["full", "ragged"])
-@pytest.mark.parametrize("chunks,cnt,direct", [(1, 3, 1), (2, 3, 1), (1, 0, 1), (1, 3, 0), (2, 0, 0)])
+@pytest.mark.parametrize("chunks,cnt,direct", [(1, 3, 1), (2, 3, 1), (1, 0, 1), (1, 3, 0), (2, 0, 0), (1, 3, -1), (2, 3, -1)])
 def test_combine_matches_oracle(gpu_device, oracle, cfg, is_ragged, chunks, cnt, direct, fused_small):
     """direct=1: the handle is the last dispatch's, rows come from its routing
-    state; direct=0: the general path that re-derives rows from the handle."""
+    state; direct=0: the general path that re-derives rows from the handle (the reduce kernel searches it, up to 256
+    tokens and with streaming hints); direct=-1: a resolve launch turns the handle into routes first."""
     nt = ragged(cfg, is_ragged)
     announce(f"combine {cfg} ragged={nt} chunks={chunks} nt={cnt} direct={direct} fused_small={fused_small}")
     data = generate(cfg, seed=3)
     h = run_dispatch(cfg, data, num_tokens=nt, poison=False,
-                     options={"combine_chunks": chunks, "combine_nt": cnt, "combine_direct": direct})
+                     options={"combine_chunks": chunks, "combine_nt": cnt, "combine_direct": max(direct, 0),
+                              "combine_search_tokens": 0 if direct < 0 else 256})
     factor = torch.arange(cfg.num_experts).float() * 0.1 + 1.0
     h.alloc_combine_io()
     h.expert_out.fill_(float("nan"))                       # rows outside the handle must never be read
@@ -240,7 +242,7 @@ def test_combine_launch_shapes_match_oracle(gpu_device, oracle, waves, occupancy
 
 
 @pytest.mark.parametrize("direct", [1, 0])
-def test_combine_skips_inactive_ranks(gpu_device, oracle, direct, fused_small):
+def test_combine_skips_inactive_ranks(gpu_device, oracle, direct, fused_small, search_tokens):
     cfg = EPConfig("inactive", 4, 16, 1024, 16, 4, False)
     announce(f"combine with an inactive rank direct={direct}")
     data = generate(cfg, seed=4)
@@ -299,7 +301,7 @@ def test_dispatch_with_silent_rank(gpu_device, oracle, fused_small):
 
 
 @pytest.mark.parametrize("direct", [1, 0])
-def test_ids_outside_the_expert_range_name_no_expert(gpu_device, oracle, direct, fused_small):
+def test_ids_outside_the_expert_range_name_no_expert(gpu_device, oracle, direct, fused_small, search_tokens):
     """The reference asserts nothing about top-k ids; here anything outside [0, E) is treated like -1 by every
     kernel (and by the oracle), instead of indexing out of bounds."""
     cfg = EPConfig("stray_ids", 4, 24, 512, 8, 4, True)

@@ -39,18 +39,21 @@ def _case(seed: int):
         active[rng.randrange(R), rng.randrange(R)] = 0
     direct = rng.choice([0, 1])
     summed = rng.choice([0, 1])      # both routing plans (prefix pass as its own launch, or inside pack)
-    return cfg, num_tokens, present, active, direct, summed
+    search = rng.choice([0, 256])    # a handle looked up by a resolve launch, or by the reduce kernels
+    return cfg, num_tokens, present, active, direct, summed, search
 
 
 # more seeds for a longer sweep: MC_EP_RANDOM_WORLDS=300 python -m pytest tests/test_gpu_random_shapes.py -m gpu
 @pytest.mark.parametrize("seed", range(int(os.environ.get("MC_EP_RANDOM_WORLDS", "32"))))
 def test_random_world(gpu_device, oracle, seed):
-    cfg, num_tokens, present, active, direct, summed = _case(seed)
-    announce(f"random world seed={seed} {cfg} tokens={num_tokens} present={present} direct={direct} summed={summed}")
+    cfg, num_tokens, present, active, direct, summed, search = _case(seed)
+    announce(f"random world seed={seed} {cfg} tokens={num_tokens} present={present} direct={direct} summed={summed} "
+             f"search={search}")
     data = generate(cfg, seed=1000 + seed)
     h = WorldHarness(cfg, num_tokens=num_tokens)
     h.world.set_option("combine_direct", direct)
     h.world.set_option("routing_sum", summed)
+    h.world.set_option("combine_search_tokens", search)
     h.load(data)
     h.alloc_dispatch_outputs(poison=True)
     h.alloc_combine_io()

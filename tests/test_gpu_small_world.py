@@ -1,9 +1,9 @@
-"""The one-launch dispatch of small worlds (`dispatch_small_kernel`: at most 8 ranks and, by default, 4096
-selections; every wave rebuilds the routing it needs from the ranks' index lists) against the CPU oracle, bit
-for bit, and against the library's own count / pack / scale-transpose path: shapes at the edges of what it
-takes (list lengths around the 128- and 512-entry steps of its counting loop, odd list lengths, the most ranks
-and selections it accepts, every top-k bracket), ragged and silent ranks, a rank that receives nothing,
-repeated experts, stray ids, index lists at either alignment, and the shapes it must leave to the other path."""
+"""The one-launch dispatch of small worlds (up to 32 ranks and, by default, 4096 selections; every block, or every wave,
+rebuilds the routing it needs from the ranks' index lists) against the CPU oracle, bit for bit, and against the
+library's own count / pack / scale-transpose path: shapes at the edges of what it takes (list lengths around the
+512-entry rounds of its counting, odd list lengths, the most selections it accepts, every top-k bracket), ragged and
+silent ranks, a rank that receives nothing, repeated experts, stray ids, index lists at either alignment, and the shapes
+it must leave to the other path."""
 import pytest
 import torch
 
