@@ -42,8 +42,9 @@ def kernel_sources_sha256(root: str = ROOT) -> str:
 # kernel-name fragments -> the short names bench.py uses
 KERNELS = [("copy_kernel", "copy"), ("count_kernel", "count"), ("prefix_kernel", "prefix"), ("pack_fp8_kernel", "pack"),
            ("pack_bf16_kernel", "pack"), ("scale_transpose_kernel", "scales"), ("resolve_kernel", "resolve"),
-           ("reduce_packed_kernel", "reduce_packed"), ("reduce_kernel", "reduce"), ("cast_back_kernel", "cast_back"),
-           ("dispatch_small_kernel", "dispatch_small")]
+           ("reduce_packed_kernel", "reduce_packed"), ("reduce_kernel", "reduce"), ("cast_chunks_kernel", "cast_chunks"),
+           ("cast_back_kernel", "cast_back"), ("dispatch_small_kernel", "dispatch_small"),
+           ("dispatch_alone_kernel", "dispatch_small")]
 
 
 def per_kernel_kib(directory: str) -> Dict[str, List[float]]:

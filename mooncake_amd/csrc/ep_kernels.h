@@ -226,7 +226,11 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
 // packed rows below packed_recv_count -> bf16 rows times factor[expert]; max_rows bounds the world's valid rows
 constexpr int kCastRows = 16;         // packed rows of one expert per work item of the cast-back kernel
 long long cast_back_chunks(long long max_rows, int num_experts);
-hipError_t launch_cast_back(const uint64_t* d_tbl, const float* d_factor, bool use_fp8,
+constexpr int kCastWaves = 4;         // waves per block of the kernel
+constexpr int kCastCols = 1024;       // columns of a row per block
+// whether the blocks' chunks come from a work list; d_chunk_map then holds 16 bytes x (cast_back_chunks(max_rows, E) + 1)
+bool cast_back_listed(long long max_rows, int num_experts, int hidden);
+hipError_t launch_cast_back(const uint64_t* d_tbl, void* d_chunk_map, const float* d_factor, bool use_fp8,
                             long long max_rows, const Dims& d, hipStream_t stream);
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
 // waves per CU the synthetic streams run at from now on (0: as many as fit)

@@ -40,7 +40,8 @@
 //                   (mooncake_ep_kernel.cu:711-753); a selection counts while
 //                   topk_idx, as combine is given it, still names the expert
 //                   (:719-732).
-//   cast_back_kernel  the consumer of the packed layout: valid rows back to
+//   cast_back_kernel  the consumer of the packed layout (cast_chunks_kernel: its
+//                   work list in worlds of many experts): valid rows back to
 //                   bf16, times a per-expert factor
 //                   (per_token_cast_back, mooncake-wheel/tests/ep_test_utils.py:50-53;
 //                   the mock expert of mooncake-ep/tests/test_ep_grid.py:168-173).
@@ -1654,13 +1655,69 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
     }
 }
 
+// Work list of the cast-back kernel for worlds of many experts (cast_back_listed): which (expert, row chunk) each
+// chunk number is; map[0].x is the number of chunks.  Per block: a thread per expert fetches the count, one wave
+// scans ceil(count / kCastRows) over the experts in LDS, then a thread per chunk finds its expert by bisection of the
+// scanned begins.
+constexpr int kCastMaxExperts = 4096;
+constexpr int kCastMapBlocks = 8;      // each repeats the scan (cheap) and writes an eighth of the entries
+
+template <int TW>
+__global__ __launch_bounds__(1024) void cast_chunks_kernel(const uint64_t* __restrict__ tbl_mem, RankPtr counts,
+                                                           int4* __restrict__ map, int R, int E, int max_tokens,
+                                                           int max_chunks, ArgTable<TW> arg_tbl) {
+    const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
+    __shared__ int lds_count[kCastMaxExperts];
+    __shared__ int lds_begin[kCastMaxExperts + 1];
+    const int lane = wave_lane();
+    const int L = E / R;
+    const int64_t RM = (int64_t)R * max_tokens;
+    for (int ee = threadIdx.x; ee < E; ee += blockDim.x) {
+        const int qq = ee / L;
+        const uint64_t cnt = rank_ptr(tbl, counts, XF_RECV_COUNT, R, qq);
+        int c = 0;
+        // a rank without tensors takes no part (evenly spaced counts are those of ranks that all do)
+        if (counts.base != 0 || (cnt != 0 && tbl[XF_RECV_X * R + qq] != 0 && tbl[XF_OUT * R + qq] != 0))
+            c = load_i32(cnt + (uint64_t)(ee - qq * L) * 4);
+        lds_count[ee] = c < 0 ? 0 : (c > RM ? (int)RM : c);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        int carry = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int ee = e0 + lane;
+            const int n = (ee < E) ? (lds_count[ee] + kCastRows - 1) / kCastRows : 0;
+            const int incl = wave_scan_inclusive(n);
+            if (ee < E) lds_begin[ee] = carry + incl - n;
+            carry += __builtin_amdgcn_readlane(incl, 63);
+        }
+        if (lane == 0) {
+            lds_begin[E] = carry;
+            if (blockIdx.x == 0) map[0] = make_int4(carry < max_chunks ? carry : max_chunks, 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    const int total = lds_begin[E] < max_chunks ? lds_begin[E] : max_chunks;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
+        // the last expert whose first chunk number is <= i (experts without rows share their successor's begin)
+        int lo = 0, hi = E;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (lds_begin[mid] <= i) lo = mid; else hi = mid;
+        }
+        map[1 + i] = make_int4(lo, i - lds_begin[lo], lds_count[lo], 0);
+    }
+}
+
 // A block takes one chunk (kCastRows consecutive packed rows of one expert)
 // times kCastCols columns, so only rows below packed_recv_count cost anything.
 // Which expert the block's chunk number belongs to follows from the counts
 // alone, and every block finds it by itself: a thread adds up ceil(count /
 // kCastRows) over a run of experts, the block scans the sums, and the thread
-// whose run holds the number says which.  That is one load and two barriers in
-// front of the first row, where a work list cost a launch (5 us) and a load.
+// whose run holds the number says which.  That is a load or two and two barriers
+// in front of the first row, where a work list costs a launch (5 us) and a load;
+// with long runs in many blocks the list is the cheaper one (LISTED,
+// cast_back_listed).
 //
 // Each of the kCastWaves waves converts kCastRows / kCastWaves consecutive rows,
 // all their loads in flight together (with one row per wave the kernel was held
@@ -1674,61 +1731,69 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
 // 8 x 256 tokens fp8 144.8 / 150.4 / - us, 32 x 128 271.9 / 276.7 / -, 8 x 1024
 // 533.0 / 533.3 / 538.1, Mixtral 107.5 / 105.8 / 108.3; the payload, read once,
 // is better loaded with the streaming hint (bf16, 8 x 512: 187 against 201).
-constexpr int kCastWaves = 4;
-constexpr int kCastCols = 1024;
-constexpr int kCastMaxExperts = 4096;
-
-template <bool FP8, int TW>
+template <bool FP8, int TW, bool LISTED>
 __global__ __launch_bounds__(kCastWaves * 64) void cast_back_kernel(const uint64_t* __restrict__ tbl_mem, RankPtr counts,
+                                                         const int4* __restrict__ map,
                                                          const float* __restrict__ factor, int R, int E, int H,
                                                          int max_tokens, int parts, ArgTable<TW> arg_tbl) {
     const uint64_t* tbl = TW > 0 ? arg_tbl.v : tbl_mem;
-    __shared__ int lds_wave[kCastWaves];
-    __shared__ int lds_item[3];
     const int lane = wave_lane();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int target = blockIdx.x / parts, part = blockIdx.x - target * parts;
     const int L = E / R;
     const int64_t RM = (int64_t)R * max_tokens;
 
-    // this thread's run of experts
-    const int run = (E + kCastWaves * 64 - 1) / (kCastWaves * 64);
-    const int e_first = threadIdx.x * run;
-    auto valid_rows = [&](int ee) -> int {
-        if (ee >= E) return 0;
-        const int qq = ee / L;
-        const uint64_t cnt = rank_ptr(tbl, counts, XF_RECV_COUNT, R, qq);
-        // a rank without tensors takes no part (evenly spaced counts are those of ranks that all do)
-        if (counts.base == 0 && (cnt == 0 || tbl[XF_RECV_X * R + qq] == 0 || tbl[XF_OUT * R + qq] == 0)) return 0;
-        const int c = load_i32(cnt + (uint64_t)(ee - qq * L) * 4);
-        return c < 0 ? 0 : (c > RM ? (int)RM : c);
-    };
-    int chunks = 0;
-    for (int i = 0; i < run; ++i) chunks += (valid_rows(e_first + i) + kCastRows - 1) / kCastRows;
-    const int incl = wave_scan_inclusive(chunks);
-    if (lane == 63) lds_wave[wave] = incl;
-    if (threadIdx.x == 0) lds_item[0] = -1;
-    __syncthreads();
-    int begin = incl - chunks;
+    int e, chunk, count;
+    if constexpr (LISTED) {
+        const int total = map[0].x;
+        if (target >= total) return;        // block-uniform
+        const int4 item = map[1 + target];
+        e = __builtin_amdgcn_readfirstlane(item.x);
+        chunk = __builtin_amdgcn_readfirstlane(item.y);
+        count = __builtin_amdgcn_readfirstlane(item.z);
+    } else {
+        __shared__ int lds_wave[kCastWaves];
+        __shared__ int lds_item[3];
+        // this thread's run of experts
+        const int run = (E + kCastWaves * 64 - 1) / (kCastWaves * 64);
+        const int e_first = threadIdx.x * run;
+        auto valid_rows = [&](int ee) -> int {
+            if (ee >= E) return 0;
+            const int qq = ee / L;
+            const uint64_t cnt = rank_ptr(tbl, counts, XF_RECV_COUNT, R, qq);
+            // a rank without tensors takes no part (evenly spaced counts are those of ranks that all do)
+            if (counts.base == 0 && (cnt == 0 || tbl[XF_RECV_X * R + qq] == 0 || tbl[XF_OUT * R + qq] == 0)) return 0;
+            const int c = load_i32(cnt + (uint64_t)(ee - qq * L) * 4);
+            return c < 0 ? 0 : (c > RM ? (int)RM : c);
+        };
+        int chunks = 0;
+        for (int i = 0; i < run; ++i) chunks += (valid_rows(e_first + i) + kCastRows - 1) / kCastRows;
+        const int incl = wave_scan_inclusive(chunks);
+        if (lane == 63) lds_wave[wave] = incl;
+        if (threadIdx.x == 0) lds_item[0] = -1;
+        __syncthreads();
+        int begin = incl - chunks;
 #pragma unroll
-    for (int w = 0; w < kCastWaves - 1; ++w) begin += w < wave ? lds_wave[w] : 0;
-    if (begin <= target && target < begin + chunks) {
-        for (int i = 0; i < run; ++i) {
-            const int c = valid_rows(e_first + i), n = (c + kCastRows - 1) / kCastRows;
-            if (target < begin + n) {
-                lds_item[0] = e_first + i;
-                lds_item[1] = target - begin;
-                lds_item[2] = c;
-                break;
+        for (int w = 0; w < kCastWaves - 1; ++w) begin += w < wave ? lds_wave[w] : 0;
+        if (begin <= target && target < begin + chunks) {
+            for (int i = 0; i < run; ++i) {
+                const int c = valid_rows(e_first + i), n = (c + kCastRows - 1) / kCastRows;
+                if (target < begin + n) {
+                    lds_item[0] = e_first + i;
+                    lds_item[1] = target - begin;
+                    lds_item[2] = c;
+                    break;
+                }
+                begin += n;
             }
-            begin += n;
         }
+        __syncthreads();
+        e = __builtin_amdgcn_readfirstlane(lds_item[0]);
+        if (e < 0) return;                      // beyond the last chunk
+        chunk = __builtin_amdgcn_readfirstlane(lds_item[1]);
+        count = __builtin_amdgcn_readfirstlane(lds_item[2]);
     }
-    __syncthreads();
-    const int e = __builtin_amdgcn_readfirstlane(lds_item[0]);
-    if (e < 0) return;                      // beyond the last chunk
-    const int row0 = __builtin_amdgcn_readfirstlane(lds_item[1]) * kCastRows + wave * (kCastRows / kCastWaves);
-    const int count = __builtin_amdgcn_readfirstlane(lds_item[2]);
+    const int row0 = chunk * kCastRows + wave * (kCastRows / kCastWaves);
     if (row0 >= count) return;              // wave-uniform
 
     const int q = e / L, le = e - q * L;
@@ -2296,12 +2361,11 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
 #undef MCEP_P4
 }
 
-hipError_t launch_cast_back(const uint64_t* d_tbl, const float* d_factor, bool use_fp8,
+hipError_t launch_cast_back(const uint64_t* d_tbl, void* d_chunk_map, const float* d_factor, bool use_fp8,
                             long long max_rows, const Dims& d, hipStream_t stream) {
     const int parts = (d.H + kCastCols - 1) / kCastCols;
     const long long blocks = cast_back_chunks(max_rows, d.E) * parts;
     if (blocks <= 0) return hipSuccess;
-    // (every block looks at all the counts, which is meant for no more than this many)
     if (blocks > 0x7fffffffll || d.E > kCastMaxExperts) return hipErrorInvalidValue;
     // The table is in the arguments, with the counts' address and spacing beside it where they are even: one
     // dependent load less in front of every block.
@@ -2317,13 +2381,29 @@ hipError_t launch_cast_back(const uint64_t* d_tbl, const float* d_factor, bool u
             even = even && c[r] != 0 && c[r] == c[0] + (uint64_t)(stride * r) && d.host_table[XF_RECV_X * d.R + r] != 0;
         if (even) counts = RankPtr{c[0], stride};
     }
+    const long long chunks = cast_back_chunks(max_rows, d.E);
+    const bool listed = cast_back_listed(max_rows, d.E, d.H);
+    int4* map = (int4*)d_chunk_map;
+    if (listed && map == nullptr) return hipErrorInvalidValue;
+#define MCEP_CAST_L(FP8, TW, LISTED)                                                                                \
+    hipLaunchKernelGGL((cast_back_kernel<FP8, TW, LISTED>), dim3((unsigned)blocks), dim3(kCastWaves * 64), 0,       \
+                       stream, d_tbl, counts, map, d_factor, d.R, d.E, d.H, d.max_tokens, parts,                    \
+                       arg_table<TW>(d.host_table, words))
 #define MCEP_CAST(FP8, TW)                                                                                          \
-    hipLaunchKernelGGL((cast_back_kernel<FP8, TW>), dim3((unsigned)blocks), dim3(kCastWaves * 64), 0, stream, d_tbl, \
-                       counts, d_factor, d.R, d.E, d.H, d.max_tokens, parts, arg_table<TW>(d.host_table, words))
+    do {                                                                                                            \
+        if (!listed) {                                                                                              \
+            MCEP_CAST_L(FP8, TW, false);                                                                            \
+            break;                                                                                                  \
+        }                                                                                                           \
+        hipLaunchKernelGGL(cast_chunks_kernel<TW>, dim3(kCastMapBlocks), dim3(1024), 0, stream, d_tbl, counts, map,  \
+                           d.R, d.E, d.max_tokens, (int)chunks, arg_table<TW>(d.host_table, words));                     \
+        MCEP_CAST_L(FP8, TW, true);                                                                                 \
+    } while (0)
     if (use_fp8 && d.host_table != nullptr) MCEP_CAST(true, kWords);
     else if (use_fp8) MCEP_CAST(true, 0);
     else if (d.host_table != nullptr) MCEP_CAST(false, kWords);
     else MCEP_CAST(false, 0);
+#undef MCEP_CAST_L
 #undef MCEP_CAST
     return hipGetLastError();
 }

@@ -89,4 +89,13 @@ long long cast_back_chunks(long long max_rows, int num_experts) {
     return chunks < max_rows ? chunks : max_rows;
 }
 
+bool cast_back_listed(long long max_rows, int num_experts, int hidden) {
+    // Every block reads a thread's run of counts after each other, ceil(E / 256) of them.  Listed / searched, us, by
+    // blocks x run: 1024 experts, 128 tokens of hidden 1024, top-8 (4096) 8.6 / 6.8; 8 x 20 tokens of hidden 6784, top-7, 768
+    // experts (22344) 12.3 / 13.0, 1024 experts 13.0 / 18.3; 2048 experts, 128 tokens of 7168 (57344) 15.4 / 34.3.
+    const long long run = (num_experts + kCastWaves * 64 - 1) / (kCastWaves * 64);
+    const long long blocks = cast_back_chunks(max_rows, num_experts) * ((hidden + kCastCols - 1) / kCastCols);
+    return run > 2 && blocks * run > 16384;
+}
+
 }  // namespace mcep

@@ -240,6 +240,8 @@ struct mc_ep_world {
     size_t row_src_cap = 0;
     int32_t* d_counts = nullptr;
     size_t counts_cap = 0;
+    uint32_t* d_chunk_map = nullptr;     // work list of the cast-back kernel (many experts), 4 words per entry
+    size_t chunk_map_cap = 0;
     // what the last dispatch was called with, so that a combine given that
     // dispatch's handle can reuse its routing state instead of re-deriving rows
     struct LastDispatch {
@@ -277,7 +279,7 @@ struct mc_ep_world {
         const bool switched = hipGetDevice(&prev) == hipSuccess && prev != device && hipSetDevice(device) == hipSuccess;
         (void)hipDeviceSynchronize();
         void* owned[] = {d_tbl[0], d_tbl[1], d_tbl[2], d_captured_tbl[0], d_captured_tbl[1], d_captured_tbl[2],
-                         d_ucount, d_ucount_t, d_ubegin, d_selpos, d_selrow, d_row_src, d_counts, d_routes,
+                         d_ucount, d_ucount_t, d_ubegin, d_selpos, d_selrow, d_row_src, d_counts, d_chunk_map, d_routes,
                          d_scale_stage, d_zero_row};
         for (void* p : owned)
             if (p) (void)hipFree(p);
@@ -1338,7 +1340,11 @@ int mc_ep_world_cast_back(mc_ep_world_t* w, const uint64_t* recv_x_ptrs, const u
     // valid rows of the world: at most one per selection, and no more than the layout holds
     long long max_rows = (long long)num_experts * R * max_tokens;
     if (num_topk > 0 && (long long)R * max_tokens * num_topk < max_rows) max_rows = (long long)R * max_tokens * num_topk;
-    MC_HIP(launch_cast_back(d_tbl, (const float*)expert_factor_ptr, use_fp8, max_rows, d, stream));
+    if (cast_back_listed(max_rows, num_experts, hidden)) {
+        const size_t map_words = (size_t)(cast_back_chunks(max_rows, num_experts) + 1) * 4;
+        if (int rc = ensure_scratch(w, &w->d_chunk_map, &w->chunk_map_cap, map_words)) return rc;
+    }
+    MC_HIP(launch_cast_back(d_tbl, w->d_chunk_map, (const float*)expert_factor_ptr, use_fp8, max_rows, d, stream));
     return MC_EP_OK;
 }
 

@@ -36,7 +36,7 @@ hipError_t launch_reduce_packed(const uint64_t*, const CombineRoute*, uint32_t, 
                                 hipStream_t s) {
     return launched(s);
 }
-hipError_t launch_cast_back(const uint64_t*, const float*, bool, long long, const Dims&, hipStream_t s) {
+hipError_t launch_cast_back(const uint64_t*, void*, const float*, bool, long long, const Dims&, hipStream_t s) {
     return launched(s);
 }
 hipError_t launch_copy(void*, const void*, size_t, hipStream_t s) { return launched(s); }

@@ -1,6 +1,7 @@
 """The cast-back kernel's search for the rows of its 16-row chunks, at its edges, against the oracle bit for bit:
-counts around the chunk size, experts without rows, one to five experts per searching thread, scales whose columns are
-no multiple of four rows, more ranks than travel in kernel arguments, unevenly spaced count tensors, an absent rank."""
+counts around the chunk size, experts without rows, one to sixteen experts per searching thread, scales whose columns are
+no multiple of four rows, more ranks than travel in kernel arguments, worlds
+of so many experts that the chunks come from a work list, unevenly spaced count tensors, an absent rank."""
 import pytest
 import torch
 
@@ -19,7 +20,8 @@ EDGES = [0, 1, 15, 16, 17, 0, 0, 31, 32, 33, 4, 5]
 @pytest.mark.parametrize("shape", [
     # ranks, tokens, hidden, experts, absent rank
     (1, 33, 1152, 1, None), (1, 35, 128, 12, None), (3, 12, 1024, 255, 1), (4, 9, 256, 260, None), (2, 17, 2176, 514, 0),
-    (3, 11, 128, 1281, None), (32, 2, 128, 64, 7), (33, 1, 256, 99, 32),
+    (3, 11, 128, 1281, None), (2, 20, 128, 2050, None), (4, 9, 256, 4096, 2),
+    (33, 3, 1152, 1056, 5), (32, 2, 128, 64, 7), (33, 1, 256, 99, 32),
 ], ids=lambda s: "x".join(str(v) for v in s))
 def test_chunk_edges(gpu_device, oracle, shape, use_fp8):
     R, T, H, E, absent = shape
