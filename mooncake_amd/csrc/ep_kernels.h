@@ -228,7 +228,7 @@ constexpr int kCastRows = 16;         // packed rows of one expert per work item
 long long cast_back_chunks(long long max_rows, int num_experts);
 constexpr int kCastWaves = 4;         // waves per block of the kernel
 constexpr int kCastCols = 1024;       // columns of a row per block
-// whether the blocks' chunks come from a work list; d_chunk_map then holds 16 bytes x (cast_back_chunks(max_rows, E) + 1)
+// whether a work list pays (d_chunk_map: 16 bytes x (cast_back_chunks(max_rows, E) + 1); null: the blocks search)
 bool cast_back_listed(long long max_rows, int num_experts, int hidden);
 hipError_t launch_cast_back(const uint64_t* d_tbl, void* d_chunk_map, const float* d_factor, bool use_fp8,
                             long long max_rows, const Dims& d, hipStream_t stream);

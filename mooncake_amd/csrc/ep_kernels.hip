@@ -2382,9 +2382,8 @@ hipError_t launch_cast_back(const uint64_t* d_tbl, void* d_chunk_map, const floa
         if (even) counts = RankPtr{c[0], stride};
     }
     const long long chunks = cast_back_chunks(max_rows, d.E);
-    const bool listed = cast_back_listed(max_rows, d.E, d.H);
     int4* map = (int4*)d_chunk_map;
-    if (listed && map == nullptr) return hipErrorInvalidValue;
+    const bool listed = map != nullptr;
 #define MCEP_CAST_L(FP8, TW, LISTED)                                                                                \
     hipLaunchKernelGGL((cast_back_kernel<FP8, TW, LISTED>), dim3((unsigned)blocks), dim3(kCastWaves * 64), 0,       \
                        stream, d_tbl, counts, map, d_factor, d.R, d.E, d.H, d.max_tokens, parts,                    \

@@ -1340,11 +1340,13 @@ int mc_ep_world_cast_back(mc_ep_world_t* w, const uint64_t* recv_x_ptrs, const u
     // valid rows of the world: at most one per selection, and no more than the layout holds
     long long max_rows = (long long)num_experts * R * max_tokens;
     if (num_topk > 0 && (long long)R * max_tokens * num_topk < max_rows) max_rows = (long long)R * max_tokens * num_topk;
-    if (cast_back_listed(max_rows, num_experts, hidden)) {
-        const size_t map_words = (size_t)(cast_back_chunks(max_rows, num_experts) + 1) * 4;
+    // (a recorded call has the list only where an eager one has made room for it)
+    const size_t map_words = (size_t)(cast_back_chunks(max_rows, num_experts) + 1) * 4;
+    const bool listed = cast_back_listed(max_rows, num_experts, hidden) && (!cap.active || map_words <= w->chunk_map_cap);
+    if (listed)
         if (int rc = ensure_scratch(w, &w->d_chunk_map, &w->chunk_map_cap, map_words)) return rc;
-    }
-    MC_HIP(launch_cast_back(d_tbl, w->d_chunk_map, (const float*)expert_factor_ptr, use_fp8, max_rows, d, stream));
+    MC_HIP(launch_cast_back(d_tbl, listed ? w->d_chunk_map : nullptr, (const float*)expert_factor_ptr, use_fp8, max_rows, d,
+                            stream));
     return MC_EP_OK;
 }
 

@@ -164,3 +164,34 @@ def test_a_one_launch_call_prepares_for_recording_the_others(gpu_device, oracle,
         torch.cuda.synchronize()
         ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, cfg.use_fp8)
         compare_dispatch(h, ref, check_poison=True)
+
+
+@pytest.mark.parametrize("warm", [False, True], ids=["searched", "listed"])
+def test_cast_back_of_many_experts_recorded(gpu_device, oracle, warm):
+    """The work list of a cast back needs scratch; recorded without it, the kernel's blocks search for themselves."""
+    R, T, H, E = 1, 8, 256, 1800
+    cfg = EPConfig("graph_cast", R, T, H, E, 0, True)
+    announce(f"recorded cast back {cfg} warm={warm}")
+    h = WorldHarness(cfg, world=ep.World(R))
+    h.alloc_dispatch_outputs(poison=False)
+    h.alloc_combine_io()
+    gen = torch.Generator().manual_seed(92)
+    h.recv_x.copy_(torch.randint(0, 0x7f, h.recv_x.shape, generator=gen).to(torch.uint8))
+    h.recv_scales_phys.copy_(torch.rand(h.recv_scales_phys.shape, generator=gen) + 0.01)
+    factor = (torch.rand(E, generator=gen) + 0.5).to(gpu_device)
+    torch.cuda.synchronize()
+    if warm:
+        h.cast_back(factor)
+        torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        h.cast_back(factor)
+    for i in range(3):
+        h.recv_count.copy_(torch.randint(0, T + 1, h.recv_count.shape, generator=gen, dtype=torch.int32))
+        want = oracle.cast_back(h.recv_x.cpu().view(torch.uint8), h.recv_scales().cpu(), h.recv_count.cpu(), factor.cpu(),
+                                fill=0x5A5A)
+        for call in (g.replay, lambda: h.cast_back(factor)):
+            h.expert_out.view(torch.int16).fill_(0x5A5A)
+            call()
+            torch.cuda.synchronize()
+            assert torch.equal(h.expert_out.cpu().view(torch.int16), want.view(torch.int16)), f"pass {i}"
