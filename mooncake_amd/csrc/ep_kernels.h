@@ -193,6 +193,7 @@ void plan_units(Dims& d, const Tuning& t);
 struct SmallPlan {
     bool fused = false;
     bool alone = false;        // dispatch_alone_kernel: every wave counts by itself; else dispatch_small_kernel
+    bool could = false;        // the shared count can take it, if only because a recorded call has nothing else
     bool single = false;       // few enough lists that a wave counting alone could take them
 };
 SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t);

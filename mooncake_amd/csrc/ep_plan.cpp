@@ -69,6 +69,7 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
     // 11.5 / 13.1, 8.4 / 12.4; top-1, 4096 tokens (32768) 12.5 / 15.1 and 19.6 / 18.3, hot 12.8 / 33.3.  Rows of half a slab
     // and less have not been measured over that range, and stay with the separate launches.
     const long long walked = (long long)R * (((long long)most * K + kSmallListRound - 1) / kSmallListRound);
+    p.could = hidden > 512 && R <= kSmallRanks && R <= kSmallWaveRanks * waves && (lists + waves - 1) / waves <= limit;
     p.fused = hidden > 512 && R <= kSmallRanks && R <= kSmallWaveRanks * waves &&
               (walked + waves - 1) / waves <= limit && (chosen || tokens * walked <= (use_fp8 ? 16384 : 8192));
     return p;

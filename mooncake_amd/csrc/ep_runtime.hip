@@ -549,7 +549,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     // lists (dispatch_small_kernel, dispatch_alone_kernel); the rank table then travels in kernel arguments.
     const SmallPlan small = phases == MC_EP_PHASE_ALL ? plan_small(num_tokens, R, num_topk, hidden, use_fp8 != 0, w->tuning)
                                                       : SmallPlan{};
-    const bool fused = small.fused;
+    bool fused = small.fused;
     DeviceGuard guard(w->device);
     w->launches = 0;
     struct Tally {                                // the option "last_dispatch_launches", on every way out
@@ -612,6 +612,11 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         if (int rc = capture_of(stream, &cap)) return rc;
         RecordingScope recording(cap.active);
         if (int rc = order_begin(w, stream, cap)) return rc;
+        // A recorded call that the one launch can take does not fail for want of the separate launches' scratch.
+        if (cap.active && !fused && small.could)
+            fused = w->ucount_cap < UE || w->ubegin_cap < UE || w->ucount_t_cap < (size_t)num_experts * kMaxSummedUnits ||
+                    w->selpos_cap < (size_t)R * max_tokens * num_topk || w->counts_cap < (size_t)num_experts ||
+                    w->row_src_cap < (size_t)num_experts * R * max_tokens || w->scale_stage_cap < stage_floats;
         // (two entries at least: dispatch_small_kernel may read 8 bytes there)
         if (int rc = ensure_scratch(w, &w->d_selrow, &w->selrow_cap, (size_t)R * max_tokens * num_topk + 1)) return rc;
         // The one-launch dispatch keeps no routing state but selrow.  An eager one prepares the world for the separate

@@ -195,3 +195,35 @@ def test_cast_back_of_many_experts_recorded(gpu_device, oracle, warm):
             call()
             torch.cuda.synchronize()
             assert torch.equal(h.expert_out.cpu().view(torch.int16), want.view(torch.int16)), f"pass {i}"
+
+
+def test_a_recorded_call_takes_the_one_launch_rather_than_fail(gpu_device, oracle):
+    """The eager call's list is one that a wave counts alone, which leaves no scratch for the separate launches.  The recorded
+    one has seven rounds of one list: by the measured lines the separate launches, but the shared count can take it."""
+    cfg = EPConfig("graph_could", 1, 3584, 640, 8, 1, True)
+    announce(f"recorded without scratch for the separate launches {cfg}")
+    world = ep.World(1)
+    few = WorldHarness(cfg, world=world, num_tokens=[100])
+    few.load(generate(cfg, seed=94))
+    few.alloc_dispatch_outputs()
+    few.dispatch()
+    torch.cuda.synchronize()
+    assert world.get_option("last_dispatch_launches") == 1
+    data = generate(cfg, seed=95)
+    h = WorldHarness(cfg, world=world)
+    h.load(data)
+    h.alloc_dispatch_outputs(poison=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        h.dispatch()
+    assert world.get_option("last_dispatch_launches") == 1
+    ref = oracle.dispatch(data["x"], data["topk_idx"], [3584], 3584, 8, True)
+    for _ in range(3):
+        g.replay()
+        few.dispatch()
+        torch.cuda.synchronize()
+        compare_dispatch(h, ref, check_poison=True)
+    h.dispatch()                                    # an eager call makes room for the separate launches and takes them
+    torch.cuda.synchronize()
+    assert world.get_option("last_dispatch_launches") > 1
+    compare_dispatch(h, ref, check_poison=True)
