@@ -108,3 +108,35 @@ def test_a_table_left_in_memory_is_the_next_call_s(gpu_device, oracle, ranks, se
             torch.cuda.synchronize()
             assert torch.equal(h.combined.view(torch.int16), want.view(torch.int16))
             h.expert_out.copy_(rows)
+
+
+@pytest.mark.parametrize("source", ["dispatch", "searched", "resolved"])
+@pytest.mark.parametrize("ranks", [3, 32])
+def test_a_table_is_left_by_a_block_without_tokens(gpu_device, oracle, ranks, source):
+    """The waves of the first block end early where the first rank has no tokens; the table is in memory all the same."""
+    cfg = EPConfig("left_early", ranks, 8, 256, 2 * ranks, 2, True)
+    nt = [0] + [(r * 5) % 8 + 1 for r in range(1, ranks)]
+    announce(f"rank table left by an empty block ranks={ranks} {source}")
+    world = ep.World(ranks)
+    world.set_option("combine_search_tokens", 0 if source == "resolved" else 256)
+    a, b = _harness(cfg, world, 5, nt), _harness(cfg, world, 6, nt)
+    a.dispatch()
+    b.dispatch()
+    if source == "dispatch":
+        a.dispatch()
+    for h in (a, a, b, b, a, a):
+        h.combined.fill_(7.0)
+        h.combine()
+        torch.cuda.synchronize()
+        _check(h, oracle, h.combined.cpu())
+    rows = a.expert_out.clone()
+    a.cast_back()
+    a.combine()
+    want = a.combined.clone()
+    a.expert_out.copy_(rows)
+    for _ in range(2):
+        a.combined.fill_(7.0)
+        a.combine_packed()
+        torch.cuda.synchronize()
+        for r, n in enumerate(a.num_tokens):
+            assert torch.equal(a.combined[r, :n].view(torch.int16), want[r, :n].view(torch.int16))
