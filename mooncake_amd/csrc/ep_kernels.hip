@@ -1541,25 +1541,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
     float w = 0.0f, f = 1.0f;
     int sstride = 0;                     // bytes between a row's consecutive scale groups (0: the zero row)
     int live = 1;                        // loaded here, looked at after the payload loads are issued (not: kFromRoutes)
-    constexpr int kLanes = lanes_per_selection<FROM, KMAX>();      // selection k's row ends up in lane k * kLanes
+    // selection k's row ends up in the lanes from k * kLanes on
+    constexpr int kLanes = FP8 ? lanes_per_selection<kFromHandle, KMAX>() : lanes_per_selection<FROM, KMAX>();
+    const int sel = lane / kLanes;
     {
         int e = 0, slot = 0;
         bool ok = false;
         float wl = 0.0f;
         if (FROM != kFromRoutes) {
             const uint64_t w_row = rank_ptr(tbl, cs.topk_weights, CF_TOPK_W, R, r) + (uint64_t)((int64_t)t * K) * 4;
-            wl = load_f32(w_row + (uint64_t)(lane / kLanes < K ? lane / kLanes : 0) * 4);
+            wl = load_f32(w_row + (uint64_t)(sel < K ? sel : 0) * 4);
             DirectRow d;
             if constexpr (FROM == kFromHandle) d = search_row<kLanes>(tbl, cs, R, E, K, max_tokens, r, t, lane);
-            else d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, lane);
+            else d = direct_row(tbl, sc, cs, R, E, K, max_tokens, r, t, sel);
             ok = d.has;
             e = d.e;
             slot = d.slot;
             live = d.live;
         } else {
             uint4 rt = make_uint4(0, 0, 0, 0);
-            if (lane < K) rt = *(const uint4*)(routes + ((int64_t)r * max_tokens + t) * K + lane);
-            ok = (lane < K) && (rt.w == stamp) && (int)rt.y < E && (int64_t)rt.x < RM;
+            if (sel < K) rt = *(const uint4*)(routes + ((int64_t)r * max_tokens + t) * K + sel);
+            ok = (sel < K) && (rt.w == stamp) && (int)rt.y < E && (int64_t)rt.x < RM;
             e = ok ? (int)rt.y : 0;
             slot = ok ? (int)rt.x : 0;
             wl = __uint_as_float(rt.z);
@@ -1589,26 +1591,35 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
         on[c] = elem[c] < H;
         poff[c] = on[c] ? (int64_t)elem[c] * (FP8 ? 1 : 2) : 0;
     }
-    const int group = on[0] ? (elem[0] >> 7) : 0;
-
     uint4 v[KMAX][CH];
     float sv[KMAX], wk[KMAX], fk[KMAX];
+    // A slab's scales of all K rows, eight groups a row, in one load (above top-8 two): a selection's lanes fetch its groups,
+    // and every lane picks the one of its own group up when it is needed.  A load per row, each lane its own group's scale,
+    // was K vector loads and K addresses in front of the arithmetic: 16 x 256 tokens, hidden 1152, top-5 in eight rows 21.6 ->
+    // 20.1 us, 32 x 87, 1792, top-9 in sixteen 27.5 -> 25.7, 32 x 128, 7168, top-8, which is bound by its bytes, 60.6 -> 60.3.
+    constexpr int kFetch = kLanes >= 8 ? 1 : 8 / kLanes;
+    float mine[kFetch];
+    if (FP8) {
+#pragma unroll
+        for (int i = 0; i < kFetch; ++i) {
+            const int j = i * kLanes + (lane & (kLanes - 1));
+            const int g = s * 8 + (j < 8 ? j : 7);
+            mine[i] = load_f32(ssrc + (uint64_t)((int64_t)(g < G ? g : G - 1) * sstride));
+        }
+    }
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
         const uint64_t p = read_lane_u64(src, k * kLanes);
 #pragma unroll
         for (int c = 0; c < CH; ++c) v[k][c] = load16<true>((const void*)(p + poff[c]));
-        if (FP8) {
-            const uint64_t sp = read_lane_u64(ssrc, k * kLanes);
-            const int st = __builtin_amdgcn_readlane(sstride, k * kLanes);
-            sv[k] = load_f32(sp + (uint64_t)((int64_t)group * st));
-        } else {
-            sv[k] = 1.0f;
-        }
     }
 
     // a row of a rank the token's owner sees as inactive was fetched before that was known: drop it
-    if (FROM != kFromRoutes && live == 0) w = 0.0f;
+    if (FROM != kFromRoutes && live == 0) {
+        w = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kFetch; ++i) mine[i] = 0.0f;
+    }
     // the expert's factor was loaded behind the row table, like `live`: looked at only now, when the payload
     // loads are on their way
     asm volatile("" : "+v"(f));
@@ -1619,7 +1630,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
         if (FROM != kFromRoutes && __builtin_amdgcn_readlane(live, k * kLanes) == 0) {
 #pragma unroll
             for (int c = 0; c < CH; ++c) v[k][c] = make_uint4(0, 0, 0, 0);
+        }
+        if (FP8) {
+            const int own = lane >> 3;                   // the lane's group among the slab's eight
             sv[k] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kFetch; ++i) {
+                const int from = k * kLanes + (own & (kLanes - 1));
+                const float x = __int_as_float(__builtin_amdgcn_ds_bpermute(from * 4, __float_as_int(mine[i])));
+                if (kFetch == 1 || own / kLanes == i) sv[k] = x;
+            }
+        } else {
+            sv[k] = 1.0f;
         }
     }
 #pragma unroll
@@ -2297,7 +2319,12 @@ hipError_t launch_reduce(const uint64_t* d_tbl, const CombineRoute* d_routes, ui
     if (d.K <= 2) MCEP_K(2);
     if (d.K <= 4) MCEP_K(4);
     if (d.K <= 6) MCEP_K(6);
+    // (8 x 512 tokens, hidden 4096, bf16, us, padded / exact: top-7 in eight rows 45.5 / 43.5, top-9 in twelve 56.8 / 53.0,
+    // top-10 60.2 / 58.1; top-3 in four 23.5 / 23.4, top-5 in six 33.8 / 34.0, top-11 in twelve 62.3 / 61.8)
+    if (d.K <= 7) MCEP_K(7);
     if (d.K <= 8) MCEP_K(8);
+    if (d.K <= 9) MCEP_K(9);
+    if (d.K <= 10) MCEP_K(10);
     if (d.K <= 12) MCEP_K(12);
     MCEP_K(16);
 #undef MCEP_K
@@ -2346,11 +2373,6 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
     (direct       ? launch_reduce_packed_t<KMAX, FP8, FACTOR, kFromDispatch>(rl, d_factor, d, t, stream) \
      : src.search ? launch_reduce_packed_t<KMAX, FP8, FACTOR, kFromHandle>(rl, d_factor, d, t, stream)   \
                   : launch_reduce_packed_t<KMAX, FP8, FACTOR, kFromRoutes>(rl, d_factor, d, t, stream))
-#define MCEP_PK(KMAX)                                                                                \
-    do {                                                                                             \
-        if (use_fp8) return fac ? MCEP_P4(KMAX, true, true) : MCEP_P4(KMAX, true, false);            \
-        return fac ? MCEP_P4(KMAX, false, true) : MCEP_P4(KMAX, false, false);                       \
-    } while (0)
     // a bf16 payload with few rows per token: two chunks per lane, as in the combine kernel
 #define MCEP_P2(KMAX, FACTOR)                                                                        \
     (direct       ? launch_reduce_packed_t<KMAX, false, FACTOR, kFromDispatch, 2>(rl, d_factor, d, t, stream) \
@@ -2360,11 +2382,41 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
     if (!use_fp8 && ch == 2 && d.K <= 2) return fac ? MCEP_P2(2, true) : MCEP_P2(2, false);
     if (!use_fp8 && ch == 2 && d.K <= 4) return fac ? MCEP_P2(4, true) : MCEP_P2(4, false);
 #undef MCEP_P2
-    if (d.K <= 2) MCEP_PK(2);
-    if (d.K <= 4) MCEP_PK(4);
-    if (d.K <= 8) MCEP_PK(8);
-    MCEP_PK(16);
-#undef MCEP_PK
+    // Rows a variant has beyond the token's own are the zero row, fetched and multiplied like any other.  For an fp8 payload,
+    // whose rows cost arithmetic as much as bytes, each top-k has its own up to 12: combine of 8 x 512 tokens, hidden 4096, us,
+    // padded to 4, 8 or 16 rows / exact: top-3 23.8 / 21.5, top-5 33.5 / 27.2, top-6 34.6 / 30.6, top-7 35.8 / 33.9, top-9
+    // 63.3 / 40.8, top-10 64.2 / 46.0, top-11 64.5 / 47.3; 8 x 1024, hidden 7168, top-1 50.5 / 42.0.  For bf16 payloads those
+    // that gain 2 % of the combine and more: top-5 38.3 / 34.4, top-6 41.4 / 39.3, top-9 61.9 / 53.9, top-10 65.9 / 58.6,
+    // top-11 in 12 rows 66.5 / 63.0; top-7 44.5 / 44.3.
+#define MCEP_PK8(KMAX) \
+    if (use_fp8 && d.K <= KMAX) return fac ? MCEP_P4(KMAX, true, true) : MCEP_P4(KMAX, true, false)
+#define MCEP_PK16(KMAX) \
+    if (!use_fp8 && d.K <= KMAX) return fac ? MCEP_P4(KMAX, false, true) : MCEP_P4(KMAX, false, false)
+    MCEP_PK8(1);
+    MCEP_PK8(2);
+    MCEP_PK8(3);
+    MCEP_PK8(4);
+    MCEP_PK8(5);
+    MCEP_PK8(6);
+    MCEP_PK8(7);
+    MCEP_PK8(8);
+    MCEP_PK8(9);
+    MCEP_PK8(10);
+    MCEP_PK8(11);
+    MCEP_PK8(12);
+    MCEP_PK8(16);
+    MCEP_PK16(2);
+    MCEP_PK16(4);
+    MCEP_PK16(5);
+    MCEP_PK16(6);
+    MCEP_PK16(8);
+    MCEP_PK16(9);
+    MCEP_PK16(10);
+    MCEP_PK16(12);
+    MCEP_PK16(16);
+    return hipErrorInvalidValue;
+#undef MCEP_PK8
+#undef MCEP_PK16
 #undef MCEP_P4
 }
 
