@@ -107,7 +107,10 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * them, and goes through as many rounds of every rank as the longest list has;
  * by default it may then be at most 16384 (bf16: 8192) rounds for all tokens
  * together - and 0
- * always takes the count / pack / scale-transpose launches;
+ * always takes the count / pack / scale-transpose launches; "scales_direct": 1
+ * (default) leaves the last of them out where an fp8 dispatch has at most 327680
+ * scales (selections times hidden / 128, hidden above 512) and all its phases run
+ * in one call;
  * "last_dispatch_launches", "last_combine_launches": read them to learn how
  * many kernels the world's last dispatch / combine call enqueued (a rank-table
  * upload counts); "fp8_arith": 0 (default) the fp8 scale arithmetic of the reference's

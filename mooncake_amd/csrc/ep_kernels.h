@@ -174,6 +174,7 @@ struct Tuning {
     int combine_occupancy = -1;   // waves of the combine kernel a CU runs at a time; 0: as many as fit, -1: by top-k
     int packed_map = 1;        // packed combine of an fp8 payload: 1 = slabs owned by XCDs, 0 = (rank, slab) groups per XCD
     int routing_sum = 1;       // allow the summed routing plan (see UnitPlan) where the shape permits
+    int scales_direct = 1;     // allow the pack kernel to store the scales in place where they are few (see scales_direct())
     int comm_stream = 0;       // 1: per-rank rounds always run on the world's communication stream
     int fused_small = 1;       // dispatch of a small world (see dispatch_small_kernel) in one launch
     int fused_small_max = 4096;   // ... when the world names at most this many selections
@@ -189,6 +190,8 @@ struct Tuning {
 // Chooses the unit plan for a shape (summed when allowed, the shape permits and there are tokens).
 // (plan_units, plan_small, combine_reads_table, count_lds_bytes and cast_back_chunks are host arithmetic: ep_plan.cpp.)
 void plan_units(Dims& d, const Tuning& t);
+// Whether the pack kernel of an fp8 dispatch (all phases in one call) stores the scales where they belong by itself.
+bool scales_direct(const Dims& d, bool use_fp8, const Tuning& t);
 // Whether a dispatch of the world takes one launch (the sizes alone decide), and which of the two kernels.
 struct SmallPlan {
     bool fused = false;

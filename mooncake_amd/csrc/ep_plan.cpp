@@ -30,6 +30,20 @@ void plan_units(Dims& d, const Tuning& t) {
     d.plan = p;
 }
 
+bool scales_direct(const Dims& d, bool use_fp8, const Tuning& t) {
+    // Scales straight into their columns, 4-byte stores R * max_tokens floats apart, against a staging row per token and the
+    // launch that transposes them, in thousands of scales (selections x groups).  Dispatch / the cycle with the packed
+    // combine, us, transposed -> direct: 41 (640 tokens, hidden 1024, top-8) 9.8 / 18.2 -> 7.4 / 15.3; 110 (2 x 858, 1024, top-8,
+    // hot experts) 11.0 / 20.8 -> 8.8 / 18.6; 122 (1020, 3072, top-5) 11.2 / 36.9 -> 9.5 / 35.0; 262 (8 x 128, 4096, top-8)
+    // 14.4 / 28.4 -> 13.2 / 25.9; 351 (32 x 87, 1792, top-9) 19.8 / 42.4 -> 16.9 / 38.2; 459 (8 x 128, 7168, top-8) 22.1 /
+    // 38.6 -> 22.6 / 39.4, (2 x 1024, 7168, top-4) 24.8 / 46.9 -> 24.3 / 46.0; 524 (16 x 128, 4096, top-8) 25.3 / 42.6 ->
+    // 24.4 / 42.6.  A large world's 1.8 million take 30 us.  Rows of half a slab and less have not been measured.
+    constexpr long long kMostScales = 320 * 1024;
+    // (the variants exist with written-through rows only, which payloads of that size have by default)
+    return use_fp8 && t.scales_direct != 0 && (t.pack_nt < 0 || (t.pack_nt & 4)) && d.H > 512 &&
+           (long long)d.R * d.Tgrid * d.K * (d.H / 128) <= kMostScales;
+}
+
 SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t) {
     long long tokens = 0, lists = 0;           // tokens; rounds of kSmallListRound entries, each rank's list by itself
     int most = 0;

@@ -689,7 +689,9 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     if ((phases & (MC_EP_PHASE_DATA | MC_EP_PHASE_FINISH)) && tgrid > 0) {
         MC_HIP(launch_pack(d_tbl, sc, src, stage, d, use_fp8 != 0, w->tuning,
                            (phases & MC_EP_PHASE_DATA) != 0, (phases & MC_EP_PHASE_FINISH) != 0, stream));
-        w->launches += ((phases & MC_EP_PHASE_DATA) ? 1 : 0) + (((phases & MC_EP_PHASE_FINISH) && use_fp8) ? 1 : 0);
+        const bool transposed = use_fp8 && (phases & MC_EP_PHASE_FINISH) &&
+                                !((phases & MC_EP_PHASE_DATA) && scales_direct(d, true, w->tuning));
+        w->launches += ((phases & MC_EP_PHASE_DATA) ? 1 : 0) + (transposed ? 1 : 0);
     }
     // under the carried plan the pack launch also produces ubegin and the counts: only now is the
     // routing state complete for a combine to reuse
@@ -1222,6 +1224,7 @@ static int* option_slot(Tuning& t, const char* name) {
     if (!strcmp(name, "packed_map")) return &t.packed_map;
     if (!strcmp(name, "combine_occupancy")) return &t.combine_occupancy;
     if (!strcmp(name, "routing_sum")) return &t.routing_sum;
+    if (!strcmp(name, "scales_direct")) return &t.scales_direct;
     if (!strcmp(name, "combine_waves")) return &t.combine_waves;
     if (!strcmp(name, "combine_nt")) return &t.combine_nt;
     if (!strcmp(name, "last_dispatch_launches")) return &t.last_dispatch_launches;
