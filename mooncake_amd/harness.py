@@ -92,6 +92,11 @@ class WorldHarness:
         self._prepared[key] = call
         return call
 
+    def _stacked(self, R: int):
+        """What takes whole-world calls straight from the stacked tensors, if the world has it."""
+        native = getattr(self.world, "_native", None)
+        return native if native is not None and self.world.num_ranks == R else None
+
     def _stream(self, stream: Optional[torch.cuda.Stream]) -> int:
         if stream is not None:
             return int(stream.cuda_stream)
@@ -114,6 +119,12 @@ class WorldHarness:
                 self._ptrs(self.recv_count, R, present), self._ptrs(self.src_info, R, present),
                 self._ptrs(self.layout_range, R, present), self._stream(stream))
             return
+        native = self._stacked(R)
+        if native is not None and native.dispatch_stacked(
+                self.x, self.topk_idx, self.recv_x, self.recv_scales_phys, self.recv_count, self.src_info,
+                self.layout_range, self.num_tokens, present, c.hidden, c.num_topk, c.max_tokens, c.num_experts,
+                c.use_fp8, phases, self._stream(stream)):
+            return
         key = self._key("dispatch", present, self.x, self.topk_idx, self.recv_x, self.recv_scales_phys, self.recv_count,
                         self.src_info, self.layout_range)
         call = self._prepared.get(key)
@@ -131,6 +142,12 @@ class WorldHarness:
                 present: Optional[Sequence[int]] = None) -> None:
         c = self.cfg
         R = c.num_ranks
+        native = self._stacked(R)
+        if native is not None and native.combine_stacked(
+                self.expert_out, None, self.topk_idx, self.topk_weights, self.src_info, self.layout_range,
+                self.active_ranks, self.combined, self.num_tokens, present, c.hidden, c.num_topk, c.max_tokens,
+                c.num_experts, False, 0, phases, self._stream(stream)):
+            return
         key = self._key("combine", present, self.expert_out, self.topk_idx, self.topk_weights, self.src_info,
                         self.layout_range, self.active_ranks, self.combined)
         call = self._prepared.get(key)
@@ -151,6 +168,12 @@ class WorldHarness:
         self._factor = None if factor_per_expert is None else \
             factor_per_expert.to(device=self.device, dtype=torch.float32).contiguous()
         fptr = 0 if self._factor is None else self._factor.data_ptr()
+        native = self._stacked(R)
+        if native is not None and native.combine_stacked(
+                self.recv_x, self.recv_scales_phys if c.use_fp8 else None, self.topk_idx, self.topk_weights,
+                self.src_info, self.layout_range, self.active_ranks, self.combined, self.num_tokens, present, c.hidden,
+                c.num_topk, c.max_tokens, c.num_experts, True, fptr, phases, self._stream(stream)):
+            return
         key = (fptr, *self._key("combine_packed", present, self.recv_x, self.recv_scales_phys, self.topk_idx,
                                 self.topk_weights, self.src_info, self.layout_range, self.active_ranks, self.combined))
         call = self._prepared.get(key)
@@ -182,9 +205,15 @@ class WorldHarness:
             self.alloc_combine_io()
         self._factor = None if factor_per_expert is None else \
             factor_per_expert.to(device=self.device, dtype=torch.float32).contiguous()
+        fptr = 0 if self._factor is None else self._factor.data_ptr()
+        native = self._stacked(R)
+        if native is not None and native.cast_back_stacked(
+                self.recv_x, self.recv_scales_phys if c.use_fp8 else None, self.recv_count, fptr, self.expert_out, present,
+                c.hidden, c.num_topk, c.max_tokens, c.num_experts, self._stream(stream)):
+            return
         self.world.cast_back(self._ptrs(self.recv_x, R, present),
                              self._ptrs(self.recv_scales_phys, R, present) if c.use_fp8 else None,
-                             self._ptrs(self.recv_count, R), 0 if self._factor is None else self._factor.data_ptr(),
+                             self._ptrs(self.recv_count, R), fptr,
                              self._ptrs(self.expert_out, R), c.hidden, c.num_topk, c.max_tokens, c.num_experts,
                              self._stream(stream))
 
