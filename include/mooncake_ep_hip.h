@@ -106,7 +106,9 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * (32 in all), where a block has a wave per 1024 hidden elements, 4 to 8 of
  * them, and goes through as many rounds of every rank as the longest list has;
  * by default it may then be at most 16384 (bf16: 8192) rounds for all tokens
- * together - and 0
+ * together; and, by default, above 4096 up to "fused_shared_max" (16384)
+ * selections from top-3 up and between 513 and 4096 hidden elements, where
+ * blocks of several tokens read at most 6144 rounds together - and 0
  * always takes the count / pack / scale-transpose launches; "scales_direct": 1
  * (default) leaves the last of them out where an fp8 dispatch has at most 327680
  * scales (selections times hidden / 128, hidden above 512) and all its phases run

@@ -69,6 +69,10 @@ constexpr int kSmallWaves = 8;        // most waves a block of dispatch_small_ke
 constexpr int small_block_waves(int hidden) {
     return (hidden + 1023) / 1024 > kSmallWaves ? kSmallWaves : (hidden > 4096 ? (hidden + 1023) / 1024 : 4);
 }
+// tokens of a block where several share one (SmallPlan::block_tokens): a wave per slab, eight waves or nearly
+constexpr int small_block_tokens(int hidden) {
+    return (hidden + 1023) / 1024 >= kSmallWaves ? 1 : kSmallWaves / ((hidden + 1023) / 1024);
+}
 struct SmallTable {
     uint64_t v[(int)DF_COUNT * kSmallRanks];
 };
@@ -151,6 +155,7 @@ struct Dims {
     int max_tokens;   // num_max_dispatch_tokens_per_rank
     int Tgrid;        // max over ranks of T_r (grid extent in tokens per rank)
     UnitPlan plan;    // set by plan_units()
+    int block_tokens = 1;      // one-launch dispatch: SmallPlan::block_tokens
     const uint64_t* host_table = nullptr;   // the call's rank table, to travel in kernel arguments; null: it is on the device
     int units_per_rank() const { return plan.per_rank; }
     int units() const { return plan.total; }
@@ -178,6 +183,7 @@ struct Tuning {
     int comm_stream = 0;       // 1: per-rank rounds always run on the world's communication stream
     int fused_small = 1;       // dispatch of a small world (see dispatch_small_kernel) in one launch
     int fused_small_max = 4096;   // ... when the world names at most this many selections
+    int fused_shared_max = 16384;  // ... and up to this many where blocks of several tokens share the lists (plan_small)
     int fused_small_rounds = -1;  // ... in at most this many rounds of kSmallListRound index-list entries per wave
                                   // (plan_small); -1: what measurement chose
     int last_dispatch_launches = 0;   // read-only in spirit: kernels the world's last dispatch / combine call enqueued
@@ -197,6 +203,7 @@ struct SmallPlan {
     bool fused = false;
     bool alone = false;        // dispatch_alone_kernel: every wave counts by itself; else dispatch_small_kernel
     bool could = false;        // the shared count can take it, if only because a recorded call has nothing else
+    int block_tokens = 1;      // dispatch_small_kernel: tokens of a block, which share one walk through the lists
     bool single = false;       // few enough lists that a wave counting alone could take them
 };
 SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t);

@@ -397,6 +397,17 @@ __device__ __forceinline__ int sel_stride(const UnitPlan& up, int K) {
     return 64 / kp;
 }
 
+// sum over aligned groups of `lanes` lanes (4 to 64 of them), for every lane: inside rows of 16 lanes in the DPP data path
+__device__ __forceinline__ int lanes_sum(int sum, int lanes) {
+    sum += __builtin_amdgcn_mov_dpp(sum, 0xB1, 0xF, 0xF, true);                    // quad_perm [1,0,3,2]
+    sum += __builtin_amdgcn_mov_dpp(sum, 0x4E, 0xF, 0xF, true);                    // quad_perm [2,3,0,1]
+    if (lanes >= 8) sum += __builtin_amdgcn_mov_dpp(sum, 0x141, 0xF, 0xF, true);   // row_half_mirror
+    if (lanes >= 16) sum += __builtin_amdgcn_mov_dpp(sum, 0x140, 0xF, 0xF, true);  // row_mirror
+    if (lanes >= 32) sum += __shfl_xor(sum, 16);
+    if (lanes >= 64) sum += __shfl_xor(sum, 32);
+    return sum;
+}
+
 __device__ __forceinline__ int summed_begin(const RoutingScratch& sc, const SelKey& k, const UnitPlan& up, int r, int t,
                                             int K, int j, int lps) {
     const int unit_max = r * up.per_rank + ((t * K + K - 1) >> up.shift);   // wave-uniform bound
@@ -410,14 +421,7 @@ __device__ __forceinline__ int summed_begin(const RoutingScratch& sc, const SelK
         sum += (u < k.unit ? v.x : 0) + (u + 1 < k.unit ? v.y : 0) + (u + 2 < k.unit ? v.z : 0) +
                (u + 3 < k.unit ? v.w : 0);
     }
-    // sum over the group's lanes (4 to 64 of them): inside rows of 16 lanes in the DPP data path
-    sum += __builtin_amdgcn_mov_dpp(sum, 0xB1, 0xF, 0xF, true);                  // quad_perm [1,0,3,2]
-    sum += __builtin_amdgcn_mov_dpp(sum, 0x4E, 0xF, 0xF, true);                  // quad_perm [2,3,0,1]
-    if (lps >= 8) sum += __builtin_amdgcn_mov_dpp(sum, 0x141, 0xF, 0xF, true);   // row_half_mirror
-    if (lps >= 16) sum += __builtin_amdgcn_mov_dpp(sum, 0x140, 0xF, 0xF, true);  // row_mirror
-    if (lps >= 32) sum += __shfl_xor(sum, 16);
-    if (lps >= 64) sum += __shfl_xor(sum, 32);
-    return sum;
+    return lanes_sum(sum, lps);
 }
 
 // ---------------------------------------------------------------------------
@@ -789,6 +793,14 @@ __global__ __launch_bounds__(512) void pack_bf16_kernel(const uint64_t* __restri
 // 4 x 128, 2048, top-4, bf16 7.1 -> 5.6; 1 x 384, 7168, top-8, fp8 14.1 -> 9.3.  Against count + pack + transpose, which
 // these took: 8 x 64, 4096, top-6, fp8 3.2 + 6.5 + 4.0 (and two gaps) -> 7.4; 12 ragged ranks of 70, 1152, top-5, fp8
 // 3.4 + 5.0 + 4.8 -> 8.5; 16 x 32 and 32 x 16, 7168, top-8, fp8 17 -> 12.2 and 14.6.
+// MULTI: up to hidden 4096, where a token has four waves' work at most, a block of eight (or six) waves takes several
+// consecutive tokens of a rank.  They share one walk through the lists in front of the first of them - what bounds worlds of
+// many tokens and lists is that walk, and the LDS additions of the blocks of a CU - and a token adds the selections that the
+// block's earlier tokens have: a selection is worked on by 4 to 64 lanes, which compare its expert with those entries in
+// LDS.  That step costs 0.3 to 1.3 us, so worlds of few rounds keep a token a block (plan_small).  Dispatch, us, a token
+// a block / several: 12 ragged ranks of 70, hidden 1152, top-5, fp8 7.2 / 5.9; 24 x 20, 3072, top-8, fp8 8.2 / 7.4; 1024
+// tokens of 768, top-4, hot experts 7.0 / 5.4.  Count + pack / several: 640 tokens of 2048, top-8, fp8 8.2 / 6.8; 2 x 860,
+// 1024, top-8, fp8 8.8 / 8.0, bf16 9.6 / 8.1.
 constexpr int kSmallExperts = 8;
 constexpr int kSmallSpan = 4096;                    // experts a data block counts at a time (16 KB of LDS)
 constexpr int kSmallDepth = kSmallListRound / 64;   // entries per lane and round
@@ -921,7 +933,7 @@ __device__ __forceinline__ SmallSlab small_load(const char* xtok, int s, int H, 
     return p;
 }
 
-// Where the token's selections go, lane k selection k: the payload row and (fp8) its scales' column, 0 for none.  The
+// Where the token's selections go, lane k * stride selection k: the payload row and (fp8) its scales' column, 0 for none.  The
 // slab-0 wave leaves selrow and src_info.
 struct SmallRow {
     uint64_t row = 0, srow = 0;
@@ -930,7 +942,7 @@ struct SmallRow {
 template <bool FP8>
 __device__ __forceinline__ SmallRow small_row(int32_t* selrow, uint64_t base, uint64_t info, uint64_t sbase, int K,
                                               int max_tokens, int H, int64_t RM, int r, int t, int e, int le, int slot,
-                                              bool valid, bool first_slab, int lane) {
+                                              bool valid, bool first_slab, int lane, int stride = 1) {
     const bool ok = valid && slot < RM && base != 0;
     const int64_t grow = (int64_t)le * RM + slot;
     SmallRow to;
@@ -938,29 +950,31 @@ __device__ __forceinline__ SmallRow small_row(int32_t* selrow, uint64_t base, ui
         to.row = base + (uint64_t)grow * (uint64_t)H * (FP8 ? 1 : 2);
         if (FP8) to.srow = sbase + (uint64_t)((int64_t)le * (H >> 7) * RM + slot) * 4;
     }
-    if (first_slab && lane < K) {
+    const int k = lane / stride;
+    if (first_slab && k < K && k * stride == lane) {
         // where the selection went, for a combine of this dispatch's handle: expert * R*max + row, or -1
-        selrow[((int64_t)r * max_tokens + t) * K + lane] = ok ? (int)((int64_t)e * RM + slot) : -1;
+        selrow[((int64_t)r * max_tokens + t) * K + k] = ok ? (int)((int64_t)e * RM + slot) : -1;
         if (ok) *(MCEP_GLOBAL int32_t*)(uintptr_t)(info + (uint64_t)grow * 4) = t;
     }
     return to;
 }
 
 template <bool FP8, bool NATIVE, int HINT>
-__device__ __forceinline__ void small_store(const SmallSlab& p, const SmallRow& to, int K, int H, int64_t RM, int lane) {
+__device__ __forceinline__ void small_store(const SmallSlab& p, const SmallRow& to, int K, int H, int64_t RM, int lane,
+                                            int stride = 1) {
     if (FP8) {
         float scale_inv;
         const uint4 out = quantise16<NATIVE>(p.a, p.b, &scale_inv);
         const uint64_t goff = (uint64_t)((int64_t)(p.elem0 >> 7) * RM) * 4;
         for (int k = 0; k < K; ++k) {
-            const uint64_t dst = read_lane_u64(to.row, k);
+            const uint64_t dst = read_lane_u64(to.row, k * stride);
             if (dst == 0) continue;
             if (p.act_a) store16_row<HINT>(dst, p.elem0, out, H);
-            if (p.act_a && (lane & 7) == 0) *(MCEP_GLOBAL float*)(uintptr_t)(read_lane_u64(to.srow, k) + goff) = scale_inv;
+            if (p.act_a && (lane & 7) == 0) *(MCEP_GLOBAL float*)(uintptr_t)(read_lane_u64(to.srow, k * stride) + goff) = scale_inv;
         }
     } else {
         for (int k = 0; k < K; ++k) {
-            const uint64_t dst = read_lane_u64(to.row, k);
+            const uint64_t dst = read_lane_u64(to.row, k * stride);
             if (dst == 0) continue;
             if (p.act_a) store16_row<HINT>(dst, p.elem0 * 2, p.a, H * 2);
             if (p.act_b) store16_row<HINT>(dst, p.elem0 * 2 + kSlabBytes / 2, p.b, H * 2);
@@ -968,38 +982,66 @@ __device__ __forceinline__ void small_store(const SmallSlab& p, const SmallRow& 
     }
 }
 
-template <bool FP8, bool NATIVE, int TW>
+// How the data blocks of dispatch_small_kernel are dealt out.
+struct SmallBlocks {
+    int per_rank;        // blocks of a rank
+    int tokens;          // tokens of a block (MULTI; else one)
+    int step;            // waves of a token
+    int sel_lanes;       // MULTI: lanes that work on one of a token's selections (4 to 64)
+    int step_inverse;    // 256 / step + 1: wave * step_inverse >> 8 is wave / step up to eight waves
+};
+
+template <bool MULTI, bool FP8, bool NATIVE, int TW>
 __global__ __launch_bounds__(kSmallWaves * 64) void dispatch_small_kernel(ArgTable<TW> tb, int32_t* __restrict__ selrow,
                                                                           int R, int E, int K, int max_tokens, int H,
-                                                                          int slabs, int Tgrid, int expert_blocks) {
+                                                                          int slabs, int Tgrid, int expert_blocks,
+                                                                          SmallBlocks blocks) {
     const int lane = wave_lane();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     if ((int)blockIdx.x < expert_blocks) {
         small_experts(tb.v, selrow, R, E, K, max_tokens, Tgrid, blockIdx.x * kSmallExperts, wave, waves);
         return;
     }
-    const int n = blockIdx.x - expert_blocks;
-    const int r = n / Tgrid, t = n - r * Tgrid;
+    // the block's tokens, t0 on, and the wave's among them: a wave per slab, `step` of them a token
+    const int n = blockIdx.x - expert_blocks, per_rank = MULTI ? blocks.per_rank : Tgrid;
+    const int r = n / per_rank, t0 = (n - r * per_rank) * (MULTI ? blocks.tokens : 1);
+    const int step = MULTI ? blocks.step : waves;
+    const int nth = MULTI ? (wave * blocks.step_inverse) >> 8 : 0, first_slab = wave - nth * step;
     const int T = (int)tb.v[DF_NUM_TOKENS * R + r];
     const uint64_t own_list = tb.v[DF_TOPK_IDX * R + r], own_x = tb.v[DF_X * R + r];
     asm volatile("" ::"s"(T), "s"(own_list), "s"(own_x));         // (one wait for the three)
-    if (t >= T) return;                                           // the whole block
+    if (t0 >= T) return;                                          // the whole block
+    const bool live = !MULTI || t0 + nth < T;                     // else the wave has no token and counts only
+    const int t = live ? t0 + nth : t0;
     const char* xtok = (const char*)own_x + (int64_t)t * H * 2;
 
     // the payload loads first: everything below hides behind them
-    SmallSlab slab = small_load<FP8>(xtok, wave, H, lane);
+    SmallSlab slab = small_load<FP8>(xtok, first_slab, H, lane);
 
-    // the token's K experts, one per lane, and the first round of the lists in front of it
-    const int li = lane < K ? lane : 0;
+    // the token's K experts, one per lane (MULTI: one per `stride` lanes), the entries of all the block's tokens (wave 0),
+    // and the first round of the lists in front of the block
+    const int stride = MULTI ? blocks.sel_lanes : 1, sel = lane / stride;
+    const int li = sel < K ? sel : 0;
     const int64_t e64 = *(const MCEP_GLOBAL int64_t*)(uintptr_t)(own_list + (uint64_t)((int64_t)t * K + li) * 8);
-    const auto lists = [&] { return ListWalk(tb.v, own_list, R, K, r, t * K, Tgrid * K, waves, wave); };
+    constexpr int kOwn = MULTI ? kSmallWaves * kMaxTopK / 64 : 1;
+    __shared__ int lds_own[kOwn * 64];
+    int64_t own[kOwn];
+    if (MULTI && wave == 0) {
+        const int own_n = (T - t0 < blocks.tokens ? T - t0 : blocks.tokens) * K;
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) {
+            const int at = i * 64 + lane;
+            own[i] = *(const MCEP_GLOBAL int64_t*)(uintptr_t)(own_list + (uint64_t)((int64_t)t0 * K + (at < own_n ? at : 0)) * 8);
+        }
+    }
+    const auto lists = [&] { return ListWalk(tb.v, own_list, R, K, r, t0 * K, Tgrid * K, waves, wave); };
     ListWalk walk = lists();
     int64_t v[2][kSmallDepth];
     int whose = 0, n_round[2];
     bool go = walk.more();
     n_round[0] = walk.fetch(v[0], &whose);
 
-    const bool valid = lane < K && (uint64_t)e64 < (uint64_t)E;
+    const bool valid = sel < K && (uint64_t)e64 < (uint64_t)E;
     const int e = valid ? (int)e64 : 0;
     const int L = E / R, q = e / L, le = e - q * L;
     // the owner's tensors: asked for as soon as the expert is known, needed after the count
@@ -1023,6 +1065,10 @@ __global__ __launch_bounds__(kSmallWaves * 64) void dispatch_small_kernel(ArgTab
                 if (!take(0)) break;
                 if (!take(1)) break;
             }
+        if (MULTI && wave == 0 && first == 0) {
+#pragma unroll
+            for (int i = 0; i < kOwn; ++i) lds_own[i * 64 + lane] = (uint64_t)own[i] < (uint64_t)E ? (int)own[i] : -1;
+        }
         __syncthreads();
         if (valid && e >= first && e - first < span) slot = lds_hist[e - first];
         first += span;
@@ -1035,16 +1081,27 @@ __global__ __launch_bounds__(kSmallWaves * 64) void dispatch_small_kernel(ArgTab
         n_round[0] = walk.fetch(v[0], &whose);
         __syncthreads();                                          // this span has been read
     }
-    // plus the token's own earlier selections of the same expert (a repeated expert gets a row per occurrence)
-    for (int k = 0; k + 1 < K; ++k) {
-        const int earlier = __builtin_amdgcn_readlane(valid ? e : -1, k);
-        if (lane > k && earlier == e) slot += 1;
+    // plus the selections of the same expert that the token itself (a repeated expert gets a row per occurrence) and the
+    // block's earlier tokens have in front
+    if constexpr (MULTI) {
+        int found = 0;
+        const int before = sel < K ? nth * K + sel : 0;
+#pragma clang loop unroll(disable)
+        for (int i = lane - sel * stride; i < before; i += stride) found += lds_own[i] == e ? 1 : 0;
+        slot += lanes_sum(found, stride);
+    } else {
+        for (int k = 0; k + 1 < K; ++k) {
+            const int earlier = __builtin_amdgcn_readlane(valid ? e : -1, k);
+            if (lane > k && earlier == e) slot += 1;
+        }
     }
+    if (!live) return;                                            // (behind the last barrier)
     const int64_t RM = (int64_t)R * max_tokens;
-    const SmallRow to = small_row<FP8>(selrow, base, info, sbase, K, max_tokens, H, RM, r, t, e, le, slot, valid, wave == 0, lane);
-    for (int s = wave; s < slabs; s += waves) {                  // (once, unless hidden is above 8192)
-        if (s != wave) slab = small_load<FP8>(xtok, s, H, lane);
-        small_store<FP8, NATIVE, kStoreThrough>(slab, to, K, H, RM, lane);
+    const SmallRow to = small_row<FP8>(selrow, base, info, sbase, K, max_tokens, H, RM, r, t, e, le, slot, valid,
+                                       first_slab == 0, lane, stride);
+    for (int s = first_slab; s < slabs; s += step) {             // (once, unless hidden is above 8192)
+        if (s != first_slab) slab = small_load<FP8>(xtok, s, H, lane);
+        small_store<FP8, NATIVE, kStoreThrough>(slab, to, K, H, RM, lane, stride);
     }
 }
 
@@ -2221,20 +2278,28 @@ hipError_t launch_dispatch_small(const SmallTable& tb, int32_t* d_selrow, const 
     }
     const int slabs = (d.H + 1023) / 1024;
     const int expert_blocks = (d.E + kSmallExperts - 1) / kSmallExperts;
-    const long long total = (long long)expert_blocks + (long long)d.R * d.Tgrid;
+    const int step = slabs < kSmallWaves ? slabs : kSmallWaves;
+    const int tokens = d.block_tokens;
+    const bool multi = tokens > 1;
+    if (multi && tokens != small_block_tokens(d.H)) return hipErrorInvalidValue;
+    const int slots = d.K <= 1 ? 1 : (d.K <= 2 ? 2 : (d.K <= 4 ? 4 : (d.K <= 8 ? 8 : 16)));
+    const SmallBlocks deal{(d.Tgrid + tokens - 1) / tokens, tokens, step, 64 / slots, 256 / step + 1};
+    const long long total = (long long)expert_blocks + (long long)d.R * deal.per_rank;
     if (total > 0x7fffffffll) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)total), block(small_block_waves(d.H) * 64);
+    const dim3 grid((unsigned)total), block((multi ? step * tokens : small_block_waves(d.H)) * 64);
     const size_t lds = (size_t)(d.E < kSmallSpan ? d.E : kSmallSpan) * sizeof(int);
     // (the fewer argument bytes the cheaper the launch, as for the count kernel)
     constexpr int kFew = (int)DF_COUNT * 8, kMany = (int)DF_COUNT * kSmallRanks;
     const int words = (int)DF_COUNT * d.R;
-#define MCEP_SMALL_TABLE(FP8, NATIVE, TW)                                                                              \
-    hipLaunchKernelGGL((dispatch_small_kernel<FP8, NATIVE, TW>), grid, block, lds, stream, arg_table<TW>(tb.v, words), \
-                       d_selrow, d.R, d.E, d.K, d.max_tokens, d.H, slabs, d.Tgrid, expert_blocks)
-#define MCEP_SMALL(FP8, NATIVE)                                 \
-    do {                                                        \
-        if (words <= kFew) MCEP_SMALL_TABLE(FP8, NATIVE, kFew); \
-        else MCEP_SMALL_TABLE(FP8, NATIVE, kMany);              \
+#define MCEP_SMALL_TABLE(MULTI, FP8, NATIVE, TW)                                                                       \
+    hipLaunchKernelGGL((dispatch_small_kernel<MULTI, FP8, NATIVE, TW>), grid, block, lds, stream, arg_table<TW>(tb.v, words), \
+                       d_selrow, d.R, d.E, d.K, d.max_tokens, d.H, slabs, d.Tgrid, expert_blocks, deal)
+#define MCEP_SMALL(FP8, NATIVE)                                                \
+    do {                                                                       \
+        if (multi && words <= kFew) MCEP_SMALL_TABLE(true, FP8, NATIVE, kFew); \
+        else if (multi) MCEP_SMALL_TABLE(true, FP8, NATIVE, kMany);            \
+        else if (words <= kFew) MCEP_SMALL_TABLE(false, FP8, NATIVE, kFew);    \
+        else MCEP_SMALL_TABLE(false, FP8, NATIVE, kMany);                      \
     } while (0)
     if (!use_fp8) MCEP_SMALL(false, false);
     else if (t.fp8_arith == 1) MCEP_SMALL(true, true);

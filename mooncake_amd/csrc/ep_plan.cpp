@@ -53,8 +53,27 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
         if (num_tokens[r] > most) most = num_tokens[r];
     }
     SmallPlan p;
-    if (t.fused_small == 0 || most == 0 || tokens * K > (long long)t.fused_small_max) return p;
+    if (t.fused_small == 0 || most == 0) return p;
     const bool chosen = t.fused_small_rounds >= 0;      // the option replaces the measured lines
+    const long long walked = (long long)R * (((long long)most * K + kSmallListRound - 1) / kSmallListRound);
+    const int together = small_block_tokens(hidden);
+    if (tokens * K > (long long)t.fused_small_max) {
+        // Too many for a token a block.  Up to hidden 4096 several tokens share one: the lists are read that many times
+        // less, by eight waves.  Priced by the rounds of all blocks together.  Dispatch, us, apart / in one: fp8, 640
+        // tokens of hidden 2048, top-8 (1600) 8.2 / 6.8, 16 x 112, 1024, top-4 (3584) 7.6 / 6.7, 4 x 256, 2048, top-8 (4096)
+        // 9.3 / 8.9, 1020, 3072, top-5 (5100) 9.5 / 8.3, 2 x 860, 1024, top-8 (6020) 8.8 / 7.9; (8192) 2048, 1024, top-8
+        // 9.2 / 10.3, 8 x 128, 4096 13.1 / 12.6, 4096, 1024, top-2 8.8 / 14.9; (14256) 9.6 / 10.6.  bf16 8.4 / 6.8, 7.5 / 6.4,
+        // 10.7 / 8.8, 10.0 / 8.5, 9.5 / 8.1; 10.3 / 10.0, 14.8 / 13.1, 8.0 / 13.6; 10.2 / 10.2.  Not top-1 and top-2, whose
+        // selections may all name one expert and then queue for its counter.
+        const bool pays = tokens * K > 4096 && tokens * K <= (long long)t.fused_shared_max && !chosen && K > 2 &&
+                          hidden > 512 && together > 1 && R <= kSmallRanks && walked <= 4 * kSmallWaves &&
+                          tokens * walked <= 6144ll * together;
+        if (pays) {
+            p.fused = p.could = true;
+            p.block_tokens = together;
+        }
+        return p;
+    }
     const long long limit = chosen ? t.fused_small_rounds : (use_fp8 ? 6 : 4);
     const int waves = small_block_waves(hidden);
     p.single = R <= kSmallWaveRanks && lists <= limit;
@@ -82,10 +101,14 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
     // top-2, 2048 tokens (16384) 11.4 / 10.1 and 16.0 / 12.4, bf16 8.1 / 9.6 and 13.6 / 12.9, with one hot expert in eight
     // 11.5 / 13.1, 8.4 / 12.4; top-1, 4096 tokens (32768) 12.5 / 15.1 and 19.6 / 18.3, hot 12.8 / 33.3.  Rows of half a slab
     // and less have not been measured over that range, and stay with the separate launches.
-    const long long walked = (long long)R * (((long long)most * K + kSmallListRound - 1) / kSmallListRound);
     p.could = hidden > 512 && R <= kSmallRanks && R <= kSmallWaveRanks * waves && (lists + waves - 1) / waves <= limit;
     p.fused = hidden > 512 && R <= kSmallRanks && R <= kSmallWaveRanks * waves &&
               (walked + waves - 1) / waves <= limit && (chosen || tokens * walked <= (use_fp8 ? 16384 : 8192));
+    // Several tokens a block, where the blocks' reading of the lists is what takes the time.  One token a block / several,
+    // us, by rounds of all tokens: 12 ragged ranks of 70, hidden 1152, top-5 (10080) 7.3 / 5.9; 24 x 20, 3072, top-8 (11520)
+    // 8.3 / 7.4; 16 x 32, 2048, bf16 (8192) 7.5 / 6.9; 1024 tokens of 768, top-4 (8192) 7.1 / 5.4; but 8 x 64, 4096, top-6
+    // (4096) 6.9 / 7.1, 4 x 128, 2048, top-4, bf16 (2048) 4.9 / 5.3: the others' selections in the block are a step more.
+    if (tokens * walked >= 6144) p.block_tokens = together;
     return p;
 }
 

@@ -561,6 +561,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     if (!static_scratch && (phases & MC_EP_PHASE_LAYOUT) && w->unfinished)
         if (int rc = finish_round(w, w->unfinished.get())) return rc;
     Dims d{R, num_experts, num_topk, hidden, max_tokens, tgrid};
+    d.block_tokens = small.block_tokens;
     plan_units(d, w->tuning);
     // The count kernel keeps per-wave counts and prefixes of every expert in LDS.  A world whose lists a wave could count
     // alone needs none of it; any other one has to fit, also where the rule above happens to give it one launch.
@@ -1231,6 +1232,7 @@ static int* option_slot(Tuning& t, const char* name) {
     if (!strcmp(name, "last_combine_launches")) return &t.last_combine_launches;
     if (!strcmp(name, "fused_small")) return &t.fused_small;
     if (!strcmp(name, "fused_small_max")) return &t.fused_small_max;
+    if (!strcmp(name, "fused_shared_max")) return &t.fused_shared_max;
     if (!strcmp(name, "fused_small_rounds")) return &t.fused_small_rounds;
     if (!strcmp(name, "blocking")) return &t.blocking;
     if (!strcmp(name, "block_timeout_ms")) return &t.block_timeout_ms;

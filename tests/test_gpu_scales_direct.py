@@ -32,7 +32,7 @@ def test_scales_in_place(gpu_device, oracle, cfg, launches, plan, arith):
     data = generate(cfg, seed=17)
     if K > 1:
         data["topk_idx"][0, ::5, K - 1] = data["topk_idx"][0, ::5, 0]     # a repeated expert has a row per occurrence
-    h = run_dispatch(cfg, data, num_tokens=nt, poison=True, options={"routing_sum": plan, "fp8_arith": arith})
+    h = run_dispatch(cfg, data, num_tokens=nt, poison=True, options={"routing_sum": plan, "fp8_arith": arith, "fused_small": 0})
     oracle.set_fp8_arith(arith)
     try:
         ref = oracle.dispatch(data["x"], data["topk_idx"], nt, cfg.max_tokens, cfg.num_experts, True)
@@ -63,7 +63,7 @@ def test_scales_in_place_of_a_silent_rank_and_by_option(gpu_device, oracle, noal
     got = []
     for direct in (1, 0):
         announce(f"scales in place: a silent rank, noalloc={noalloc} direct={direct}")
-        h = run_dispatch(cfg, data, poison=True, present=[1, 0, 1], options={"scales_direct": direct})
+        h = run_dispatch(cfg, data, poison=True, present=[1, 0, 1], options={"scales_direct": direct, "fused_small": 0})
         if noalloc:
             h.recv_scales_phys.fill_(float("nan"))
             h.dispatch(present=[1, 0, 1], noalloc=True)
