@@ -109,7 +109,7 @@ struct RoutingScratch {
     int32_t* selrow;     // [R * max_tokens * K]  expert * R*max + packed row of the selection, -1: none; left by the
                          //                       pack kernel for a combine of the same handle
     int32_t* counts;     // [E]     rows per expert (0 for experts of ranks that take no part)
-    int32_t* row_src;    // [E, R * max_tokens]  packed row -> source token slot (rank * max_tokens + token)
+    int32_t* row_src;    // [E, R * max_tokens]  packed row -> source token slot (rank * max_tokens + token); fp8 only
 };
 
 // One resolved source row of combine's general path (a handle that is not the

@@ -74,3 +74,39 @@ def test_size_rule_of_shared_blocks(gpu_device, oracle):
         assert h.world.get_option("last_dispatch_launches") == launches, (cfg, options)
         ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, True)
         compare_dispatch(h, ref, check_poison=True)
+
+
+def test_recorded_shared_blocks_replay(gpu_device, oracle):
+    """The one launch for thousands of selections in a graph: replays on fresh inputs, with eager calls in between."""
+    from mooncake_amd import ep
+    from mooncake_amd.harness import WorldHarness
+
+    cfg = EPConfig("recorded", 2, 300, 2048, 16, 8, True)
+    announce(f"one-launch dispatch, several tokens a block, recorded {cfg}")
+    h = WorldHarness(cfg, world=ep.World(2))
+    h.load(generate(cfg, seed=85))
+    h.alloc_dispatch_outputs()
+    h.alloc_combine_io()
+    h.expert_out.normal_()
+    h.dispatch()
+    h.combine()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        h.dispatch()
+        h.combine()
+    assert h.world.get_option("last_dispatch_launches") == 1
+    for seed in (86, 87, 88):
+        data = generate(cfg, seed=seed)
+        h.x.copy_(data["x"])
+        h.topk_idx.copy_(data["topk_idx"])
+        h.topk_weights.copy_(data["topk_weights"])
+        g.replay()
+        torch.cuda.synchronize()
+        ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, True)
+        compare_dispatch(h, ref, check_poison=False)
+        want = oracle.combine(h.expert_out.cpu(), data["topk_idx"], data["topk_weights"], ref["src_info"],
+                              ref["layout_range"], h.num_tokens, cfg.max_tokens, cfg.num_experts)
+        assert torch.equal(h.combined.cpu().view(torch.int16), want.view(torch.int16)), seed
+        h.dispatch()
+        torch.cuda.synchronize()
