@@ -63,9 +63,13 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
         // tokens of hidden 2048, top-8 (1600) 8.2 / 6.8, 16 x 112, 1024, top-4 (3584) 7.6 / 6.7, 4 x 256, 2048, top-8 (4096)
         // 9.3 / 8.9, 1020, 3072, top-5 (5100) 9.5 / 8.3, 2 x 860, 1024, top-8 (6020) 8.8 / 7.9; (8192) 2048, 1024, top-8
         // 9.2 / 10.3, 8 x 128, 4096 13.1 / 12.6, 4096, 1024, top-2 8.8 / 14.9; (14256) 9.6 / 10.6.  bf16 8.4 / 6.8, 7.5 / 6.4,
-        // 10.7 / 8.8, 10.0 / 8.5, 9.5 / 8.1; 10.3 / 10.0, 14.8 / 13.1, 8.0 / 13.6; 10.2 / 10.2.  Not top-1 and top-2, whose
-        // selections may all name one expert and then queue for its counter.
+        // 10.7 / 8.8, 10.0 / 8.5, 9.5 / 8.1; 10.3 / 10.0, 14.8 / 13.1, 8.0 / 13.6; 10.2 / 10.2.  Every token naming the same
+        // experts, or nine in ten an eighth of them, gains as much from top-3 up (2000, 640, top-3 of 3: fp8 9.8 / 6.1, bf16
+        // 6.8 / 5.8); not top-1 and top-2, whose selections may all name one expert and queue for its counter.  Many
+        // selections are many in the block too: bf16, 500, 1024, top-9 7.0 / 6.4, 8 x 80, 640, top-11 7.2 / 7.1, but
+        // 2 x 250, 1024, top-16 8.1 / 8.6 (fp8, with two launches saved, 10.2 / 8.9).
         const bool pays = tokens * K > 4096 && tokens * K <= (long long)t.fused_shared_max && !chosen && K > 2 &&
+                          (use_fp8 || K <= 12) &&
                           hidden > 512 && together > 1 && R <= kSmallRanks && walked <= 4 * kSmallWaves &&
                           tokens * walked <= 6144ll * together;
         if (pays) {
@@ -107,8 +111,9 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
     // Several tokens a block, where the blocks' reading of the lists is what takes the time.  One token a block / several,
     // us, by rounds of all tokens: 12 ragged ranks of 70, hidden 1152, top-5 (10080) 7.3 / 5.9; 24 x 20, 3072, top-8 (11520)
     // 8.3 / 7.4; 16 x 32, 2048, bf16 (8192) 7.5 / 6.9; 1024 tokens of 768, top-4 (8192) 7.1 / 5.4; but 8 x 64, 4096, top-6
-    // (4096) 6.9 / 7.1, 4 x 128, 2048, top-4, bf16 (2048) 4.9 / 5.3: the others' selections in the block are a step more.
-    if (tokens * walked >= 6144) p.block_tokens = together;
+    // (4096) 6.9 / 7.1, 4 x 128, 2048, top-4, bf16 (2048) 4.9 / 5.3: the others' selections in the block are a step more, and
+    // a longer one above top-8: 16 x 24, 1024, top-9 (6144) 6.8 / 7.2, 24 x 12, 1024, top-11 (6912) 7.9 / 7.9.
+    if (tokens * walked >= (K <= 8 ? 6144 : 8192)) p.block_tokens = together;
     return p;
 }
 

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     EPConfig("eight_k8", 1, 600, 1024, 16, 8, True),                       # 4800 selections, one list
-    EPConfig("eight_k16", 2, 150, 640, 32, 16, False, routing="zipf"),     # 128 entries in a block
+    EPConfig("eight_k16", 2, 150, 640, 32, 16, True, routing="zipf"),      # 128 entries in a block
     EPConfig("four_k9", 4, 124, 1152, 36, 9, True, masked_fraction=0.2),   # 4464
     EPConfig("four_k3", 12, 117, 2048, 24, 3, False, routing="zipf"),      # 4212
     EPConfig("two_of_three", 2, 300, 2944, 18, 8, True),                   # six waves
