@@ -10,7 +10,9 @@
 // Buffer.dispatch_tensors and combine_tensors are the exception: the reference wrapper's
 // checks, its outputs and the call itself in one native step, for the Python `Buffer`
 // above (a rank's dispatch took 4.1 us of host time through Python and a combine 5.2,
-// nearly all of it tensor attributes, torch.empty and the pool's look-up).
+// nearly all of it tensor attributes, torch.empty and the pool's look-up).  So are
+// World.dispatch_stacked, combine_stacked and cast_back_stacked, which read the ranks'
+// addresses off one tensor per argument.
 //
 // What the reference does not have: World (the expert-parallel world as logical ranks
 // of one GPU; Buffer takes the one it belongs to as an optional fifth argument and
@@ -460,7 +462,7 @@ struct PreparedCombine {
 // Python costs 0.4 us to learn, is the first one's plus r strides.  Everything is read off the tensors at each call and
 // nothing kept.  A call answers false, having done nothing, where an argument is neither None nor a plain torch.Tensor (or
 // Parameter; another subclass may have its own idea of indexing): the caller then marshals it in Python.
-// Host time of a call, us (the box's CPU runs at one of two speeds): 4 ranks, dispatch and combine 5.2 to 6.1 -> 4.0 to 4.9
+// Host time of a call, us (of two speeds that one host ran at): 4 ranks, dispatch and combine 5.2 to 6.1 -> 4.0 to 4.9
 // (keyed and looked up in Python before), cast back 16 to 17 -> 4.5 to 5.8 (a slice per rank and tensor before); 32 ranks,
 // dispatch 10.7 to 12.9 -> 7.3 to 9.9, combine 5.8 to 7.2 -> 4.7 to 6.5, cast back 120 -> 4.8 to 6.6.
 class Stacked {
