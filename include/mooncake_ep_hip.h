@@ -53,8 +53,11 @@ extern "C" {
 
 /* phases of a whole-world call (the reference's LOW_LATENCY_SEND_PHASE /
  * LOW_LATENCY_RECV_PHASE split, mooncake_ep_configs.cuh:16-17, maps onto the
- * kernels each call is made of; a later phase needs the earlier ones of the
- * same call to have run) */
+ * kernels each call is made of.  A later phase goes on from what the earlier
+ * ones of the same call - same shape, tensors and token counts - left in the
+ * world; where the world holds none of that, because another dispatch has run
+ * since or an all-phases call took one launch, a dispatch launches the earlier
+ * phases with it, from the tensors it is given) */
 #define MC_EP_PHASE_LAYOUT 1   /* dispatch: routing counts;  combine: handle -> row resolve */
 #define MC_EP_PHASE_DATA 2     /* dispatch: pack (packed_recv_count / src_info / layout_range are complete after
                                   this phase, not before); combine: weighted reduce */

@@ -667,7 +667,8 @@ __device__ __forceinline__ uint4 quantise16(uint4 a, uint4 b, float* scale_inv) 
 //   SCALES  where the world has few scales (scales_direct) they go into the output
 //           from here all the same, a launch of 5 us less: 640 tokens of hidden
 //           1024, top-8, 9.8 -> 7.5 us the dispatch, 2 x 858 11.0 -> 9.0.  The staging
-//           row is written too (0.15 us): the last phase may be asked for again.
+//           row is written too (0.15 us): the last phase may be asked for again.  (After the
+//           one-launch dispatch, which stages nothing, the runtime makes the whole call again.)
 //   NATIVE  which of the reference's two statements of the scale arithmetic (see quantise16)
 template <bool SCALES, bool NTL, bool NATIVE, int HINT>
 __global__ __launch_bounds__(512) void pack_fp8_kernel(const uint64_t* __restrict__ tbl,

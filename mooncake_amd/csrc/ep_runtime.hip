@@ -242,14 +242,22 @@ struct mc_ep_world {
     size_t counts_cap = 0;
     uint32_t* d_chunk_map = nullptr;     // work list of the cast-back kernel (many experts), 4 words per entry
     size_t chunk_map_cap = 0;
+    bool one_launch_captured = false;                    // ... one that takes the one launch
+    bool phases_captured = false;                        // a graph goes on from what a dispatch outside it left
     // what the last dispatch was called with, so that a combine given that
-    // dispatch's handle can reuse its routing state instead of re-deriving rows
+    // dispatch's handle can reuse its routing state instead of re-deriving rows,
+    // and a later phase called by itself knows whether the scratch is its own
     struct LastDispatch {
         bool valid = false;
         int hidden = 0, num_topk = 0, max_tokens = 0, num_experts = 0;
+        bool use_fp8 = false;
+        UnitPlan plan;
         std::vector<uint64_t> topk_idx, recv_x, src_info, layout_range;
         std::vector<int32_t> num_tokens;
         bool data_done = false;                   // its pack phase has been launched too (and did not fail)
+        bool counted = false;                     // the scratch holds its counts and positions (not after the one launch)
+        bool staged = false;                      // ... and its staged scales and row sources
+        bool finished = false;                    // every phase of it has been launched
         bool captured = false;                    // recorded into a graph, and which capture
         unsigned long long capture_id = 0;
     } last;
@@ -511,11 +519,36 @@ int order_begin(mc_ep_world* w, hipStream_t stream, const Capture& cap) {
     return MC_EP_OK;
 }
 
+// The phases that a dispatch of `phases` has to launch.  A later phase goes on from what the world's scratch holds; where
+// that is not this call's - another dispatch of the world has run since, or the one launch, which leaves no such state - the
+// phases in front of it run with it, from the call's own tensors.  Graph replays run dispatches the host never sees: once a
+// one-launch dispatch of the world lives in a graph, what a call left that is complete may be older than the last replay.
+int phases_needed(mc_ep_world* w, const Dims& d, const uint64_t* topk_idx, const int32_t* num_tokens, bool use_fp8,
+                  const uint64_t* recv_x, int phases, const Capture& cap) {
+    const bool finish = use_fp8 && (phases & MC_EP_PHASE_FINISH);       // (a bf16 dispatch has no last phase)
+    if (!(phases & MC_EP_PHASE_DATA) && !finish) return phases;
+    const auto& ld = w->last;
+    const bool same_capture = cap.active && ld.captured && ld.capture_id == cap.id;
+    // (an allocation-free dispatch has scratch of its own: phases that it came in between go on)
+    bool own = ld.counted && (ld.valid || !ld.finished) && ld.hidden == d.H && ld.num_topk == d.K && ld.max_tokens == d.max_tokens &&
+               ld.num_experts == d.E && ld.use_fp8 == use_fp8 && ld.plan.per_rank == d.plan.per_rank &&
+               ld.plan.shift == d.plan.shift && ld.plan.summed == d.plan.summed && ld.plan.carried == d.plan.carried &&
+               !(w->one_launch_captured && ld.finished && !same_capture);
+    for (int r = 0; r < d.R && own; ++r)
+        own = topk_idx[r] == ld.topk_idx[r] && num_tokens[r] == ld.num_tokens[r] && recv_x[r] == ld.recv_x[r];
+    const bool counts_again = (phases & MC_EP_PHASE_LAYOUT) || !own;
+    if (finish && (counts_again || !ld.staged)) phases |= MC_EP_PHASE_DATA;
+    if (counts_again) return phases | MC_EP_PHASE_LAYOUT;
+    // such a graph depends on the dispatches that run in front of its replays: those may not take the one launch any more
+    if (cap.active && !same_capture) w->phases_captured = true;
+    return phases;
+}
+
 int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_idx, const int32_t* num_tokens,
                         int hidden, int num_topk, int max_tokens, int num_experts, int use_fp8,
                         const uint64_t* recv_x, const uint64_t* recv_scales, const uint64_t* recv_count,
                         const uint64_t* src_info, const uint64_t* layout_range, int phases, hipStream_t stream,
-                        bool static_scratch = false) {
+                        bool static_scratch = false, bool second_part = false) {
     const int R = w->R;
     if (int rc = check_dims(w, hidden, num_topk, max_tokens, num_experts)) return rc;
     MC_ASSERT(x != nullptr && topk_idx != nullptr && num_tokens != nullptr);
@@ -545,11 +578,19 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         tbl[DF_NUM_TOKENS * R + r] = (uint64_t)num_tokens[r];
         if (num_tokens[r] > tgrid) tgrid = num_tokens[r];
     }
+    Dims d{R, num_experts, num_topk, hidden, max_tokens, tgrid};
+    plan_units(d, w->tuning);
+    // (a round's second part is enqueued before anything touches what its first one left)
+    if (!second_part && phases != MC_EP_PHASE_ALL) {
+        Capture cap;
+        if (int rc = capture_of(stream, &cap)) return rc;
+        phases = phases_needed(w, d, topk_idx, num_tokens, use_fp8 != 0, recv_x, phases, cap);
+    }
     // A world that names few selections is dispatched in one launch, which rebuilds the routing it needs from the index
     // lists (dispatch_small_kernel, dispatch_alone_kernel); the rank table then travels in kernel arguments.
     const SmallPlan small = phases == MC_EP_PHASE_ALL ? plan_small(num_tokens, R, num_topk, hidden, use_fp8 != 0, w->tuning)
                                                       : SmallPlan{};
-    bool fused = small.fused;
+    bool fused = small.fused && (small.single || !w->phases_captured);
     DeviceGuard guard(w->device);
     w->launches = 0;
     struct Tally {                                // the option "last_dispatch_launches", on every way out
@@ -560,9 +601,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     // that still waits for its hook has to be enqueued first
     if (!static_scratch && (phases & MC_EP_PHASE_LAYOUT) && w->unfinished)
         if (int rc = finish_round(w, w->unfinished.get())) return rc;
-    Dims d{R, num_experts, num_topk, hidden, max_tokens, tgrid};
     d.block_tokens = small.block_tokens;
-    plan_units(d, w->tuning);
     // The count kernel keeps per-wave counts and prefixes of every expert in LDS.  A world whose lists a wave could count
     // alone needs none of it; any other one has to fit, also where the rule above happens to give it one launch.
     const bool single = fused && small.single;
@@ -618,6 +657,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
             fused = w->ucount_cap < UE || w->ubegin_cap < UE || w->ucount_t_cap < (size_t)num_experts * kMaxSummedUnits ||
                     w->selpos_cap < (size_t)R * max_tokens * num_topk || w->counts_cap < (size_t)num_experts ||
                     w->row_src_cap < (size_t)num_experts * R * max_tokens || w->scale_stage_cap < stage_floats;
+        if (phases & MC_EP_PHASE_LAYOUT) w->last.counted = false;       // until its launch has succeeded
         // (two entries at least: dispatch_small_kernel may read 8 bytes there)
         if (int rc = ensure_scratch(w, &w->d_selrow, &w->selrow_cap, (size_t)R * max_tokens * num_topk + 1)) return rc;
         // The one-launch dispatch keeps no routing state but selrow.  An eager one prepares the world for the separate
@@ -653,9 +693,11 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         sc = routing_scratch(w);
     }
     // what a combine has to know to recognise this dispatch's handle (see mc_ep_world::LastDispatch)
-    auto remember = [&](bool data_done) {
+    auto remember = [&](bool one_launch) {
         auto& ld = w->last;
         ld.valid = true;
+        ld.use_fp8 = use_fp8 != 0;
+        ld.plan = d.plan;
         ld.hidden = hidden; ld.num_topk = num_topk; ld.max_tokens = max_tokens; ld.num_experts = num_experts;
         ld.topk_idx.assign(topk_idx, topk_idx + R);
         ld.recv_x.assign(recv_x, recv_x + R);
@@ -664,8 +706,11 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         ld.num_tokens.assign(num_tokens, num_tokens + R);
         ld.captured = cap.active;
         ld.capture_id = cap.id;
-        ld.data_done = data_done;
+        ld.data_done = ld.finished = one_launch;
+        ld.counted = !one_launch;
+        ld.staged = false;
         if (cap.active) w->dispatch_captured = true;
+        if (cap.active && one_launch) w->one_launch_captured = true;
     };
     if (fused) {
         SmallTable st{};
@@ -696,7 +741,11 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     }
     // under the carried plan the pack launch also produces ubegin and the counts: only now is the
     // routing state complete for a combine to reuse
-    if (!static_scratch && (phases & MC_EP_PHASE_DATA)) w->last.data_done = true;
+    if (!static_scratch && (phases & MC_EP_PHASE_DATA)) {
+        w->last.data_done = true;
+        w->last.staged = use_fp8 != 0;
+    }
+    if (!static_scratch && (use_fp8 ? (phases & MC_EP_PHASE_FINISH) : (phases & MC_EP_PHASE_DATA))) w->last.finished = true;
     return MC_EP_OK;
 }
 
@@ -980,7 +1029,7 @@ int launch_dispatch_round(mc_ep_world* w, PendingRound<DispatchPost>& pr) {
         DeviceGuard g(w->device);
         if (int e = world_dispatch_impl(w, x.data(), idx.data(), nt.data(), hidden, num_topk, max_tokens, num_experts,
                                         use_fp8, rx.data(), rs.data(), rc.data(), si.data(), lr.data(),
-                                        MC_EP_PHASE_FINISH, launch))
+                                        MC_EP_PHASE_FINISH, launch, false, true))
             return e;
         if (round->done) MC_HIP(hipEventRecord(round->done, launch));
         round->waited.assign(1, launch);

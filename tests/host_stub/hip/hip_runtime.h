@@ -54,6 +54,7 @@ inline std::atomic<long> g_calls{0};          // API calls of any kind
 inline std::atomic<long> g_live_events{0};    // created and not yet destroyed
 inline std::atomic<long> g_live_streams{0};
 inline std::atomic<long> g_live_allocs{0};
+inline std::atomic<unsigned long long> g_capture{0};   // 0, or the capture that every stream but the null one is in
 inline ihipStream_t g_null_stream;
 inline ihipStream_t* resolve(hipStream_t s) { return s ? s : &g_null_stream; }
 inline void touch() { g_calls.fetch_add(1, std::memory_order_relaxed); }
@@ -103,8 +104,9 @@ inline hipError_t hipStreamQuery(hipStream_t s) {
 }
 inline hipError_t hipStreamGetCaptureInfo(hipStream_t, hipStreamCaptureStatus* status, unsigned long long* id) {
     hip_stub::touch();
-    *status = hipStreamCaptureStatusNone;
-    if (id) *id = 0;
+    const unsigned long long capture = hip_stub::g_capture.load(std::memory_order_relaxed);
+    *status = capture ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    if (id) *id = capture;
     return hipSuccess;
 }
 inline hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { hip_stub::touch(); return hipSuccess; }

@@ -6,6 +6,8 @@
 namespace mcep {
 
 std::atomic<long> g_stub_launches{0};
+// the parts of a dispatch, each by itself (tests/host_stub/phases_driver.cpp)
+std::atomic<long> g_stub_counts{0}, g_stub_packs{0}, g_stub_finishes{0}, g_stub_one_launch{0};
 
 static hipError_t launched(hipStream_t stream) {
     g_stub_launches.fetch_add(1, std::memory_order_relaxed);
@@ -15,13 +17,17 @@ static hipError_t launched(hipStream_t stream) {
 
 hipError_t launch_table_write(uint64_t*, const uint64_t*, int, hipStream_t s) { return launched(s); }
 hipError_t launch_count(const uint64_t*, const RoutingScratch&, const DispatchSource&, const Dims&, hipStream_t s) {
+    g_stub_counts.fetch_add(1, std::memory_order_relaxed);
     return launched(s);
 }
 hipError_t launch_pack(const uint64_t*, const RoutingScratch&, const DispatchSource&, float*, const Dims&, bool,
-                       const Tuning&, bool, bool, hipStream_t s) {
+                       const Tuning&, bool run_pack, bool run_finish, hipStream_t s) {
+    g_stub_packs.fetch_add(run_pack ? 1 : 0, std::memory_order_relaxed);
+    g_stub_finishes.fetch_add(run_finish ? 1 : 0, std::memory_order_relaxed);
     return launched(s);
 }
 hipError_t launch_dispatch_small(const SmallTable&, int32_t*, const Dims&, bool, bool, const Tuning&, hipStream_t s) {
+    g_stub_one_launch.fetch_add(1, std::memory_order_relaxed);
     return launched(s);
 }
 hipError_t launch_resolve(const uint64_t*, CombineRoute*, uint32_t, bool, const Dims&, const Tuning&, hipStream_t s) {

@@ -27,7 +27,7 @@ def clang():
     return None
 
 
-def build(tmp_path, runtime_source, name, sanitize=True):
+def build(tmp_path, runtime_source, name, sanitize=True, driver="tsan_driver.cpp"):
     cxx = clang()
     if cxx is None:
         pytest.skip("no clang with a ThreadSanitizer runtime on this machine")
@@ -35,7 +35,7 @@ def build(tmp_path, runtime_source, name, sanitize=True):
     cmd = [cxx, "-std=c++17", "-O1", "-g"] + (["-fsanitize=thread"] if sanitize else []) + \
           ["-I", STUB, "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-x", "c++", runtime_source,
            os.path.join(CSRC, "ep_plan.cpp"), os.path.join(STUB, "kernels_stub.cpp"),
-           os.path.join(STUB, "tsan_driver.cpp"), "-o", out, "-pthread"]
+           os.path.join(STUB, driver), "-o", out, "-pthread"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0 and "tsan" in proc.stdout and "cannot find" in proc.stdout:
         pytest.skip("this clang has no ThreadSanitizer runtime")
