@@ -109,8 +109,8 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * (32 in all), where a block has a wave per 1024 hidden elements, 4 to 8 of
  * them, and goes through as many rounds of every rank as the longest list has;
  * by default it may then be at most 16384 (bf16: 8192) rounds for all tokens
- * together; and, by default, above 4096 up to "fused_shared_max" (16384)
- * selections from top-3 (bf16: to top-12) up and between 513 and 4096 hidden
+ * together; and, while "fused_small_max" is the default, up to
+ * "fused_shared_max" (16384) selections from top-3 (bf16: to top-12) up and between 513 and 4096 hidden
  * elements, where
  * blocks of several tokens read at most 6144 rounds together - and 0
  * always takes the count / pack / scale-transpose launches; "scales_direct": 1

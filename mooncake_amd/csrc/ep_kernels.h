@@ -161,6 +161,8 @@ struct Dims {
     int units() const { return plan.total; }
 };
 
+constexpr int kFusedSmallMax = 4096;  // default of Tuning::fused_small_max
+
 // Tuning knobs, settable at run time for measurement sweeps.
 struct Tuning {
     int pack_waves = 4;        // waves per block in the pack kernel
@@ -182,8 +184,9 @@ struct Tuning {
     int scales_direct = 1;     // allow the pack kernel to store the scales in place where they are few (see scales_direct())
     int comm_stream = 0;       // 1: per-rank rounds always run on the world's communication stream
     int fused_small = 1;       // dispatch of a small world (see dispatch_small_kernel) in one launch
-    int fused_small_max = 4096;   // ... when the world names at most this many selections
-    int fused_shared_max = 16384;  // ... and up to this many where blocks of several tokens share the lists (plan_small)
+    int fused_small_max = kFusedSmallMax;   // ... when the world names at most this many selections
+    int fused_shared_max = 16384;  // ... and, while that is the default, up to this many where blocks of several tokens
+                                  // share the lists (plan_small)
     int fused_small_rounds = -1;  // ... in at most this many rounds of kSmallListRound index-list entries per wave
                                   // (plan_small); -1: what measurement chose
     int last_dispatch_launches = 0;   // read-only in spirit: kernels the world's last dispatch / combine call enqueued

@@ -68,7 +68,8 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
         // 6.8 / 5.8); not top-1 and top-2, whose selections may all name one expert and queue for its counter.  Many
         // selections are many in the block too: bf16, 500, 1024, top-9 7.0 / 6.4, 8 x 80, 640, top-11 7.2 / 7.1, but
         // 2 x 250, 1024, top-16 8.1 / 8.6 (fp8, with two launches saved, 10.2 / 8.9).
-        const bool pays = tokens * K > 4096 && tokens * K <= (long long)t.fused_shared_max && !chosen && K > 2 &&
+        // A program that set "fused_small_max" has said how many selections the one launch may have.
+        const bool pays = t.fused_small_max == kFusedSmallMax && tokens * K <= (long long)t.fused_shared_max && !chosen && K > 2 &&
                           (use_fp8 || K <= 12) &&
                           hidden > 512 && together > 1 && R <= kSmallRanks && walked <= 4 * kSmallWaves &&
                           tokens * walked <= 6144ll * together;
