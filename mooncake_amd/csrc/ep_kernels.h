@@ -63,9 +63,11 @@ struct TableChunk {
 constexpr int kSmallRanks = 32;
 constexpr int kSmallWaveRanks = 8;
 constexpr int kSmallListRound = 512;  // index-list entries a wave of the one-launch dispatch has in flight at a time
+constexpr int kSmallExperts = 8;      // experts a block of dispatch_small_kernel counts for recv_count and layout_range
+constexpr int kCUs = 256;
 constexpr int kSmallWaves = 8;        // most waves a block of dispatch_small_kernel has
-// its waves per block (a block is one token): one per 1024-element slab, at least four, so that a block of few slabs does
-// not wait for long lists
+// its waves per block where a block is one token: one per 1024-element slab, at least four, so that a block of few slabs
+// does not wait for long lists
 constexpr int small_block_waves(int hidden) {
     return (hidden + 1023) / 1024 > kSmallWaves ? kSmallWaves : (hidden > 4096 ? (hidden + 1023) / 1024 : 4);
 }
@@ -209,7 +211,7 @@ struct SmallPlan {
     int block_tokens = 1;      // dispatch_small_kernel: tokens of a block, which share one walk through the lists
     bool single = false;       // few enough lists that a wave counting alone could take them
 };
-SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t);
+SmallPlan plan_small(const int32_t* num_tokens, int R, int E, int K, int hidden, bool use_fp8, const Tuning& t);
 // Whether the reduce kernels look anything up in the rank table: nothing when every tensor they touch is evenly spaced.
 bool combine_reads_table(const CombineSource& src, bool direct);
 

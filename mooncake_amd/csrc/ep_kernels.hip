@@ -802,7 +802,6 @@ __global__ __launch_bounds__(512) void pack_bf16_kernel(const uint64_t* __restri
 // a block / several: 12 ragged ranks of 70, hidden 1152, top-5, fp8 7.2 / 5.9; 24 x 20, 3072, top-8, fp8 8.2 / 7.4; 1024
 // tokens of 768, top-4, hot experts 7.0 / 5.4.  Count + pack / several: 640 tokens of 2048, top-8, fp8 8.2 / 6.8; 2 x 860,
 // 1024, top-8, fp8 8.8 / 8.0, bf16 9.6 / 8.1.
-constexpr int kSmallExperts = 8;
 constexpr int kSmallSpan = 4096;                    // experts a data block counts at a time (16 KB of LDS)
 constexpr int kSmallDepth = kSmallListRound / 64;   // entries per lane and round
 

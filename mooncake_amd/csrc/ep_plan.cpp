@@ -44,7 +44,7 @@ bool scales_direct(const Dims& d, bool use_fp8, const Tuning& t) {
            (long long)d.R * d.Tgrid * d.K * (d.H / 128) <= kMostScales;
 }
 
-SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool use_fp8, const Tuning& t) {
+SmallPlan plan_small(const int32_t* num_tokens, int R, int E, int K, int hidden, bool use_fp8, const Tuning& t) {
     long long tokens = 0, lists = 0;           // tokens; rounds of kSmallListRound entries, each rank's list by itself
     int most = 0;
     for (int r = 0; r < R; ++r) {
@@ -57,6 +57,13 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
     const bool chosen = t.fused_small_rounds >= 0;      // the option replaces the measured lines
     const long long walked = (long long)R * (((long long)most * K + kSmallListRound - 1) / kSmallListRound);
     const int together = small_block_tokens(hidden);
+    // Blocks a CU gets, with a token a block and with several: its 256-fold steps are what the time goes by.  The experts'
+    // blocks, eight experts each, walk all the lists.
+    long long shared_blocks = 0;
+    for (int r = 0; r < R; ++r) shared_blocks += ((num_tokens[r] > 0 ? num_tokens[r] : 0) + together - 1) / together;
+    const long long expert_blocks = ((long long)E + kSmallExperts - 1) / kSmallExperts;
+    const long long apart_layers = (tokens + expert_blocks + kCUs - 1) / kCUs;
+    const long long layers = (shared_blocks + expert_blocks + kCUs - 1) / kCUs;
     if (tokens * K > (long long)t.fused_small_max) {
         // Too many for a token a block.  Up to hidden 4096 several tokens share one: the lists are read that many times
         // less, by eight waves.  Priced by the rounds of all blocks together.  Dispatch, us, apart / in one: fp8, 640
@@ -68,11 +75,24 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
         // 6.8 / 5.8); not top-1 and top-2, whose selections may all name one expert and queue for its counter.  Many
         // selections are many in the block too: bf16, 500, 1024, top-9 7.0 / 6.4, 8 x 80, 640, top-11 7.2 / 7.1, but
         // 2 x 250, 1024, top-16 8.1 / 8.6 (fp8, with two launches saved, 10.2 / 8.9).
+        // Those figures have few experts, whose blocks find room beside the tokens' on the 256 CUs.  A second block on a CU
+        // walks all the lists once more, which separate launches do not up to 1024 experts (beyond, they have a prefix launch
+        // and cost more): 32 x 46, 1024, top-8, 512 / 640 experts bf16 9.8 / 8.7, 10.0 / 10.5, fp8 9.5 / 9.1, 9.7 / 11.2;
+        // 24 x 42, 2048, 528 experts 10.9 / 10.5, 10.1 / 10.6; 2 x 860, 1024, 512 experts 10.3 / 9.5, 9.7 / 10.1; 8 x 72, 4096,
+        // 768 experts, walking 16 rounds 11.7 / 9.9, 12.6 / 10.3; 32 x 46, 1024 experts 12.2 / 10.9, 12.1 / 11.4.
+        // Short rows in the lists of many ranks, each a round of its own, are packed sooner than the rounds are walked, in
+        // bf16, by selections x hidden: 32 x 17, 640 (2.8 million) 6.6 / 7.4, 1024 (4.5) 7.0 / 7.8, 2048 (8.9) 8.4 / 7.9;
+        // 32 x 32, 1024 (8.4) 7.9 / 8.1; 28 x 24, 1024 (5.5) 7.2 / 7.4; 24 x 24 (4.7) 6.9 / 7.2, 24 x 30 (5.9) 7.3 / 7.3, 12 x 100,
+        // top-6 (7.4) 7.9 / 7.2; walking 20 rounds 20 x 28 (4.6) 7.0 / 6.9; with 512 experts 32 x 22, 1024 (5.8) 8.0 / 7.9;
+        // top-4 32 x 33, 640 (2.7) 6.6 / 6.8, 1024 (4.3) 6.9 / 7.0, 32 x 40 (5.2) 7.3 / 7.0, 28 x 40, 640 (2.9) 6.7 / 6.4.
         // A program that set "fused_small_max" has said how many selections the one launch may have.
+        const bool crowded = E < 1024 && layers > 1 && layers * walked > (use_fp8 ? 32 : 56);
+        const bool short_rows = !use_fp8 && E < 512 && (K > 4 ? walked > 20 && tokens * K * hidden <= walked * (1ll << 18)
+                                                              : walked > 28 && tokens * K * hidden <= (1ll << 22));
         const bool pays = t.fused_small_max == kFusedSmallMax && tokens * K <= (long long)t.fused_shared_max && !chosen && K > 2 &&
                           (use_fp8 || K <= 12) &&
                           hidden > 512 && together > 1 && R <= kSmallRanks && walked <= 4 * kSmallWaves &&
-                          tokens * walked <= 6144ll * together;
+                          tokens * walked <= 6144ll * together && !crowded && !short_rows;
         if (pays) {
             p.fused = p.could = true;
             p.block_tokens = together;
@@ -111,10 +131,21 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int K, int hidden, bool u
               (walked + waves - 1) / waves <= limit && (chosen || tokens * walked <= (use_fp8 ? 16384 : 8192));
     // Several tokens a block, where the blocks' reading of the lists is what takes the time.  One token a block / several,
     // us, by rounds of all tokens: 12 ragged ranks of 70, hidden 1152, top-5 (10080) 7.3 / 5.9; 24 x 20, 3072, top-8 (11520)
-    // 8.3 / 7.4; 16 x 32, 2048, bf16 (8192) 7.5 / 6.9; 1024 tokens of 768, top-4 (8192) 7.1 / 5.4; but 8 x 64, 4096, top-6
+    // 8.3 / 7.4; 16 x 32, 1024, bf16 (8192) 7.5 / 6.6; 1024 tokens of 768, top-4 (8192) 7.1 / 5.4; but 8 x 64, 4096, top-6
     // (4096) 6.9 / 7.1, 4 x 128, 2048, top-4, bf16 (2048) 4.9 / 5.3: the others' selections in the block are a step more, and
     // a longer one above top-8: 16 x 24, 1024, top-9 (6144) 6.8 / 7.2, 24 x 12, 1024, top-11 (6912) 7.9 / 7.9.
-    if (tokens * walked >= (K <= 8 ? 6144 : 8192)) p.block_tokens = together;
+    // And only where a CU gets that many fewer of the blocks, which are eight waves and not four.  fp8, blocks a CU gets: one for
+    // two 16 x 24, 2048, top-8 (6144) 6.7 / 6.8, 16 x 26 (6656) 6.9 / 6.8; two for three, hidden 2048 and less: 16 x 32, 2048, 1280
+    // experts 8.2 / 8.7, 24 x 16, 1152, top-5, 1296 experts 8.1 / 8.5, from hidden 2049 on, in smaller blocks: 24 x 20, 3072, 528
+    // experts 9.3 / 9.1; three for five 12 x 64, 1024, 3588 experts 9.5 / 9.0; two for two 20 x 20, 3072, 520 experts 7.7 / 8.5,
+    // three for three 9.1 / 10.8.  bf16: one for two 16 x 26, 2048 (6656) 6.5 / 6.7, hidden 4096 7.3 / 7.8; two for four 4 x 200, 3072,
+    // top-4 6.6 / 6.8, but up to hidden 2048 16 x 32, 2560 experts 9.2 / 8.8; three for five 1024, 4096, top-4 8.1 / 8.4; two for five 1024 of 768, top-4, 1280 experts 7.2 / 6.3, one for
+    // three 16 x 32, 1024 7.5 / 6.6, one for four 8 x 96, 2048, top-5 6.8 / 6.2.  Top-1 and top-2, every token naming one expert
+    // or not: 12 x 64, 1024, top-1, fp8 6.3 / 5.0; 2048, 1024, top-2 9.1 / 6.0, one expert 12.4 / 7.3.
+    const bool fewer = use_fp8 ? (hidden > 2048 ? 2 * apart_layers >= 3 * layers : 3 * apart_layers >= 5 * layers)
+                               : 2 * apart_layers >= 5 * layers || (hidden <= 2048 && layers >= 2 && apart_layers >= 2 * layers);
+    const int line = K > 8 ? 8192 : (use_fp8 && apart_layers < 3 * layers ? 6400 : 6144);
+    if (fewer && tokens * walked >= line) p.block_tokens = together;
     return p;
 }
 

@@ -588,7 +588,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     }
     // A world that names few selections is dispatched in one launch, which rebuilds the routing it needs from the index
     // lists (dispatch_small_kernel, dispatch_alone_kernel); the rank table then travels in kernel arguments.
-    const SmallPlan small = phases == MC_EP_PHASE_ALL ? plan_small(num_tokens, R, num_topk, hidden, use_fp8 != 0, w->tuning)
+    const SmallPlan small = phases == MC_EP_PHASE_ALL ? plan_small(num_tokens, R, num_experts, num_topk, hidden, use_fp8 != 0, w->tuning)
                                                       : SmallPlan{};
     bool fused = small.fused && (small.single || !w->phases_captured);
     DeviceGuard guard(w->device);
