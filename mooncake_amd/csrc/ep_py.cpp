@@ -460,8 +460,9 @@ struct PreparedCombine {
 
 // The whole-world calls from stacked tensors: rank r's tensor is slice r of one tensor, and its address, which indexing in
 // Python costs 0.4 us to learn, is the first one's plus r strides.  Everything is read off the tensors at each call and
-// nothing kept.  A call answers false, having done nothing, where an argument is neither None nor a plain torch.Tensor (or
-// Parameter; another subclass may have its own idea of indexing): the caller then marshals it in Python.
+// nothing kept.  A call answers false, having done nothing, where a tensor is neither None nor a plain torch.Tensor (or
+// Parameter; another subclass may have its own idea of indexing) with a slice per rank, or the token counts or
+// the ranks that take part are not plain lists: the caller then marshals it in Python, or is refused there.
 // Host time of a call, us (of two speeds that one host ran at): 4 ranks, dispatch and combine 5.2 to 6.1 -> 4.0 to 4.9
 // (keyed and looked up in Python before), cast back 16 to 17 -> 4.5 to 5.8 (a slice per rank and tensor before); 32 ranks,
 // dispatch 10.7 to 12.9 -> 7.3 to 9.9, combine 5.8 to 7.2 -> 4.7 to 6.5, cast back 120 -> 4.8 to 6.6.
@@ -469,41 +470,44 @@ class Stacked {
    public:
     explicit Stacked(const World& w) : ranks_(w.num_ranks) { words_.reserve((size_t)8 * ranks_); }
 
-    // which ranks take part (None: all) and, of those, how many tokens
-    void take_part(const py::handle& present) {
-        if (present.is_none()) return;
-        const py::sequence flags = py::reinterpret_borrow<py::sequence>(present);
+    // Every step below answers false where it is given anything but the plain form.  No Python code runs in between (a
+    // list's items are looked at only where they are plain numbers), so nothing can change under it.
+
+    // which ranks take part (None: all): a list or a tuple of numbers, one per rank
+    bool take_part(const py::handle& present) {
+        if (present.is_none()) return true;
+        PyObject* p = present.ptr();
+        const bool list = PyList_CheckExact(p);
+        if (!(list || PyTuple_CheckExact(p)) || Py_SIZE(p) != ranks_) return false;
         present_.resize(ranks_);
         for (int r = 0; r < ranks_; ++r) {
-            const int on = PyObject_IsTrue(py::object(flags[r]).ptr());
-            if (on < 0) throw py::error_already_set();
-            present_[r] = on != 0;
+            PyObject* on = list ? PyList_GET_ITEM(p, r) : PyTuple_GET_ITEM(p, r);
+            if (!PyBool_Check(on) && !PyLong_CheckExact(on)) return false;
+            present_[r] = PyObject_IsTrue(on) != 0;
         }
+        return true;
     }
-    void tokens(const py::handle& counts) {
-        if (PyList_CheckExact(counts.ptr())) {           // (0.8 us less for 32 ranks than pybind11's conversion)
-            const Py_ssize_t n = PyList_GET_SIZE(counts.ptr());
-            counts_.reserve((size_t)n);
-            for (Py_ssize_t r = 0; r < n; ++r) {
-                const long v = PyLong_AsLong(PyList_GET_ITEM(counts.ptr(), r));
-                if (v == -1 && PyErr_Occurred()) throw py::error_already_set();
-                counts_.push_back(as_int(v));
-            }
-        } else {
-            counts_ = counts.cast<I32s>();
+    // and, of those, how many tokens: a list of numbers, one per rank
+    bool tokens(const py::handle& counts) {
+        if (!PyList_CheckExact(counts.ptr()) || PyList_GET_SIZE(counts.ptr()) != ranks_) return false;
+        counts_.resize(ranks_);
+        for (int r = 0; r < ranks_; ++r) {
+            PyObject* n = PyList_GET_ITEM(counts.ptr(), r);
+            int overflow = 0;
+            const long v = PyLong_CheckExact(n) ? PyLong_AsLongAndOverflow(n, &overflow) : -1;
+            if (overflow != 0 || v < 0 || v > INT_MAX) return false;
+            counts_[r] = (!present_.empty() && !present_[r]) ? 0 : (int)v;
         }
-        if ((int)counts_.size() != ranks_) throw std::invalid_argument("num_tokens: one per rank");
-        for (size_t r = 0; r < present_.size(); ++r)
-            if (!present_[r]) counts_[r] = 0;
+        return true;
     }
-    // adds a tensor's addresses (zeros for None, and, of_present, for ranks that take no part)
+    // a tensor's addresses (zeros for None, and, of_present, for ranks that take no part)
     bool add(const py::handle& h, bool of_present = false) {
         const size_t at = words_.size();
         words_.resize(at + ranks_, 0);
         if (h.is_none()) return true;
         if (!THPVariable_CheckExact(h.ptr())) return false;
         const at::Tensor& t = THPVariable_Unpack(h.ptr());
-        if (t.dim() < 1 || t.size(0) < ranks_) throw py::index_error("a stacked tensor has a slice per logical rank");
+        if (t.layout() != at::kStrided || t.dim() < 1 || t.size(0) < ranks_) return false;
         if (t.numel() == 0) return true;               // (an empty tensor has no address)
         const uint64_t first = address(t);
         const int64_t step = t.stride(0) * (int64_t)t.element_size();
@@ -526,10 +530,8 @@ bool dispatch_stacked(const World& w, py::handle x, py::handle topk_idx, py::han
                       py::handle present, int hidden, int num_topk, int max_tokens, int num_experts, bool use_fp8,
                       int phases, uint64_t stream_ptr) {
     Stacked s(w);
-    s.take_part(present);
-    s.tokens(num_tokens);
-    if (!s.add(x) || !s.add(topk_idx) || !s.add(recv_x, true) || !s.add(recv_scales, true) || !s.add(recv_count, true) ||
-        !s.add(src_info, true) || !s.add(layout_range, true))
+    if (!s.take_part(present) || !s.tokens(num_tokens) || !s.add(x) || !s.add(topk_idx) || !s.add(recv_x, true) ||
+        !s.add(recv_scales, true) || !s.add(recv_count, true) || !s.add(src_info, true) || !s.add(layout_range, true))
         return false;
     check(mc_ep_world_dispatch(w.h, s[0], s[1], s.counts(), hidden, num_topk, max_tokens, num_experts, use_fp8 ? 1 : 0,
                                s[2], use_fp8 ? s[3] : nullptr, s[4], s[5], s[6], phases, stream_ptr));
@@ -542,10 +544,8 @@ bool combine_stacked(const World& w, py::handle x, py::handle scales, py::handle
                      py::handle num_tokens, py::handle present, int hidden, int num_topk, int max_tokens, int num_experts,
                      bool packed, uint64_t factor_ptr, int phases, uint64_t stream_ptr) {
     Stacked s(w);
-    s.take_part(present);
-    s.tokens(num_tokens);
-    if (!s.add(x, true) || !s.add(scales, true) || !s.add(topk_idx) || !s.add(topk_weights) || !s.add(src_info) ||
-        !s.add(layout_range) || !s.add(active_ranks) || !s.add(out))
+    if (!s.take_part(present) || !s.tokens(num_tokens) || !s.add(x, true) || !s.add(scales, true) || !s.add(topk_idx) ||
+        !s.add(topk_weights) || !s.add(src_info) || !s.add(layout_range) || !s.add(active_ranks) || !s.add(out))
         return false;
     if (packed)
         check(mc_ep_world_combine_packed(w.h, s[0], scales.is_none() ? nullptr : s[1], factor_ptr, s[2], s[3], s[4], s[5],
@@ -561,8 +561,8 @@ bool cast_back_stacked(const World& w, py::handle recv_x, py::handle scales, py:
                        py::handle out, py::handle present, int hidden, int num_topk, int max_tokens, int num_experts,
                        uint64_t stream_ptr) {
     Stacked s(w);
-    s.take_part(present);
-    if (!s.add(recv_x, true) || !s.add(scales, true) || !s.add(recv_count) || !s.add(out)) return false;
+    if (!s.take_part(present) || !s.add(recv_x, true) || !s.add(scales, true) || !s.add(recv_count) || !s.add(out))
+        return false;
     check(mc_ep_world_cast_back(w.h, s[0], scales.is_none() ? nullptr : s[1], s[2], factor_ptr, s[3], hidden, num_topk,
                                 max_tokens, num_experts, stream_ptr));
     return true;

@@ -89,3 +89,49 @@ def test_stacked_calls_refuse_what_marshalled_ones_refuse(gpu_device, monkeypatc
         h.num_tokens, h.topk_idx = tokens, None
         with pytest.raises(RuntimeError):
             h.dispatch()
+
+
+def test_forms_that_marshalled_calls_take(gpu_device, monkeypatch):
+    """Ranks that take part and token counts in other forms than lists of numbers, and tensors that end with the last
+    rank that takes part."""
+    import numpy as np
+
+    cfg = EPConfig("forms", R, T, 640, 8, 3, True)
+    data = generate(cfg, seed=7)
+    on, nt = [1, 1, 1, 0], [T, 0, 5, 11]
+    forms = {
+        "lists": (on, nt),
+        "tensors": (torch.tensor(on), torch.tensor(nt)),
+        "on_the_gpu": (torch.tensor(on, device=gpu_device), list(torch.tensor(nt, device=gpu_device))),
+        "arrays": (np.array(on), np.array(nt, dtype=np.int64)),
+        "tuples": (tuple(map(bool, on)), tuple(nt)),
+        "by_rank": (dict(enumerate(on)), [float(n) for n in nt]),
+        "texts": (["yes", "yes", "yes", ""], [np.int32(n) for n in nt]),
+        "longer": (on + [1], nt),
+    }
+    got = {}
+    for stacked in (True, False):
+        for name, (present, tokens) in forms.items():
+            announce(f"stacked calls: {name}, stacked={stacked}")
+            h = harness(cfg, data, nt, False)
+            h.num_tokens = tokens
+            if not stacked:
+                monkeypatch.setattr(h, "_stacked", lambda ranks: None)
+            got[name, stacked] = cycle(h, present, None)
+        announce(f"stacked calls: tensors of three ranks, stacked={stacked}")
+        h = harness(cfg, data, nt, False)
+        if not stacked:
+            monkeypatch.setattr(h, "_stacked", lambda ranks: None)
+        for name in ("recv_x", "recv_scales_phys"):
+            setattr(h, name, getattr(h, name)[:R - 1])
+        h.expert_out.zero_()
+        h.dispatch(present=on)
+        h.cast_back(present=on)
+        h.combine(present=on)
+        h.combine_packed(present=on)
+        torch.cuda.synchronize()
+        got["three", stacked] = [h.expert_out.cpu().contiguous().view(torch.uint8)]
+    for name in forms:
+        for stacked in (True, False):
+            assert all(torch.equal(a, b) for a, b in zip(got[name, stacked], got["lists", False])), (name, stacked)
+    assert torch.equal(got["three", True][0], got["three", False][0])
