@@ -57,7 +57,9 @@ extern "C" {
  * ones of the same call - same shape, tensors and token counts - left in the
  * world; where the world holds none of that, because another dispatch has run
  * since or an all-phases call took one launch, a dispatch launches the earlier
- * phases with it, from the tensors it is given) */
+ * phases with it, from the tensors it is given.  Graph replays are not seen
+ * from the host: no replay of a world's dispatch may run between the phases of
+ * an eager call of that world) */
 #define MC_EP_PHASE_LAYOUT 1   /* dispatch: routing counts;  combine: handle -> row resolve */
 #define MC_EP_PHASE_DATA 2     /* dispatch: pack (packed_recv_count / src_info / layout_range are complete after
                                   this phase, not before); combine: weighted reduce */

@@ -242,7 +242,6 @@ struct mc_ep_world {
     size_t counts_cap = 0;
     uint32_t* d_chunk_map = nullptr;     // work list of the cast-back kernel (many experts), 4 words per entry
     size_t chunk_map_cap = 0;
-    bool one_launch_captured = false;                    // ... one that takes the one launch
     bool phases_captured = false;                        // a graph goes on from what a dispatch outside it left
     // what the last dispatch was called with, so that a combine given that
     // dispatch's handle can reuse its routing state instead of re-deriving rows,
@@ -522,7 +521,8 @@ int order_begin(mc_ep_world* w, hipStream_t stream, const Capture& cap) {
 // The phases that a dispatch of `phases` has to launch.  A later phase goes on from what the world's scratch holds; where
 // that is not this call's - another dispatch of the world has run since, or the one launch, which leaves no such state - the
 // phases in front of it run with it, from the call's own tensors.  Graph replays run dispatches the host never sees: once a
-// one-launch dispatch of the world lives in a graph, what a call left that is complete may be older than the last replay.
+// dispatch of the world lives in a graph, what a call left that is complete may be older than the last replay (or, by the
+// one launch, not there at all), and a recorded call may not have run yet when an eager one goes on from it.
 int phases_needed(mc_ep_world* w, const Dims& d, const uint64_t* topk_idx, const int32_t* num_tokens, bool use_fp8,
                   const uint64_t* recv_x, int phases, const Capture& cap) {
     const bool finish = use_fp8 && (phases & MC_EP_PHASE_FINISH);       // (a bf16 dispatch has no last phase)
@@ -533,7 +533,7 @@ int phases_needed(mc_ep_world* w, const Dims& d, const uint64_t* topk_idx, const
     bool own = ld.counted && (ld.valid || !ld.finished) && ld.hidden == d.H && ld.num_topk == d.K && ld.max_tokens == d.max_tokens &&
                ld.num_experts == d.E && ld.use_fp8 == use_fp8 && ld.plan.per_rank == d.plan.per_rank &&
                ld.plan.shift == d.plan.shift && ld.plan.summed == d.plan.summed && ld.plan.carried == d.plan.carried &&
-               !(w->one_launch_captured && ld.finished && !same_capture);
+               (same_capture || !w->dispatch_captured || !(ld.finished || (ld.captured && !cap.active)));
     for (int r = 0; r < d.R && own; ++r)
         own = topk_idx[r] == ld.topk_idx[r] && num_tokens[r] == ld.num_tokens[r] && recv_x[r] == ld.recv_x[r];
     const bool counts_again = (phases & MC_EP_PHASE_LAYOUT) || !own;
@@ -710,7 +710,6 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         ld.counted = !one_launch;
         ld.staged = false;
         if (cap.active) w->dispatch_captured = true;
-        if (cap.active && one_launch) w->one_launch_captured = true;
     };
     if (fused) {
         SmallTable st{};

@@ -174,6 +174,30 @@ void recorded() {
         hip_stub::g_capture = 0;
         EXPECT("eager", kShared.run(w, ALL, s), 1, 1, 1, 0);
     }
+    {
+        // a graph's separate launches: their replays fill the scratch, which an eager call that is complete may not take for
+        // its own any more; nor is what a recorded call leaves there before it has been replayed
+        World w(1);
+        Call other = kLarge;
+        other.gen = 1;
+        other.H = 2048;
+        EXPECT("eager", other.run(w, ALL, s), 1, 1, 1, 0);
+        hip_stub::g_capture = 3;
+        EXPECT("recorded", other.run(w, ALL, s), 1, 1, 1, 0);
+        EXPECT("recorded finish", other.run(w, FINISH, s), 0, 0, 1, 0);
+        hip_stub::g_capture = 0;
+        EXPECT("finish of the recorded call", other.run(w, FINISH, s), 1, 1, 1, 0);
+        EXPECT("eager", kLarge.run(w, ALL, s), 1, 1, 1, 0);
+        EXPECT("finish after a replay, perhaps", kLarge.run(w, FINISH, s), 1, 1, 1, 0);
+        EXPECT("data after a replay, perhaps", kLarge.run(w, DATA, s), 1, 1, 0, 0);
+        EXPECT("finish right behind it", kLarge.run(w, FINISH, s), 0, 0, 1, 0);
+        hip_stub::g_capture = 4;
+        EXPECT("recorded", kLarge.run(w, LAYOUT | DATA, s), 1, 1, 0, 0);
+        hip_stub::g_capture = 5;
+        EXPECT("the last phase in a graph of its own", kLarge.run(w, FINISH, s), 0, 0, 1, 0);
+        hip_stub::g_capture = 0;
+        EXPECT("data and finish, without a replay", kLarge.run(w, DATA | FINISH, s), 1, 1, 1, 0);
+    }
     if (hipStreamDestroy(s) != hipSuccess) ++g_failures;
 }
 

@@ -92,3 +92,32 @@ def test_recorded_later_phase_goes_on_from_eager_dispatches(gpu_device, oracle):
         torch.cuda.synchronize()
         ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, True)
         compare_dispatch(h, ref, check_poison=True)
+
+
+def test_last_phase_after_replays_of_another_call(gpu_device, oracle):
+    """Replays of a recorded call, which are not seen from the host, fill the world's scratch between a complete call and a
+    later phase of it by itself."""
+    world = ep.World(1)
+    cfg = EPConfig("eager", 1, 1024, 4224, 8, 5, True)
+    announce(f"last phase after replays {cfg}")
+    other = WorldHarness(EPConfig("recorded", 1, 1024, 4224, 8, 5, True), world=world)     # (the same shape, other tensors)
+    other.load(generate(cfg, seed=98))
+    other.alloc_dispatch_outputs()
+    other.dispatch()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        other.dispatch()
+    h = WorldHarness(cfg, world=world)
+    h.alloc_dispatch_outputs(poison=True)
+    for seed in (99, 100, 101):
+        data = generate(cfg, seed=seed)
+        h.load(data)
+        ref = oracle.dispatch(data["x"], data["topk_idx"], h.num_tokens, cfg.max_tokens, cfg.num_experts, True)
+        poison(h)
+        h.dispatch()
+        g.replay()
+        h.recv_scales_phys.fill_(float("nan"))
+        h.dispatch(phases=_lib.PHASE_FINISH)
+        torch.cuda.synchronize()
+        compare_dispatch(h, ref, check_poison=True)
