@@ -122,7 +122,8 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * in one call;
  * "last_dispatch_launches", "last_combine_launches": read them to learn how
  * many kernels the world's last dispatch / combine call enqueued (a rank-table
- * upload counts); "fp8_arith": 0 (default) the fp8 scale arithmetic of the reference's
+ * upload counts); "last_dispatch_block_tokens": how many tokens a block of its one
+ * launch had (0: it took separate ones); "fp8_arith": 0 (default) the fp8 scale arithmetic of the reference's
  * PyTorch statement as CPU PyTorch runs it - 448.0 / amax as reciprocal times
  * 448, amax / 448.0 a true division (mooncake_ep_buffer.py:699-702) - or 1 the
  * reference kernel's own, 448 / amax as one IEEE division and amax * (1 / 448)

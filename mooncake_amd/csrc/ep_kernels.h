@@ -193,6 +193,7 @@ struct Tuning {
                                   // (plan_small); -1: what measurement chose
     int last_dispatch_launches = 0;   // read-only in spirit: kernels the world's last dispatch / combine call enqueued
     int last_combine_launches = 0;    // (a rank-table upload counts; launches of other phases' calls do not)
+    int last_dispatch_block_tokens = 0;   // likewise: tokens of a block in its one launch, 0 if it took separate ones
     int blocking = 0;          // 1: a per-rank call returns only when its round has been launched (a thread per rank)
     int block_timeout_ms = 30000;   // how long such a call waits for its peers before it fails
     int block_spin_us = 200;        // ... of which this long awake (yielding the core), before it goes to sleep

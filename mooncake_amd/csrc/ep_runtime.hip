@@ -591,6 +591,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
     const SmallPlan small = phases == MC_EP_PHASE_ALL ? plan_small(num_tokens, R, num_experts, num_topk, hidden, use_fp8 != 0, w->tuning)
                                                       : SmallPlan{};
     bool fused = small.fused && (small.single || !w->phases_captured);
+    w->tuning.last_dispatch_block_tokens = 0;
     DeviceGuard guard(w->device);
     w->launches = 0;
     struct Tally {                                // the option "last_dispatch_launches", on every way out
@@ -716,6 +717,7 @@ int world_dispatch_impl(mc_ep_world* w, const uint64_t* x, const uint64_t* topk_
         memcpy(st.v, tbl, tbl_words * sizeof(uint64_t));
         MC_HIP(launch_dispatch_small(st, sc.selrow, d, use_fp8 != 0, small.alone, w->tuning, stream));
         w->launches += 1;
+        w->tuning.last_dispatch_block_tokens = small.alone ? 1 : d.block_tokens;
         if (!static_scratch) remember(true);
         return MC_EP_OK;
     }
@@ -1278,6 +1280,7 @@ static int* option_slot(Tuning& t, const char* name) {
     if (!strcmp(name, "combine_nt")) return &t.combine_nt;
     if (!strcmp(name, "last_dispatch_launches")) return &t.last_dispatch_launches;
     if (!strcmp(name, "last_combine_launches")) return &t.last_combine_launches;
+    if (!strcmp(name, "last_dispatch_block_tokens")) return &t.last_dispatch_block_tokens;
     if (!strcmp(name, "fused_small")) return &t.fused_small;
     if (!strcmp(name, "fused_small_max")) return &t.fused_small_max;
     if (!strcmp(name, "fused_shared_max")) return &t.fused_shared_max;
