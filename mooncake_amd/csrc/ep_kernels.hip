@@ -1549,10 +1549,13 @@ __device__ __forceinline__ uint32_t scale_round_twice(float a, float b, float s,
 // enters the fp32 fused multiply-add chain in k order (mooncake_ep_kernel.cu:711-753), so the result
 // is bit for bit that of the two-kernel path.
 //
-// One wave per (token, slab): 1024 elements of an fp8 payload (16 payload bytes and one scale per lane
-// and row; a 128-element scale group is 8 lanes, and the scales of a row sit R*max floats apart in the
-// column-major layout), 512 elements of a bf16 payload.  Lanes 0..K-1 find the K rows as reduce_kernel
-// does; a masked, inactive or unknown selection reads the zero row with weight 0.
+// One wave per (token, slab): 1024 elements of an fp8 payload (16 payload bytes per lane and row; a
+// 128-element scale group is 8 lanes, and the scales of a row sit R*max floats apart in the column-major
+// layout), 512 elements of a bf16 payload.  The rows are found as in reduce_kernel: a selection's by the
+// kLanes lanes of an equal share of the wave, or by one lane where a bf16 payload's selections are not
+// searched for; those lanes of an fp8 payload then fetch the row's scales of the slab's eight groups, and
+// every lane picks its own group's up.  A masked, inactive or unknown selection reads the zero row with
+// weight 0.
 //
 // Up to top-8 the register budget is that of eight waves per SIMD: left to itself the compiler spends
 // twice as many on the variant without a factor (to hoist every load), and at four waves per SIMD that
@@ -1603,7 +1606,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KMAX <= 8 ?
     const int64_t RM = (int64_t)R * max_tokens;
     const int G = H >> 7, L = E / R;
 
-    // lanes 0..K-1: where the selection's row, its scales and its factor are
+    // the selection of the lane's share of the wave (`sel`): where its row, its scales and its factor are
     uint64_t src = (uint64_t)zero_row, ssrc = (uint64_t)zero_row;
     float w = 0.0f, f = 1.0f;
     int sstride = 0;                     // bytes between a row's consecutive scale groups (0: the zero row)
