@@ -40,3 +40,31 @@ def test_every_topk_matches_oracle(gpu_device, oracle, topk, use_fp8):
                 for r, n in enumerate(nt):
                     assert torch.equal(got[r, :n].view(torch.int16), want[r, :n].view(torch.int16)), (direct, tokens, r)
                     assert bool((got[r, n:] == 7.0).all()), "rows beyond num_tokens written"
+
+
+def test_a_last_slab_of_few_elements_takes_no_longer(gpu_device):
+    """Packed combine of rows whose last slab has one scale group, against rows that are longer by three: the arithmetic is
+    done by all lanes of a wave.  (Under the mask of the lanes inside the row, eight of 64, it took 2.2 times as long.)"""
+    announce("packed combine, a last slab of one scale group")
+    best = {}
+    for hidden in (1152, 1536):
+        cfg = EPConfig("slab", 1, 64, hidden, 16, 16, True)
+        h = run_dispatch(cfg, generate(cfg, seed=120), poison=False)
+        h.alloc_combine_io()
+        factor = torch.ones(cfg.num_experts)
+        h.combine_packed(factor)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            h.dispatch()
+            for _ in range(20):
+                h.combine_packed(h._factor)
+        best[hidden] = float("inf")
+        for _ in range(20):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            g.replay()
+            end.record()
+            torch.cuda.synchronize()
+            best[hidden] = min(best[hidden], start.elapsed_time(end))
+    assert best[1152] < 1.5 * best[1536], best
