@@ -115,7 +115,7 @@ int mc_ep_world_set_rank_silent(mc_ep_world_t* world, int rank, int silent);
  * "fused_shared_max" (16384) selections from top-3 (bf16: to top-12) up and between 513 and 4096 hidden
  * elements, where
  * blocks of several tokens read at most 6144 rounds together, and less where
- * a CU gets more than one of them or a bf16 world's rows are short - and 0
+ * a CU gets more than one of them or rows are short - and 0
  * always takes the count / pack / scale-transpose launches; "scales_direct": 1
  * (default) leaves the last of them out where an fp8 dispatch has at most 327680
  * scales (selections times hidden / 128, hidden above 512) and all its phases run

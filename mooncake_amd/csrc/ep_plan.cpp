@@ -85,10 +85,25 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int E, int K, int hidden,
         // 32 x 32, 1024 (8.4) 7.9 / 8.1; 28 x 24, 1024 (5.5) 7.2 / 7.4; 24 x 24 (4.7) 6.9 / 7.2, 24 x 30 (5.9) 7.3 / 7.3, 12 x 100,
         // top-6 (7.4) 7.9 / 7.2; walking 20 rounds 20 x 28 (4.6) 7.0 / 6.9; with 512 experts 32 x 22, 1024 (5.8) 8.0 / 7.9;
         // top-4 32 x 33, 640 (2.7) 6.6 / 6.8, 1024 (4.3) 6.9 / 7.0, 32 x 40 (5.2) 7.3 / 7.0, 28 x 40, 640 (2.9) 6.7 / 6.4.
+        // Above top-8 a token's place among the block's other selections takes longer, and short rows lose by the elements
+        // that a round of the lists stands for, in thousands: bf16, top-12, 12 x 44, 1024 (270) 7.9 / 8.9, 16 x 28, 1024
+        // (344) 7.6 / 8.3, 32 x 17, 896, 512 experts (209) 8.6 / 9.4, top-10, 12 x 53, 1024 (271) 7.9 / 8.5, but 8 x 92, 1024,
+        // top-9 (424) 8.1 / 7.6, and lists of few ranks, whose rounds are full: 2 x 471, 896, top-10 8.4 / 8.0.  fp8, whose rows
+        // are half as long: 32 x 25, 896, top-12 (269) 8.6 / 10.3, 16 x 57, 768, top-9 (197) 8.0 / 9.3, 12 x 61, 768, top-10
+        // (234) 7.6 / 8.6, and with them from top-5 up 16 x 71, 640, top-8 (182) 8.1 / 9.1, 32 x 19, 896, top-7 (119) 7.6 / 8.2.
+        // With a second block on a CU, from 24 rounds on: bf16, 24 x 78, 640, top-4, 384 experts (199) 8.0 / 8.9, 8 x 251, 640,
+        // top-6 (321) 8.3 / 9.1, 24 x 37, 1152, top-8 (340) 8.7 / 9.2.
         // A program that set "fused_small_max" has said how many selections the one launch may have.
-        const bool crowded = E < 1024 && layers > 1 && layers * walked > (use_fp8 ? 32 : 56);
-        const bool short_rows = !use_fp8 && E < 512 && (K > 4 ? walked > 20 && tokens * K * hidden <= walked * (1ll << 18)
-                                                              : walked > 28 && tokens * K * hidden <= (1ll << 22));
+        const long long per_round = tokens * K * hidden / walked;
+        const bool crowded = E < 1024 && layers > 1 &&
+                             (layers * walked > (use_fp8 ? 32 : 56) || (walked >= 24 && per_round <= 7 << 16));
+        bool short_rows = false;
+        if (use_fp8)
+            short_rows = E < 1024 && (K > 8 ? walked >= 16 && per_round <= 7 << 16 : K > 4 && walked >= 24 && per_round <= 1 << 18);
+        else if (K > 8)
+            short_rows = E < 1024 && R >= 8 && walked >= 12 && per_round <= (K > 10 ? 15 << 15 : 5 << 16);
+        else if (E < 512)
+            short_rows = K > 4 ? walked > 20 && per_round <= 1 << 18 : walked > 28 && tokens * K * hidden <= (1ll << 22);
         const bool pays = t.fused_small_max == kFusedSmallMax && tokens * K <= (long long)t.fused_shared_max && !chosen && K > 2 &&
                           (use_fp8 || K <= 12) &&
                           hidden > 512 && together > 1 && R <= kSmallRanks && walked <= 4 * kSmallWaves &&
@@ -142,8 +157,20 @@ SmallPlan plan_small(const int32_t* num_tokens, int R, int E, int K, int hidden,
     // top-4 6.6 / 6.8, but up to hidden 2048 16 x 32, 2560 experts 9.2 / 8.8; three for five 1024, 4096, top-4 8.1 / 8.4; two for five 1024 of 768, top-4, 1280 experts 7.2 / 6.3, one for
     // three 16 x 32, 1024 7.5 / 6.6, one for four 8 x 96, 2048, top-5 6.8 / 6.2.  Top-1 and top-2, every token naming one expert
     // or not: 12 x 64, 1024, top-1, fp8 6.3 / 5.0; 2048, 1024, top-2 9.1 / 6.0, one expert 12.4 / 7.3.
-    const bool fewer = use_fp8 ? (hidden > 2048 ? 2 * apart_layers >= 3 * layers : 3 * apart_layers >= 5 * layers)
-                               : 2 * apart_layers >= 5 * layers || (hidden <= 2048 && layers >= 2 && apart_layers >= 2 * layers);
+    // fp8, two tokens a block, in the eight waves of four slabs: one for two 12 x 55, 4096, top-2 6.8 / 7.4, three for five 8 x
+    // 158, 3328, top-1 7.5 / 8.2, four for seven 8 x 222, 3456, top-1 9.2 / 10.5, two for four with eight rounds of lists 8 x 109,
+    // 3968, top-2 7.0 / 7.2, with more of them 16 x 51, 3328, top-1 8.2 / 7.5; in the six of three slabs three for five with
+    // eight rounds 8 x 134, 2560, top-1 7.1 / 7.3, with twelve 12 x 101, 2304, top-2 9.1 / 8.6, two for three with twelve 12 x 49,
+    // 3072, top-2 6.5 / 6.9.
+    bool fewer;
+    if (!use_fp8)
+        fewer = 2 * apart_layers >= 5 * layers || (hidden <= 2048 && layers >= 2 && apart_layers >= 2 * layers);
+    else if (hidden <= 2048 || (hidden > 3072 && K > 5))
+        fewer = 3 * apart_layers >= 5 * layers;
+    else if (hidden > 3072)
+        fewer = apart_layers >= 2 * layers && (K > 3 || walked > 8);
+    else
+        fewer = 2 * apart_layers >= 3 * layers && (K > 2 || walked > 8) && (K > 5 || walked > 16 || apart_layers > 3);
     const int line = K > 8 ? 8192 : (use_fp8 && apart_layers < 3 * layers ? 6400 : 6144);
     if (fewer && tokens * walked >= line) p.block_tokens = together;
     return p;

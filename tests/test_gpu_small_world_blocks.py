@@ -17,7 +17,7 @@ CASES = [
     EPConfig("eight_k16_bf16", 1, 512, 640, 32, 16, False),                # 8192, by the cap that the test sets
     EPConfig("eight_k1", 12, 64, 1024, 24, 1, True, routing="zipf"),       # 64 lanes on a selection
     EPConfig("eight_k2", 1, 2040, 1024, 16, 2, True, masked_fraction=0.1),
-    EPConfig("four_k9", 12, 72, 1152, 36, 9, True, masked_fraction=0.2),   # 7776
+    EPConfig("four_k9", 12, 72, 1920, 36, 9, True, masked_fraction=0.2),   # 7776
     EPConfig("four_k3", 12, 150, 2048, 24, 3, False, routing="zipf"),      # 5400
     EPConfig("two_of_three", 2, 300, 2944, 18, 8, True),                   # six waves
     EPConfig("two_of_four", 8, 80, 4096, 64, 8, False),                    # 5120
@@ -73,7 +73,8 @@ def test_size_rule_of_shared_blocks(gpu_device, oracle):
              (replace(base, hidden=4224), {}, 2, 0),                              # one token a block
              (replace(base, hidden=4096, tokens_per_rank=1228, num_topk=4), {}, 1, 2),   # 1228 x 10 rounds, 6144 x 2 at most
              (replace(base, hidden=4096, tokens_per_rank=1232, num_topk=4), {}, 2, 0),   # 1232 x 10
-             (replace(base, num_ranks=32, tokens_per_rank=22, num_experts=32), {}, 1, 8),    # 32 lists, 704 x 32 rounds
+             (replace(base, hidden=2048, num_ranks=32, tokens_per_rank=22, num_experts=32), {}, 1, 4),   # 32 lists, 704 x 32 rounds
+             (replace(base, num_ranks=32, tokens_per_rank=22, num_experts=32), {}, 2, 0),    # ... of short rows
              (replace(base, num_ranks=2, tokens_per_rank=1028, num_experts=16), {}, 2, 0),   # 16448 selections
              (replace(base, tokens_per_rank=64), {}, 1, 1)]                       # one list: a token a block
     for cfg, options, launches, tokens in cases:

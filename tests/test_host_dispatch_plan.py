@@ -43,13 +43,20 @@ LINES = [
     ((20, 20, 3072, 8, True, 2560), 1), ((16, 24, 1152, 5, True, 72), 4), ((16, 24, 1152, 5, True, 1296), 1),
     ((26, 16, 2048, 8, True, 64), 4), ((26, 16, 2048, 8, False, 64), 1), ((24, 16, 2048, 8, True, 64), 1),
     ((26, 16, 4096, 8, False, 64), 1), ((200, 4, 3072, 4, False, 64), 1), ((96, 8, 2048, 5, True, 64), 4),
+    ((55, 12, 4096, 2, True, 96), 1), ((158, 8, 3328, 1, True, 64), 1), ((222, 8, 3456, 1, True, 8), 1),
+    ((109, 8, 3968, 2, True, 8), 1), ((51, 16, 3328, 1, True, 256), 2), ((134, 8, 2560, 1, True, 64), 1),
+    ((101, 12, 2304, 2, True, 384), 2), ((49, 12, 3072, 2, True, 36), 1),
     ((1024, 1, 768, 4, False, 64), 8), ((1024, 1, 4096, 4, False, 64), 1), ((64, 12, 1024, 1, True, 12), 8),
     # more selections: separate launches where a second block on a CU, or short rows of many ranks, cost more
     ((46, 32, 1024, 8, False, 512), 8), ((46, 32, 1024, 8, False, 640), 0), ((46, 32, 1024, 8, False, 1024), 8),
     ((46, 32, 1024, 8, True, 512), 8), ((46, 32, 1024, 8, True, 640), 0), ((46, 32, 1024, 8, True, 1024), 8),
     ((860, 2, 1024, 8, False, 512), 8), ((860, 2, 1024, 8, True, 512), 0), ((72, 8, 4096, 8, True, 768), 2),
     ((42, 24, 2048, 8, True, 528), 0), ((42, 24, 2048, 8, False, 528), 4),
-    ((17, 32, 640, 8, False, 32), 0), ((17, 32, 2048, 8, False, 32), 4), ((17, 32, 640, 8, True, 32), 8),
+    ((17, 32, 640, 8, False, 32), 0), ((17, 32, 2048, 8, False, 32), 4), ((17, 32, 640, 8, True, 32), 0),
+    ((44, 12, 1024, 12, False, 36), 0), ((17, 32, 896, 12, False, 512), 0), ((53, 12, 1024, 10, False, 24), 0),
+    ((92, 8, 1024, 9, False, 72), 8), ((471, 2, 896, 10, False, 16), 8), ((78, 24, 640, 4, False, 384), 0),
+    ((251, 8, 640, 6, False, 64), 0), ((37, 24, 1152, 8, False, 192), 0), ((25, 32, 896, 12, True, 64), 0),
+    ((57, 16, 768, 9, True, 64), 0), ((71, 16, 640, 8, True, 64), 0), ((19, 32, 896, 7, True, 128), 0),
     ((28, 20, 1024, 8, False, 40), 8), ((33, 32, 640, 4, False, 32), 0), ((40, 32, 1024, 4, False, 32), 8),
 ]
 
