@@ -305,7 +305,7 @@ def time_small_world(iters):
                          "num_experts": cfg.num_experts, "num_topk": cfg.num_topk, "use_fp8": cfg.use_fp8},
                "algorithmic_bytes": alg,
                "us_at_hbm_peak": {k: round(v / HBM_PEAK_GBPS / 1e3, 2) for k, v in alg.items()}}
-        for label, fused in (("three_launch", 0), ("one_launch", 1)):
+        for label, fused in (("separate_launches", 0), ("one_launch", 1)):
             h = WorldHarness(cfg, device="cuda:0")
             h.world.set_option("fused_small", fused)
             h.load(data)

@@ -2407,7 +2407,8 @@ hipError_t launch_reduce(const uint64_t* d_tbl, const CombineRoute* d_routes, ui
     if (d.K <= 4) MCEP_K(4);
     if (d.K <= 6) MCEP_K(6);
     // (8 x 512 tokens, hidden 4096, bf16, us, padded / exact: top-7 in eight rows 45.5 / 43.5, top-9 in twelve 56.8 / 53.0,
-    // top-10 60.2 / 58.1; top-3 in four 23.5 / 23.4, top-5 in six 33.8 / 34.0, top-11 in twelve 62.3 / 61.8)
+    // top-10 60.2 / 58.1; top-3 in four 23.5 / 23.4, top-5 in six 33.8 / 34.0, top-11 in twelve 62.3 / 61.8.  100 worlds each of
+    // 4 to 2048 tokens, hidden 640 to 7168, exact over padded, geomean: top-7 0.97, top-9 0.94, top-10 0.96)
     if (d.K <= 7) MCEP_K(7);
     if (d.K <= 8) MCEP_K(8);
     if (d.K <= 9) MCEP_K(9);
@@ -2474,7 +2475,10 @@ hipError_t launch_reduce_packed(const uint64_t* d_tbl, const CombineRoute* d_rou
     // padded to 4, 8 or 16 rows / exact: top-3 23.8 / 21.5, top-5 33.5 / 27.2, top-6 34.6 / 30.6, top-7 35.8 / 33.9, top-9
     // 63.3 / 40.8, top-10 64.2 / 46.0, top-11 64.5 / 47.3; 8 x 1024, hidden 7168, top-1 50.5 / 42.0.  For bf16 payloads those
     // that gain 2 % of the combine and more: top-5 38.3 / 34.4, top-6 41.4 / 39.3, top-9 61.9 / 53.9, top-10 65.9 / 58.6,
-    // top-11 in 12 rows 66.5 / 63.0; top-7 44.5 / 44.3.
+    // top-11 in 12 rows 66.5 / 63.0; top-7 44.5 / 44.3.  100 worlds each of 4 to 2048 tokens, hidden 640 to 7168, exact over
+    // padded, geomean, the small ones gaining as much: bf16 top-5 0.92, top-6 0.95, top-9 0.85, top-10 0.87, top-11 and top-12 in 12
+    // 0.91; fp8, with the scales in one load and all lanes at work, top-1 0.91, top-3 0.92, top-5 to top-7 0.84 to 0.89, top-9 to
+    // top-12 0.73 to 0.79 (top-2, top-4 and top-8, where the rows are the same, 0.94 to 0.97).
 #define MCEP_PK8(KMAX) \
     if (use_fp8 && d.K <= KMAX) return fac ? MCEP_P4(KMAX, true, true) : MCEP_P4(KMAX, true, false)
 #define MCEP_PK16(KMAX) \

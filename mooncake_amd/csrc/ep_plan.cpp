@@ -38,6 +38,10 @@ bool scales_direct(const Dims& d, bool use_fp8, const Tuning& t) {
     // 14.4 / 28.4 -> 13.2 / 25.9; 351 (32 x 87, 1792, top-9) 19.8 / 42.4 -> 16.9 / 38.2; 459 (8 x 128, 7168, top-8) 22.1 /
     // 38.6 -> 22.6 / 39.4, (2 x 1024, 7168, top-4) 24.8 / 46.9 -> 24.3 / 46.0; 524 (16 x 128, 4096, top-8) 25.3 / 42.6 ->
     // 24.4 / 42.6.  A large world's 1.8 million take 30 us.  Rows of half a slab and less have not been measured.
+    // 400 drawn worlds of 190 to 328 thousand, direct over transposed: dispatches into three sets of outputs in turn geomean
+    // 0.85, the slowest 0.99; cycles with combine 0.93, 0.995, with the packed one 0.92, 0.996.  Dispatches into the same outputs
+    // over and over, with nothing in between, are slower at top-5 and top-6 from 32 MiB of payload on (24 x 83, 4096, top-5
+    // 16.7 / 19.4, 8 x 167, 5120, top-5 15.0 / 17.9; cycles of the first 32.5 / 32.1): the line is drawn by the cycles.
     constexpr long long kMostScales = 320 * 1024;
     // (the variants exist with written-through rows only, which payloads of that size have by default)
     return use_fp8 && t.scales_direct != 0 && (t.pack_nt < 0 || (t.pack_nt & 4)) && d.H > 512 &&
