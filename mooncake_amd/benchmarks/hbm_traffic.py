@@ -107,7 +107,7 @@ def main(argv=None) -> int:
         print()
     bench_args = (f"--config {args.workload} --no-cpu-baseline --no-flushed --no-buffer-api --no-small-world --steps 3 "
                   f"--warmup 1 --kernel-iters 2 --copy-calibration {args.copy_mib}")
-    print("Commands (on the GPU box, from the repository root; cd /tmp && export TMPDIR=/tmp first):")
+    print("Commands (from the repository root; cd /tmp && export TMPDIR=/tmp first):")
     print(f"  rocprofv3 --pmc FETCH_SIZE --output-format csv -d {args.fetch_dir} -o p -- python3 bench.py {bench_args}")
     print(f"  rocprofv3 --pmc WRITE_SIZE --output-format csv -d {args.write_dir} -o p -- python3 bench.py {bench_args}")
     print(f"  python3 -m mooncake_amd.benchmarks.hbm_traffic {args.fetch_dir} {args.write_dir} --workload {args.workload} "
