@@ -435,7 +435,7 @@ def cpu_baseline(cfg, data, bytes_total, budget_s):
     host's cores on the same workload: whole steps until the budget is spent."""
     import torch
     from oracle import oracle
-    # a one-GPU box's share of its host is 16 cores, whatever os.cpu_count() says there
+    # one GPU's share of its host is 16 cores, whatever os.cpu_count() says
     threads = min(16, os.cpu_count() or 1)
     oracle.set_threads(threads)
     R = cfg.num_ranks
